@@ -105,10 +105,6 @@ struct mcf_ctx {
   // y/z sweeps run as column marches: needs a uniform spacing along the
   // axis (ghosts included) and n >= 8
   bool fuse[3]{false, false, false};
-  // cells per segment of k_sweep_col: 256 (the whole 256^3 column) measured
-  // 1.66 / 2.32 ms per y sweep (mixed / FP64) against 1.68 / 2.37 with 128,
-  // 1.92 / 2.70 with 96 and 2.48 / 3.57 with 192 (an uneven split)
-  int col_seg = 256;
   // cooling surrogate: FP32 weights, Adam moments, gradient (4 x MLP_NP),
   // packed BF16 operands, counters {backward-Euler cells, IMC fallbacks}
   float *mlp = nullptr;
@@ -294,13 +290,38 @@ static long boxsize(const Box &b) { return (long)b.cnt[0] * b.cnt[1] * b.cnt[2];
       KLAUNCH_N(#kern, (kern<R>), dim3(nblocks(nt_)), dim3(TPB), 8.0 * (double)nt_ * (double)(narr), __VA_ARGS__); \
   } while (0)
 
-// y/z sweeps as two waves per row of columns (k_sweep_col2) on the mixed
-// path: 1.39 / 1.45 ms per y / z sweep against 1.62 / 1.70 for
-// k_sweep_col at 256^3 (250 registers, no spill, two waves per SIMD).  The
-// FP64 instance spills 224 bytes per lane to scratch at two waves per SIMD
-// (4.47 against 2.31 ms at 256^3), so FP64 takes it only for launches of
-// fewer blocks than the device has CUs, where the second wave per column
-// row is otherwise idle hardware (2.2x faster on a 72 x 44 x 136 grid).
+// y/z sweeps as two waves per 64 columns (k_sweep_col2) on the mixed path:
+// 1.42 ms per y sweep against 1.65 for k_sweep_col at 256^3 (250 registers,
+// no spill, two waves per SIMD).  The FP64 instance would spill 224 bytes per
+// lane at two waves per SIMD and is slower than k_sweep_col at every size and
+// segment measured (655 against 343 us at 128^3, 93 against 57 us at
+// 64 x 8 x 8, both at their best segment).
+
+// Cells per segment of the y/z column march over n cells and ncol columns.
+// A workgroup marches SWEEP_COLS columns and fills a CU (one wave, or one
+// producer/consumer pair, per SIMD), so the launch takes
+// ceil(workgroups / CUs) rounds of seg + COL_RAMP positions (the stencil's
+// run-in is 11 positions of partial work).  COL_RAMP = 5 (FP64) and 6
+// (mixed) fit the times measured over segments of 1..256 cells: 343 / 388 /
+// 604 us at 128^3 in FP64 with 32 / 16 / 64 cells (1, 2 and half a round),
+// 215 / 248 / 365 us mixed.  Whole columns on every grid left most CUs idle
+// below 256^3: 64^3 mixed 355 us per sweep against 62 (4 cells), 128^3 681
+// against 215 (32), FP64 200 x 72 x 136 along z 1726 (two waves) against
+// 452, 64 x 8 x 8 174 against 57 (1 cell).  256^3 keeps whole columns (1.43
+// / 2.33 ms; 128 cells 1.43 / 2.36, 64 cells 1.51 / 2.45).
+constexpr int COL_RAMP = 6;
+static int col_seg(const mcf_ctx *x, int n, long ncol) {
+  const long nb = (ncol + SWEEP_COLS - 1) / SWEEP_COLS;
+  int best = n;
+  long cost = -1;
+  for (int ns = 1; ns <= n; ++ns) {
+    const int seg = (n + ns - 1) / ns;
+    const long used = (n + seg - 1) / seg;
+    const long c = ((used * nb + x->ncu - 1) / x->ncu) * (seg + COL_RAMP);
+    if (cost < 0 || c < cost) { cost = c; best = seg; }
+  }
+  return best;
+}
 
 // ----------------------------------------------------------------------------
 // ghost fills
@@ -585,18 +606,16 @@ static int do_sweep(mcf_ctx *x, int d, double dt) {
     // One kernel instead of k_rhsmoc_col + k_remap_col (the MOC results no
     // longer go through HBM): 1.66 against 1.93 ms per sweep (mixed), 2.32
     // against 2.75 (FP64), at 1 wave per SIMD (354 / 450 registers); on the
-    // mixed path split over two waves per column row (k_sweep_col2)
+    // mixed path split over two waves per 64 columns (k_sweep_col2)
     const int n = x->g.n[d], ntr = x->g.n[d == 1 ? 2 : 1];
-    const int seg = x->col_seg;
-    dim3 gr((unsigned)((n + seg - 1) / seg), (unsigned)((x->g.n[0] + 63) / 64), (unsigned)((ntr + 3) / 4));
+    const long ncol = (long)x->g.n[0] * ntr;
+    const int seg = col_seg(x, n, ncol);
+    dim3 gr((unsigned)((n + seg - 1) / seg), (unsigned)((ncol + SWEEP_COLS - 1) / SWEEP_COLS), 1u);
     // reads rho, v(3), p, Bcc(3), face B_n, species(8); writes rho, v(3), p, species(8)
     const double by = 8.0 * (double)x->g.n[0] * x->g.n[1] * x->g.n[2] * 30;
     if (x->mixed) {
       if (d == 1) KLAUNCH_N("k_sweep_col2<1>", (k_sweep_col2<1, float>), gr, dim3(512), by, A, x->g, dt, seg);
       else KLAUNCH_N("k_sweep_col2<2>", (k_sweep_col2<2, float>), gr, dim3(512), by, A, x->g, dt, seg);
-    } else if ((long)gr.x * gr.y * gr.z < (long)x->ncu) {
-      if (d == 1) KLAUNCH_N("k_sweep_col2<1>", (k_sweep_col2<1, double>), gr, dim3(512), by, A, x->g, dt, seg);
-      else KLAUNCH_N("k_sweep_col2<2>", (k_sweep_col2<2, double>), gr, dim3(512), by, A, x->g, dt, seg);
     } else {
       if (d == 1) KLAUNCH_N("k_sweep_col<1>", (k_sweep_col<1, double>), gr, dim3(256), by, A, x->g, dt, seg);
       else KLAUNCH_N("k_sweep_col<2>", (k_sweep_col<2, double>), gr, dim3(256), by, A, x->g, dt, seg);

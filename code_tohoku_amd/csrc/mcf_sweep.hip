@@ -1082,11 +1082,11 @@ __global__ __launch_bounds__(256) void k_remap_col(SweepIO A, Geo g, double dt) 
 // coordinates (interface 0 = interface n of the last block).  For the cells
 // 1..n this is the evaluation of k_rhsmoc_col, which treats positions outside
 // 1..n as ghosts of the adjacent block.
-template <class R> struct MocOut {
-  double v[7]; // rho, m_n, m_t1, m_t2, E, Blg1, Blg2 (global component order via SweepIO)
-  double w;    // dx_lag
-  double va;   // V* of the interface to the right
-};
+//
+// Lanes take the columns of the (x, transverse) plane in order, x fastest, so
+// rows that are no multiple of 64 cells leave no lane idle but those of the
+// last workgroup (a 200-cell row in 64-cell tiles idles 22%).  The host picks
+// seg so that the workgroups fill the CUs (col_seg in mcf_host.hip).
 
 template <int D, class R>
 __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, int seg) {
@@ -1094,10 +1094,10 @@ __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, 
   constexpr int BT1 = (D + 1) % 3, BT2 = (D + 2) % 3;
   const int nx = g.n[0];
   const int n = g.n[D], ntr = g.n[D == 1 ? 2 : 1];
-  int bseg, bxc, btr;
-  xcd_tile(bseg, bxc, btr);
-  const int i = 1 + 64 * bxc + (int)(threadIdx.x & 63);
-  const int tr = 1 + 4 * btr + (int)(threadIdx.x >> 6);
+  int bseg, bcol, b2;
+  xcd_tile(bseg, bcol, b2);
+  const int id = SWEEP_COLS * bcol + (int)threadIdx.x; // column of the (x, transverse) plane, x fastest
+  const int tr = 1 + id / nx, i = 1 + id % nx;
   const int p0 = 1 + seg * bseg;
   const int p1 = min(n, p0 + seg - 1);
   const int m0 = p0 - 2; // first MOC result (m0 .. p1+2)
@@ -1107,7 +1107,7 @@ __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, 
   __shared__ double sxe[SWEEP_COL_MAXN + 4];
   for (int t = (int)threadIdx.x; t < n + 4; t += (int)blockDim.x) sxe[t] = A.xe[t];
   __syncthreads();
-  if (i > nx || tr > ntr || p0 > n) return;
+  if (tr > ntr || p0 > n) return;
   // image position of p (n >= 8, so one shift suffices for p0-6 .. p1+7)
   auto img = [&](int p) { return p < 1 ? p + n : (p > n ? p - n : p); };
   auto at = [&](int p) { return D == 1 ? ix3s(g, i, p, tr) : ix3s(g, i, tr, p); };
@@ -1379,28 +1379,28 @@ __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, 
   }
 }
 
-// A whole y or z sweep as k_sweep_col, over two waves per row of 64
+// A whole y or z sweep as k_sweep_col, over two waves per 64
 // columns: the producer wave runs the RHS and MOC chain and puts, per cell J,
 // its MOC-updated state (rho, m_n, m_t1, m_t2, E, Blg1, Blg2), dx_lag and V*
 // into an LDS slot; the consumer wave takes it one iteration later, forms
 // the Lagrangian species and remaps.  Each wave holds only its own windows,
 // so a SIMD runs a producer and a consumer wave side by side.  The arithmetic
-// is k_sweep_col's, statement for statement.  Lanes past the grid's end in x
-// or in the transverse axis march the last column and write nothing (every
-// wave reaches each barrier).
+// is k_sweep_col's, statement for statement.  Lanes past the last
+// column march it and write nothing (every wave reaches each barrier).
 template <int D, class R>
 __global__ __launch_bounds__(512) void k_sweep_col2(SweepIO A, Geo g, double dt, int seg) {
   constexpr int VN = D + 1, VT1 = (D + 1) % 3 + 1, VT2 = (D + 2) % 3 + 1;
   constexpr int BT1 = (D + 1) % 3, BT2 = (D + 2) % 3;
   const int nx = g.n[0];
   const int n = g.n[D], ntr = g.n[D == 1 ? 2 : 1];
-  int bseg, bxc, btr;
-  xcd_tile(bseg, bxc, btr);
+  int bseg, bcol, b2;
+  xcd_tile(bseg, bcol, b2);
   const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6, r4 = wv & 3;
   const bool producer = wv < 4;
-  const int i_ = 1 + 64 * bxc + lane, tr_ = 1 + 4 * btr + r4;
-  const bool act = i_ <= nx && tr_ <= ntr;
-  const int i = min(i_, nx), tr = min(tr_, ntr);
+  const int id_ = SWEEP_COLS * bcol + 64 * r4 + lane, ncol = nx * ntr;
+  const bool act = id_ < ncol;
+  const int id = min(id_, ncol - 1);
+  const int tr = 1 + id / nx, i = 1 + id % nx;
   const int p0 = 1 + seg * bseg;
   const int p1 = min(n, p0 + seg - 1);
   const int m0 = p0 - 2; // first MOC result (m0 .. p1+2)
@@ -2190,8 +2190,6 @@ template __global__ void k_rhsmoc_col<1, float>(SweepIO, Geo, double);
 template __global__ void k_rhsmoc_col<2, float>(SweepIO, Geo, double);
 template __global__ void k_sweep_col<1, double>(SweepIO, Geo, double, int);
 template __global__ void k_sweep_col<2, double>(SweepIO, Geo, double, int);
-template __global__ void k_sweep_col2<1, double>(SweepIO, Geo, double, int);
-template __global__ void k_sweep_col2<2, double>(SweepIO, Geo, double, int);
 template __global__ void k_sweep_col2<1, float>(SweepIO, Geo, double, int);
 template __global__ void k_sweep_col2<2, float>(SweepIO, Geo, double, int);
 template __global__ void k_remap_col<1, double>(SweepIO, Geo, double);

@@ -1,0 +1,61 @@
+"""Launch shapes of the kernels that split the grid by a rule on its sizes,
+against the oracle at the sizes where a split can go wrong: segments of one
+cell, a last segment or workgroup that is nearly empty, rows that are no
+multiple of a wavefront, block edges inside and at the ends of a segment.
+
+FP64 is held to 1e-12 per field after one step (the bound of the other
+parity tests: the operations are the oracle's, the transcendentals may
+differ by an ulp); mixed precision to 1e-5 (FP32 rates and states)."""
+import numpy as np
+import pytest
+
+import oracle
+from code_tohoku_amd import ics, mcf
+from code_tohoku_amd.restart import Input3D
+from helpers import interior, rel_linf, worst
+
+pytestmark = pytest.mark.gpu
+
+
+def box(nx, ny, nz, periodic):
+    q = 0.25  # cell size: a power of two, so every spacing is the same bits
+    p = Input3D(np1x=nx // 2, np2x=nx - nx // 2, np1y=ny // 2, np2y=ny - ny // 2, np1z=nz // 2, np2z=nz - nz // 2,
+                ql1x=q * (nx // 2), ql2x=q * (nx - nx // 2), ql1y=q * (ny // 2), ql2y=q * (ny - ny // 2),
+                ql1z=q * (nz // 2), ql2z=q * (nz - nz // 2))
+    if periodic:
+        p.bcx1 = p.bcx2 = 3
+    return p
+
+
+def check_step(p, st, nsplit, precision):
+    o = oracle.Oracle(p, st, nsplit=nsplit)
+    g = mcf.Domain(p, nsplit=nsplit, precision=precision)
+    g.upload(st)
+    dts, _ = o.run(1)
+    assert len(dts) == 1
+    if precision == mcf.PREC_FP64:
+        np.testing.assert_allclose(g.run(1), dts, rtol=1e-13)
+    else:
+        g.step(dts[0])
+    got, ref = interior(g.download(), p), interior(o.state(), p)
+    g.close()
+    if precision == mcf.PREC_FP64:
+        errs = rel_linf(got, ref)
+        assert worst(errs) <= 1e-12, errs
+    else:
+        for f in range(8):
+            assert np.abs(got[f] - ref[f]).max() <= 1e-5 * np.abs(ref[f]).max(), f
+
+
+@pytest.mark.parametrize("precision", [mcf.PREC_FP64, mcf.PREC_MIXED])
+@pytest.mark.parametrize("n,nsplit,periodic", [
+    ((12, 8, 9), (1, 1, 1), False),     # one-cell segments, fewer columns than a workgroup takes
+    ((33, 17, 23), (1, 1, 1), True),    # odd sides, unequal halves
+    ((66, 18, 40), (3, 2, 4), False),   # rows of 64 + 2 cells; blocks of 9 and 10 cells
+    ((130, 65, 31), (5, 5, 1), True),   # the last segment shorter than the others
+    ((61, 122, 10), (1, 2, 2), False),  # x rows of exactly one CT tile; blocks of 5 cells along z
+])
+def test_step_shapes_vs_oracle(n, nsplit, periodic, precision):
+    p = box(*n, periodic)
+    print("shape", n, nsplit, precision, flush=True)
+    check_step(p, ics.random_state(p, seed=sum(n)), nsplit, precision)

@@ -291,8 +291,8 @@ static long boxsize(const Box &b) { return (long)b.cnt[0] * b.cnt[1] * b.cnt[2];
   } while (0)
 
 // y/z sweeps as two waves per 64 columns (k_sweep_col2) on the mixed path:
-// 1.42 ms per y sweep against 1.65 for k_sweep_col at 256^3 (250 registers,
-// no spill, two waves per SIMD).  The FP64 instance would spill 224 bytes per
+// 16% faster than k_sweep_col at 256^3 (245 registers, no spill, two waves
+// per SIMD).  The FP64 instance would spill 224 bytes per
 // lane at two waves per SIMD and is slower than k_sweep_col at every size and
 // segment measured (655 against 343 us at 128^3, 93 against 57 us at
 // 64 x 8 x 8, both at their best segment).
@@ -603,10 +603,9 @@ static int do_sweep(mcf_ctx *x, int d, double dt) {
   } else if (x->fuse[d] && x->g.n[d] <= SWEEP_COL_MAXN) {
     // y/z: the whole sweep in one column march over the periodic axis; it
     // reads only interior cells (periodic images), so no fills precede it.
-    // One kernel instead of k_rhsmoc_col + k_remap_col (the MOC results no
-    // longer go through HBM): 1.66 against 1.93 ms per sweep (mixed), 2.32
-    // against 2.75 (FP64), at 1 wave per SIMD (354 / 450 registers); on the
-    // mixed path split over two waves per 64 columns (k_sweep_col2)
+    // One kernel instead of k_rhsmoc_col + k_remap_col: the MOC results do
+    // not go through HBM (14% less time in both precisions when measured).
+    // 1.04 / 1.79 ms per sweep at 256^3 (mixed / FP64)
     const int n = x->g.n[d], ntr = x->g.n[d == 1 ? 2 : 1];
     const long ncol = (long)x->g.n[0] * ntr;
     const int seg = col_seg(x, n, ncol);

@@ -345,11 +345,10 @@ __device__ __forceinline__ void rhs_states(double rho, double vn, double p, doub
                                            double dx0_d, double dxp_d, double dt, double facdep, R *q) {
   const R dxm = (R)dxm_d, dx0 = (R)dx0_d, dxp = (R)dxp_d;
   const bool mm = use_minmod_r<R>(p, rho);
-  const R g1 = vslope<R>(r_m, rho, r_p, dxm, dx0, dxp, mm);
-  const R gv = vslope<R>(v_m, vn, v_p, dxm, dx0, dxp, mm);
-  const R g5 = vslope<R>(p_m, p, p_p, dxm, dx0, dxp, mm);
-  const R gA = vslope<R>(a_m, b1, a_p, dxm, dx0, dxp, mm);
-  const R gB = vslope<R>(c_m, b2, c_p, dxm, dx0, dxp, mm);
+  const double qm[5] = {r_m, v_m, p_m, a_m, c_m}, q0[5] = {rho, vn, p, b1, b2}, qp[5] = {r_p, v_p, p_p, a_p, c_p};
+  R sl[5];
+  cell_slopes<R, 5>(qm, q0, qp, dxm, dx0, dxp, mm, sl);
+  const R g1 = sl[0], gv = sl[1], g5 = sl[2], gA = sl[3], gB = sl[4];
   R gamma;
   if constexpr (Ar<R>::strict) {
     double s4 = spc[0] + spc[1] + spc[3] + spc[4];
@@ -722,11 +721,12 @@ __global__ __launch_bounds__(256) void k_rhsmoc_col(SweepIO A, Geo g, double dt)
         double gg = 3.0 * s4 + 5.0 * spl[2];
         double gi = (2.0 * s4 + 2.0 * spl[2]) / gg;
         double e = p / (rho * gi) + 0.5 * (vx * vx + vy * vy + vz * vz) + 0.5 * (bx * bx + by * by + bz * bz) / rho;
-        rhoL = dm / dxl;
+        const Quot odl(dxl);
+        rhoL = odl(dm);
         vnL = vn - dt / dm * (pa - pam);
         eL = e - dt / dm * (pa * va - pam * vam);
-        bl1 = b1 * dxu / dxl;
-        bl2 = b2 * dxu / dxl;
+        bl1 = odl(b1 * dxu);
+        bl2 = odl(b2 * dxu);
       } else {
         double s4 = spl[0] + spl[1] + spl[3] + spl[4];
         double irho = 1.0 / rho;
@@ -756,11 +756,9 @@ __global__ __launch_bounds__(256) void k_rhsmoc_col(SweepIO A, Geo g, double dt)
         const bool inner = km >= 1 && km <= n;
         const bool mm = inner ? o1.mme : o1.mmp;
         const R dxm = (R)o0.v[5], dx0 = (R)o1.v[5], dxp = (R)o2.v[5];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) G1[v] = vslope<R>(o0.v[v], o1.v[v], o2.v[v], dxm, dx0, dxp, mm);
+        cell_slopes<R, 5>(o0.v, o1.v, o2.v, dxm, dx0, dxp, mm, G1);
         if ((km % nblk == 0 || (km - 1) % nblk == 0) && o1.mmp != mm) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) H1[v] = vslope<R>(o0.v[v], o1.v[v], o2.v[v], dxm, dx0, dxp, o1.mmp);
+          cell_slopes<R, 5>(o0.v, o1.v, o2.v, dxm, dx0, dxp, o1.mmp, H1);
         }
         if (k >= p0 + 1) {
           // interface J = k-2 between cells J and J+1 (local positions 0..n)
@@ -1148,12 +1146,13 @@ __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, 
   for (int v = 0; v < 5; ++v) { G0[v] = G1[v] = H0[v] = H1[v] = (R)0; }
   MocV<R> rvp{};            // right view of interface J-1
   double bnp = 0, vap = 0;  // B_n of interface J-1 in the right view, V* of J-1
-  // ---- REMAP window: remapped quantities of cells Jf-1 .. Jf+2 (15 each),
-  // their dx_lag, V* of face Jf, the flux of face Jf-1
-  double Q0[15], Q1[15], Q2[15], Q3[15], W0 = 0, W1 = 0, W2 = 0, W3 = 0, V1 = 0, V2 = 0, V3 = 0;
+  // ---- REMAP window: remapped quantities of cells Jf .. Jf+2 (15 each),
+  // their dx_lag, V* of face Jf, the slopes of cell Jf, the flux of face Jf-1
+  double Q1[15], Q2[15], Q3[15], W1 = 0, W2 = 0, W3 = 0, V1 = 0, V2 = 0, V3 = 0;
   double Fp[15];
+  R Gr[15];
 #pragma unroll
-  for (int v = 0; v < 15; ++v) { Q0[v] = Q1[v] = Q2[v] = Q3[v] = 0.0; Fp[v] = 0.0; }
+  for (int v = 0; v < 15; ++v) { Q1[v] = Q2[v] = Q3[v] = 0.0; Fp[v] = 0.0; Gr[v] = (R)0; }
   // pre-sweep species of the cell whose MOC result enters REMAP's window in
   // this iteration (J = q-3) and B_n of the cell REMAP updates (q-5), each
   // loaded one iteration ahead
@@ -1199,28 +1198,16 @@ __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, 
       const double dxl = xl - xlm;
       const double *spl = spw[0];
       double rhoL, vnL, eL, bl1, bl2;
-      if constexpr (Ar<R>::strict) {
-        double s4 = spl[0] + spl[1] + spl[3] + spl[4];
-        double gg = 3.0 * s4 + 5.0 * spl[2];
-        double gi = (2.0 * s4 + 2.0 * spl[2]) / gg;
-        double e = p / (rho * gi) + 0.5 * (vx * vx + vy * vy + vz * vz) + 0.5 * (bx * bx + by * by + bz * bz) / rho;
-        rhoL = dm / dxl;
-        vnL = vn - dt / dm * (pa - pam);
-        eL = e - dt / dm * (pa * va - pam * vam);
-        bl1 = b1 * dxu / dxl;
-        bl2 = b2 * dxu / dxl;
-      } else {
-        double s4 = spl[0] + spl[1] + spl[3] + spl[4];
-        double irho = 1.0 / rho;
-        double e = p * (3.0 * s4 + 5.0 * spl[2]) / (2.0 * s4 + 2.0 * spl[2]) * irho +
-                   0.5 * (vx * vx + vy * vy + vz * vz) + 0.5 * (bx * bx + by * by + bz * bz) * irho;
-        double idl = 1.0 / dxl, dtdm = dt / dm, cmp = dxu * idl;
-        rhoL = dm * idl;
-        vnL = vn - dtdm * (pa - pam);
-        eL = e - dtdm * (pa * va - pam * vam);
-        bl1 = b1 * cmp;
-        bl2 = b2 * cmp;
-      }
+      double s4 = spl[0] + spl[1] + spl[3] + spl[4];
+      double gg = 3.0 * s4 + 5.0 * spl[2];
+      double gi = (2.0 * s4 + 2.0 * spl[2]) / gg;
+      double e = p / (rho * gi) + 0.5 * (vx * vx + vy * vy + vz * vz) + 0.5 * (bx * bx + by * by + bz * bz) / rho;
+      const Quot odl(dxl);
+      rhoL = odl(dm);
+      vnL = vn - dt / dm * (pa - pam);
+      eL = e - dt / dm * (pa * va - pam * vam);
+      bl1 = odl(b1 * dxu);
+      bl2 = odl(b2 * dxu);
       o2.v[0] = rhoL; o2.v[1] = vt1; o2.v[2] = vt2; o2.v[3] = bl1; o2.v[4] = bl2; o2.v[5] = dxl;
       o2.vn = vnL; o2.e = eL;
       o2.mme = use_minmod_r<R>(eL, rhoL);
@@ -1233,11 +1220,9 @@ __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, 
         const int km = k - 1;
         const bool mm = o1.mme;
         const R dxm = (R)o0.v[5], dx0 = (R)o1.v[5], dxp = (R)o2.v[5];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) G1[v] = vslope<R>(o0.v[v], o1.v[v], o2.v[v], dxm, dx0, dxp, mm);
+        cell_slopes<R, 5>(o0.v, o1.v, o2.v, dxm, dx0, dxp, mm, G1);
         if ((km % nblk == 0 || (km - 1) % nblk == 0) && o1.mmp != mm) {
-#pragma unroll
-          for (int v = 0; v < 5; ++v) H1[v] = vslope<R>(o0.v[v], o1.v[v], o2.v[v], dxm, dx0, dxp, o1.mmp);
+          cell_slopes<R, 5>(o0.v, o1.v, o2.v, dxm, dx0, dxp, o1.mmp, H1);
         }
         if (k >= m0 + 1) {
           // interface J = k-2 between cells J and J+1; the owners of J and
@@ -1262,67 +1247,49 @@ __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, 
             const double dxl0 = o0.v[5], rho0 = o0.v[0];
             const double BayL = (double)L.Bay, VayL = (double)L.Vay, BazL = (double)L.Baz, VazL = (double)L.Vaz;
             const double BayR = (double)rvp.Bay, VayR = (double)rvp.Vay, BazR = (double)rvp.Baz, VazR = (double)rvp.Vaz;
-            if constexpr (Ar<R>::strict) {
-              Q3[VN] = o0.vn * rho0 + dt / dxl0 * 0.5 * (Bnap * Bnap - Bnam * Bnam);
-              Q3[VT1] = o0.v[1] * rho0 + dt / dxl0 * (Bnap * BayL - Bnam * BayR);
-              Q3[VT2] = o0.v[2] * rho0 + dt / dxl0 * (Bnap * BazL - Bnam * BazR);
-              Q3[4] = o0.e * rho0 + dt / dxl0 *
-                                        ((0.5 * Bnap * Vnap + BayL * VayL + BazL * VazL) * Bnap -
-                                         (0.5 * Bnam * Vnam + BayR * VayR + BazR * VazR) * Bnam);
-              Q3[5] = o0.v[3] + dt / dxl0 * (Bnap * VayL - Bnam * VayR);
-              Q3[6] = o0.v[4] + dt / dxl0 * (Bnap * VazL - Bnam * VazR);
-            } else {
-              const double fq = dt / dxl0;
-              Q3[VN] = o0.vn * rho0 + fq * 0.5 * (Bnap * Bnap - Bnam * Bnam);
-              Q3[VT1] = o0.v[1] * rho0 + fq * (Bnap * BayL - Bnam * BayR);
-              Q3[VT2] = o0.v[2] * rho0 + fq * (Bnap * BazL - Bnam * BazR);
-              Q3[4] = o0.e * rho0 + fq * ((0.5 * Bnap * Vnap + BayL * VayL + BazL * VazL) * Bnap -
-                                          (0.5 * Bnam * Vnam + BayR * VayR + BazR * VazR) * Bnam);
-              Q3[5] = o0.v[3] + fq * (Bnap * VayL - Bnam * VayR);
-              Q3[6] = o0.v[4] + fq * (Bnap * VazL - Bnam * VazR);
-            }
+            Q3[VN] = o0.vn * rho0 + dt / dxl0 * 0.5 * (Bnap * Bnap - Bnam * Bnam);
+            Q3[VT1] = o0.v[1] * rho0 + dt / dxl0 * (Bnap * BayL - Bnam * BayR);
+            Q3[VT2] = o0.v[2] * rho0 + dt / dxl0 * (Bnap * BazL - Bnam * BazR);
+            Q3[4] = o0.e * rho0 + dt / dxl0 *
+                                      ((0.5 * Bnap * Vnap + BayL * VayL + BazL * VazL) * Bnap -
+                                       (0.5 * Bnam * Vnam + BayR * VayR + BazR * VazR) * Bnam);
+            Q3[5] = o0.v[3] + dt / dxl0 * (Bnap * VayL - Bnam * VayR);
+            Q3[6] = o0.v[4] + dt / dxl0 * (Bnap * VazL - Bnam * VazR);
             Q3[0] = rho0;
             W3 = dxl0;
             V3 = Vnap;
             // Lagrangian species of cell J (M3:1466) from the pre-sweep ones
-            if constexpr (Ar<R>::strict) {
+            const Quot odl(dxl0);
 #pragma unroll
-              for (int f = 0; f < 8; ++f) Q3[7 + f] = dxu * csp[f] / dxl0;
-            } else {
-              const double cmp = dxu * (1.0 / dxl0);
-#pragma unroll
-              for (int f = 0; f < 8; ++f) Q3[7 + f] = csp[f] * cmp;
-            }
-            // REMAP of face Jf = J-2 (cells Jf-1 .. Jf+2 in Q0 .. Q3) and of
-            // cell Jf (faces Jf-1 and Jf)
+            for (int f = 0; f < 8; ++f) Q3[7 + f] = odl(dxu * csp[f]);
+            // REMAP of face Jf = J-2 (cells Jf .. Jf+2 in Q1 .. Q3, the slope of
+            // cell Jf in Gr) and of cell Jf (faces Jf-1 and Jf); five quantities
+            // at a time keep the temporaries few
             const int Jf = J - 2;
-            if (Jf >= p0 - 1) {
+            if (Jf >= p0 - 2) {
               const double vadt = V1 * dt;
               const bool up = !(vadt <= 0.0);
-              const double u4 = up ? Q1[4] : Q2[4], u0 = up ? Q1[0] : Q2[0];
               const double depend = up ? 0.5 * (W1 - vadt) * A.facdep : 0.5 * (W2 + vadt) * A.facdep;
-              const R dxm2 = (R)(up ? W0 : W1), dx02 = (R)(up ? W1 : W2), dxp2 = (R)(up ? W2 : W3);
-              const bool mmr = use_minmod_r<R>(u4, u0);
-              const R rdep = (R)depend;
-              double F[15];
+              const R sdep = up ? (R)depend : -(R)depend;
+              const bool mmr = use_minmod_r<R>(Q2[4], Q2[0]);
+              const Quot over(xe[max(Jf, 0) + 1] - xe[max(Jf, 0)]);
+              double Qn[15];
 #pragma unroll
-              for (int v = 0; v < 15; ++v) {
-                const R gr = vslope<R>(up ? Q0[v] : Q1[v], up ? Q1[v] : Q2[v], up ? Q2[v] : Q3[v], dxm2, dx02, dxp2, mmr);
-                const double qu = up ? Q1[v] : Q2[v];
-                double face;
-                if constexpr (Ar<R>::strict) face = up ? qu + depend * gr : qu - depend * gr;
-                else face = up ? qu + (double)(rdep * gr) : qu - (double)(rdep * gr);
-                F[v] = -(vadt * face);
+              for (int b = 0; b < 15; b += 5) {
+                R gn[5];
+                cell_slopes<R, 5>(Q1 + b, Q2 + b, Q3 + b, (R)W1, (R)W2, (R)W3, mmr, gn);
+#pragma unroll
+                for (int v = 0; v < 5; ++v) {
+                  const double face = (up ? Q1[b + v] : Q2[b + v]) + (double)(sdep * (up ? Gr[b + v] : gn[v]));
+                  const double F = -(vadt * face);
+                  const double num = Q1[b + v] * W1 + F - Fp[b + v];
+                  Qn[b + v] = over(num);
+                  Fp[b + v] = F;
+                  Gr[b + v] = gn[v];
+                }
               }
               if (Jf >= p0) {
                 // remapped conserved state (M3:1645-1686), primitives (M3:1291-1321)
-                const double dxE = xe[Jf + 1] - xe[Jf];
-                double Qn[15];
-#pragma unroll
-                for (int v = 0; v < 15; ++v) {
-                  if constexpr (Ar<R>::strict) Qn[v] = (Q1[v] * W1 + F[v] - Fp[v]) / dxE;
-                  else Qn[v] = (Q1[v] * W1 + F[v] - Fp[v]) * (1.0 / dxE);
-                }
                 const int c = at(Jf);
                 const double bn = cbn;
                 double rho = dmax(1.27 * A.rmin, Qn[0]);
@@ -1344,12 +1311,10 @@ __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, 
 #pragma unroll
                 for (int f = 0; f < 8; ++f) A.spo[f][c] = dmax(A.spmin[f], Qn[7 + f]);
               }
-#pragma unroll
-              for (int v = 0; v < 15; ++v) Fp[v] = F[v];
             }
 #pragma unroll
-            for (int v = 0; v < 15; ++v) { Q0[v] = Q1[v]; Q1[v] = Q2[v]; Q2[v] = Q3[v]; }
-            W0 = W1; W1 = W2; W2 = W3;
+            for (int v = 0; v < 15; ++v) { Q1[v] = Q2[v]; Q2[v] = Q3[v]; }
+            W1 = W2; W2 = W3;
             V1 = V2; V2 = V3;
           }
           rvp = Rv;
@@ -1482,28 +1447,16 @@ __global__ __launch_bounds__(512) void k_sweep_col2(SweepIO A, Geo g, double dt,
         const double dxl = xl - xlm;
         const double *spl = spw[0];
         double rhoL, vnL, eL, bl1, bl2;
-        if constexpr (Ar<R>::strict) {
-          double s4 = spl[0] + spl[1] + spl[3] + spl[4];
-          double gg = 3.0 * s4 + 5.0 * spl[2];
-          double gi = (2.0 * s4 + 2.0 * spl[2]) / gg;
-          double e = p / (rho * gi) + 0.5 * (vx * vx + vy * vy + vz * vz) + 0.5 * (bx * bx + by * by + bz * bz) / rho;
-          rhoL = dm / dxl;
-          vnL = vn - dt / dm * (pa - pam);
-          eL = e - dt / dm * (pa * va - pam * vam);
-          bl1 = b1 * dxu / dxl;
-          bl2 = b2 * dxu / dxl;
-        } else {
-          double s4 = spl[0] + spl[1] + spl[3] + spl[4];
-          double irho = 1.0 / rho;
-          double e = p * (3.0 * s4 + 5.0 * spl[2]) / (2.0 * s4 + 2.0 * spl[2]) * irho +
-                     0.5 * (vx * vx + vy * vy + vz * vz) + 0.5 * (bx * bx + by * by + bz * bz) * irho;
-          double idl = 1.0 / dxl, dtdm = dt / dm, cmp = dxu * idl;
-          rhoL = dm * idl;
-          vnL = vn - dtdm * (pa - pam);
-          eL = e - dtdm * (pa * va - pam * vam);
-          bl1 = b1 * cmp;
-          bl2 = b2 * cmp;
-        }
+        double s4 = spl[0] + spl[1] + spl[3] + spl[4];
+        double irho = 1.0 / rho;
+        double e = p * (3.0 * s4 + 5.0 * spl[2]) / (2.0 * s4 + 2.0 * spl[2]) * irho +
+                   0.5 * (vx * vx + vy * vy + vz * vz) + 0.5 * (bx * bx + by * by + bz * bz) * irho;
+        double idl = 1.0 / dxl, dtdm = dt / dm, cmp = dxu * idl;
+        rhoL = dm * idl;
+        vnL = vn - dtdm * (pa - pam);
+        eL = e - dtdm * (pa * va - pam * vam);
+        bl1 = b1 * cmp;
+        bl2 = b2 * cmp;
         o2.v[0] = rhoL; o2.v[1] = vt1; o2.v[2] = vt2; o2.v[3] = bl1; o2.v[4] = bl2; o2.v[5] = dxl;
         o2.vn = vnL; o2.e = eL;
         o2.mme = use_minmod_r<R>(eL, rhoL);
@@ -1516,11 +1469,9 @@ __global__ __launch_bounds__(512) void k_sweep_col2(SweepIO A, Geo g, double dt,
           const int km = k - 1;
           const bool mm = o1.mme;
           const R dxm = (R)o0.v[5], dx0 = (R)o1.v[5], dxp = (R)o2.v[5];
-#pragma unroll
-          for (int v = 0; v < 5; ++v) G1[v] = vslope<R>(o0.v[v], o1.v[v], o2.v[v], dxm, dx0, dxp, mm);
+          cell_slopes<R, 5>(o0.v, o1.v, o2.v, dxm, dx0, dxp, mm, G1);
           if ((km % nblk == 0 || (km - 1) % nblk == 0) && o1.mmp != mm) {
-#pragma unroll
-            for (int v = 0; v < 5; ++v) H1[v] = vslope<R>(o0.v[v], o1.v[v], o2.v[v], dxm, dx0, dxp, o1.mmp);
+            cell_slopes<R, 5>(o0.v, o1.v, o2.v, dxm, dx0, dxp, o1.mmp, H1);
           }
           if (k >= m0 + 1) {
             // interface J = k-2 between cells J and J+1; the owners of J and
@@ -1546,25 +1497,14 @@ __global__ __launch_bounds__(512) void k_sweep_col2(SweepIO A, Geo g, double dt,
               const double BayL = (double)L.Bay, VayL = (double)L.Vay, BazL = (double)L.Baz, VazL = (double)L.Vaz;
               const double BayR = (double)rvp.Bay, VayR = (double)rvp.Vay, BazR = (double)rvp.Baz, VazR = (double)rvp.Vaz;
               double Q3[7];
-              if constexpr (Ar<R>::strict) {
-                Q3[VN] = o0.vn * rho0 + dt / dxl0 * 0.5 * (Bnap * Bnap - Bnam * Bnam);
-                Q3[VT1] = o0.v[1] * rho0 + dt / dxl0 * (Bnap * BayL - Bnam * BayR);
-                Q3[VT2] = o0.v[2] * rho0 + dt / dxl0 * (Bnap * BazL - Bnam * BazR);
-                Q3[4] = o0.e * rho0 + dt / dxl0 *
-                                          ((0.5 * Bnap * Vnap + BayL * VayL + BazL * VazL) * Bnap -
-                                           (0.5 * Bnam * Vnam + BayR * VayR + BazR * VazR) * Bnam);
-                Q3[5] = o0.v[3] + dt / dxl0 * (Bnap * VayL - Bnam * VayR);
-                Q3[6] = o0.v[4] + dt / dxl0 * (Bnap * VazL - Bnam * VazR);
-              } else {
-                const double fq = dt / dxl0;
-                Q3[VN] = o0.vn * rho0 + fq * 0.5 * (Bnap * Bnap - Bnam * Bnam);
-                Q3[VT1] = o0.v[1] * rho0 + fq * (Bnap * BayL - Bnam * BayR);
-                Q3[VT2] = o0.v[2] * rho0 + fq * (Bnap * BazL - Bnam * BazR);
-                Q3[4] = o0.e * rho0 + fq * ((0.5 * Bnap * Vnap + BayL * VayL + BazL * VazL) * Bnap -
-                                            (0.5 * Bnam * Vnam + BayR * VayR + BazR * VazR) * Bnam);
-                Q3[5] = o0.v[3] + fq * (Bnap * VayL - Bnam * VayR);
-                Q3[6] = o0.v[4] + fq * (Bnap * VazL - Bnam * VazR);
-              }
+              const double fq = dt / dxl0;
+              Q3[VN] = o0.vn * rho0 + fq * 0.5 * (Bnap * Bnap - Bnam * Bnam);
+              Q3[VT1] = o0.v[1] * rho0 + fq * (Bnap * BayL - Bnam * BayR);
+              Q3[VT2] = o0.v[2] * rho0 + fq * (Bnap * BazL - Bnam * BazR);
+              Q3[4] = o0.e * rho0 + fq * ((0.5 * Bnap * Vnap + BayL * VayL + BazL * VazL) * Bnap -
+                                          (0.5 * Bnam * Vnam + BayR * VayR + BazR * VazR) * Bnam);
+              Q3[5] = o0.v[3] + fq * (Bnap * VayL - Bnam * VayR);
+              Q3[6] = o0.v[4] + fq * (Bnap * VazL - Bnam * VazR);
               Q3[0] = rho0;
 #pragma unroll
               for (int v = 0; v < 7; ++v) hand[q & 1][v][r4][lane] = Q3[v];
@@ -1594,12 +1534,13 @@ __global__ __launch_bounds__(512) void k_sweep_col2(SweepIO A, Geo g, double dt,
       vt1 = nvt1; vt2 = nvt2; bnc = nbnc; fb = nfb;
     }
   } else {
-    // ---- REMAP window: remapped quantities of cells Jf-1 .. Jf+2 (15 each),
-    // their dx_lag, V* of face Jf, the flux of face Jf-1
-    double Q0[15], Q1[15], Q2[15], Q3[15], W0 = 0, W1 = 0, W2 = 0, W3 = 0, V1 = 0, V2 = 0, V3 = 0;
+    // ---- REMAP window: remapped quantities of cells Jf .. Jf+2 (15 each),
+    // their dx_lag, V* of face Jf, the slopes of cell Jf, the flux of face Jf-1
+    double Q1[15], Q2[15], Q3[15], W1 = 0, W2 = 0, W3 = 0, V1 = 0, V2 = 0, V3 = 0;
     double Fp[15];
+    R Gr[15];
 #pragma unroll
-    for (int v = 0; v < 15; ++v) { Q0[v] = Q1[v] = Q2[v] = Q3[v] = 0.0; Fp[v] = 0.0; }
+    for (int v = 0; v < 15; ++v) { Q1[v] = Q2[v] = Q3[v] = 0.0; Fp[v] = 0.0; Gr[v] = (R)0; }
     // pre-sweep species of the cell whose MOC result enters REMAP's window in
     // this iteration (J = q-3) and B_n of the cell REMAP updates (q-5), each
     // loaded one iteration ahead
@@ -1630,44 +1571,37 @@ __global__ __launch_bounds__(512) void k_sweep_col2(SweepIO A, Geo g, double dt,
         W3 = dxl0;
         V3 = hand[q & 1][8][r4][lane];
         // Lagrangian species of cell J (M3:1466) from the pre-sweep ones
-        if constexpr (Ar<R>::strict) {
+        const double cmp = dxu * (1.0 / dxl0);
 #pragma unroll
-          for (int f = 0; f < 8; ++f) Q3[7 + f] = dxu * csp[f] / dxl0;
-        } else {
-          const double cmp = dxu * (1.0 / dxl0);
-#pragma unroll
-          for (int f = 0; f < 8; ++f) Q3[7 + f] = csp[f] * cmp;
-        }
-        // REMAP of face Jf = J-2 (cells Jf-1 .. Jf+2 in Q0 .. Q3) and of
-        // cell Jf (faces Jf-1 and Jf)
+        for (int f = 0; f < 8; ++f) Q3[7 + f] = csp[f] * cmp;
+        // REMAP of face Jf = J-2 (cells Jf .. Jf+2 in Q1 .. Q3, the slope of
+        // cell Jf in Gr) and of cell Jf (faces Jf-1 and Jf); five quantities
+        // at a time keep the temporaries few
         const int Jf = J - 2;
-        if (Jf >= p0 - 1) {
+        if (Jf >= p0 - 2) {
           const double vadt = V1 * dt;
           const bool up = !(vadt <= 0.0);
-          const double u4 = up ? Q1[4] : Q2[4], u0 = up ? Q1[0] : Q2[0];
           const double depend = up ? 0.5 * (W1 - vadt) * A.facdep : 0.5 * (W2 + vadt) * A.facdep;
-          const R dxm2 = (R)(up ? W0 : W1), dx02 = (R)(up ? W1 : W2), dxp2 = (R)(up ? W2 : W3);
-          const bool mmr = use_minmod_r<R>(u4, u0);
-          const R rdep = (R)depend;
-          double F[15];
+          const R sdep = up ? (R)depend : -(R)depend;
+          const bool mmr = use_minmod_r<R>(Q2[4], Q2[0]);
+          const Quot over(xe[max(Jf, 0) + 1] - xe[max(Jf, 0)]);
+          double Qn[15];
 #pragma unroll
-          for (int v = 0; v < 15; ++v) {
-            const R gr = vslope<R>(up ? Q0[v] : Q1[v], up ? Q1[v] : Q2[v], up ? Q2[v] : Q3[v], dxm2, dx02, dxp2, mmr);
-            const double qu = up ? Q1[v] : Q2[v];
-            double face;
-            if constexpr (Ar<R>::strict) face = up ? qu + depend * gr : qu - depend * gr;
-            else face = up ? qu + (double)(rdep * gr) : qu - (double)(rdep * gr);
-            F[v] = -(vadt * face);
+          for (int b = 0; b < 15; b += 5) {
+            R gn[5];
+            cell_slopes<R, 5>(Q1 + b, Q2 + b, Q3 + b, (R)W1, (R)W2, (R)W3, mmr, gn);
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+              const double face = (up ? Q1[b + v] : Q2[b + v]) + (double)(sdep * (up ? Gr[b + v] : gn[v]));
+              const double F = -(vadt * face);
+              const double num = Q1[b + v] * W1 + F - Fp[b + v];
+              Qn[b + v] = num * over.y;
+              Fp[b + v] = F;
+              Gr[b + v] = gn[v];
+            }
           }
           if (Jf >= p0 && act) {
             // remapped conserved state (M3:1645-1686), primitives (M3:1291-1321)
-            const double dxE = xe[Jf + 1] - xe[Jf];
-            double Qn[15];
-#pragma unroll
-            for (int v = 0; v < 15; ++v) {
-              if constexpr (Ar<R>::strict) Qn[v] = (Q1[v] * W1 + F[v] - Fp[v]) / dxE;
-              else Qn[v] = (Q1[v] * W1 + F[v] - Fp[v]) * (1.0 / dxE);
-            }
             const int c = at(Jf);
             const double bn = cbn;
             double rho = dmax(1.27 * A.rmin, Qn[0]);
@@ -1689,12 +1623,10 @@ __global__ __launch_bounds__(512) void k_sweep_col2(SweepIO A, Geo g, double dt,
 #pragma unroll
             for (int f = 0; f < 8; ++f) A.spo[f][c] = dmax(A.spmin[f], Qn[7 + f]);
           }
-#pragma unroll
-          for (int v = 0; v < 15; ++v) Fp[v] = F[v];
         }
 #pragma unroll
-        for (int v = 0; v < 15; ++v) { Q0[v] = Q1[v]; Q1[v] = Q2[v]; Q2[v] = Q3[v]; }
-        W0 = W1; W1 = W2; W2 = W3;
+        for (int v = 0; v < 15; ++v) { Q1[v] = Q2[v]; Q2[v] = Q3[v]; }
+        W1 = W2; W2 = W3;
         V1 = V2; V2 = V3;
       }
 #pragma unroll
@@ -1725,6 +1657,48 @@ __global__ __launch_bounds__(512) void k_sweep_col2(SweepIO A, Geo g, double dt,
 // those of k_moc.  The Lagrangian species go to HBM for REMAP.
 template <class R> __device__ __forceinline__ R sh_up(R v) { return __shfl_up(v, 1u, 64); }
 template <class R> __device__ __forceinline__ R sh_dn(R v) { return __shfl_down(v, 1u, 64); }
+
+// REMAP of lane p's cell (M3:1600-1686) from the wave's cells: each lane
+// forms its own cell's slopes once; the upwind flux through face p|p+1 takes
+// them from lane p or p+1, the flux of face p-1|p comes from the lane below.
+// W0, W1, W2: Lagrangian widths of p-1, p, p+1.  Five quantities at a time
+// keep the temporaries out of scratch.
+template <class R>
+__device__ __forceinline__ void x_remap(const double *Q, double W0, double W1, double W2, double vadt, bool up, double depend,
+                                        double dxE, double *Qn) {
+  const bool mm = use_minmod_r<R>(Q[4], Q[0]);
+  const bool va_any = __any(!mm);
+  const R sdep = up ? (R)depend : -(R)depend;
+  const Quot over(dxE);
+#pragma unroll
+  for (int b = 0; b < 15; b += 5) {
+    double q2[5];
+    R dp[5], dm[5], qd[5], gr[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      q2[v] = sh_dn(Q[b + v]);
+      dp[v] = (R)(q2[v] - Q[b + v]);
+      dm[v] = sh_up(dp[v]);
+      qd[v] = (R)0.0;
+    }
+    if (va_any) {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) qd[v] = (R)(q2[v] - sh_up(Q[b + v]));
+    }
+    vslopes<R, 5>([&](int v) { return dp[v]; }, [&](int v) { return dm[v]; }, [&](int v) { return qd[v]; }, (R)W0, (R)W1,
+                  (R)W2, mm, gr);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+      const R gn = sh_dn(gr[v]);
+      const double face = (up ? Q[b + v] : q2[v]) + (double)(sdep * (up ? gr[v] : gn));
+      const double F = -(vadt * face);
+      const double Fl = sh_up(F);
+      const double num = Q[b + v] * W1 + F - Fl;
+      if constexpr (Ar<R>::strict) Qn[b + v] = over(num);
+      else Qn[b + v] = num * over.y;
+    }
+  }
+}
 
 template <class R>
 __global__ __launch_bounds__(256) void k_rhsmoc_x(SweepIO A, Geo g, XSide S, double dt) {
@@ -1782,13 +1756,14 @@ __global__ __launch_bounds__(256) void k_rhsmoc_x(SweepIO A, Geo g, XSide S, dou
       double gg = 3.0 * s4 + 5.0 * spc[2];
       double gi = (2.0 * s4 + 2.0 * spc[2]) / gg;
       double e = pp / (rho * gi) + 0.5 * (vx * vx + vy * vy + vz * vz) + 0.5 * (bx_ * bx_ + by_ * by_ + bz_ * bz_) / rho;
-      rhoL = dm / dxl;
+      const Quot odl(dxl);
+      rhoL = odl(dm);
       vnL = vn - dt / dm * (pa - pam);
       eL = e - dt / dm * (pa * va - pam * vam);
-      bl1 = b1 * dxq / dxl;
-      bl2 = b2 * dxq / dxl;
+      bl1 = odl(b1 * dxq);
+      bl2 = odl(b2 * dxq);
 #pragma unroll
-      for (int f = 0; f < 8; ++f) spL[f] = dxq * spc[f] / dxl;
+      for (int f = 0; f < 8; ++f) spL[f] = odl(dxq * spc[f]);
     } else {
       double s4 = spc[0] + spc[1] + spc[3] + spc[4];
       double irho = 1.0 / rho;
@@ -1831,12 +1806,12 @@ __global__ __launch_bounds__(256) void k_rhsmoc_x(SweepIO A, Geo g, XSide S, dou
   for (int v = 0; v < 6; ++v) { vm[v] = sh_up(v0[v]); vp[v] = sh_dn(v0[v]); }
   const R dxm_r = (R)vm[5], dx0_r = (R)dxl, dxp_r = (R)vp[5];
   R G[5], H[5];
+  cell_slopes<R, 5>(vm, v0, vp, dxm_r, dx0_r, dxp_r, mm, G);
 #pragma unroll
-  for (int v = 0; v < 5; ++v) { G[v] = vslope<R>(vm[v], v0[v], vp[v], dxm_r, dx0_r, dxp_r, mm); H[v] = G[v]; }
+  for (int v = 0; v < 5; ++v) H[v] = G[v];
   const int nblk = A.nblk;
   if ((p % nblk == 0 || (p - 1) % nblk == 0) && mmp != mm) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) H[v] = vslope<R>(vm[v], v0[v], vp[v], dxm_r, dx0_r, dxp_r, mmp);
+    cell_slopes<R, 5>(vm, v0, vp, dxm_r, dx0_r, dxp_r, mmp, H);
   }
   // characteristic interface J = p between p and p+1 (local positions 0..n)
   R G1[5], H1[5];
@@ -1951,13 +1926,14 @@ __global__ __launch_bounds__(256, Ar<R>::strict ? 3 : 4) void k_sweep_x(SweepIO 
       double gg = 3.0 * s4 + 5.0 * spc[2];
       double gi = (2.0 * s4 + 2.0 * spc[2]) / gg;
       double e = pp / (rho * gi) + 0.5 * (vx * vx + vy * vy + vz * vz) + 0.5 * (bx_ * bx_ + by_ * by_ + bz_ * bz_) / rho;
-      rhoL = dm / dxl;
+      const Quot odl(dxl);
+      rhoL = odl(dm);
       vnL = vn - dt / dm * (pa - pam);
       eL = e - dt / dm * (pa * va - pam * vam);
-      bl1 = b1 * dxq / dxl;
-      bl2 = b2 * dxq / dxl;
+      bl1 = odl(b1 * dxq);
+      bl2 = odl(b2 * dxq);
 #pragma unroll
-      for (int f = 0; f < 8; ++f) spL[f] = dxq * spc[f] / dxl;
+      for (int f = 0; f < 8; ++f) spL[f] = odl(dxq * spc[f]);
     } else {
       double s4 = spc[0] + spc[1] + spc[3] + spc[4];
       double irho = 1.0 / rho;
@@ -1991,12 +1967,12 @@ __global__ __launch_bounds__(256, Ar<R>::strict ? 3 : 4) void k_sweep_x(SweepIO 
   for (int v = 0; v < 6; ++v) { vm[v] = sh_up(v0[v]); vp[v] = sh_dn(v0[v]); }
   const R dxm_r = (R)vm[5], dx0_r = (R)dxl, dxp_r = (R)vp[5];
   R G[5], H[5];
+  cell_slopes<R, 5>(vm, v0, vp, dxm_r, dx0_r, dxp_r, mm, G);
 #pragma unroll
-  for (int v = 0; v < 5; ++v) { G[v] = vslope<R>(vm[v], v0[v], vp[v], dxm_r, dx0_r, dxp_r, mm); H[v] = G[v]; }
+  for (int v = 0; v < 5; ++v) H[v] = G[v];
   const int nblk = A.nblk;
   if ((p % nblk == 0 || (p - 1) % nblk == 0) && mmp != mm) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) H[v] = vslope<R>(vm[v], v0[v], vp[v], dxm_r, dx0_r, dxp_r, mmp);
+    cell_slopes<R, 5>(vm, v0, vp, dxm_r, dx0_r, dxp_r, mmp, H);
   }
   // characteristic interface J = p between p and p+1 (local positions 0..n)
   R G1[5], H1[5];
@@ -2067,31 +2043,14 @@ __global__ __launch_bounds__(256, Ar<R>::strict ? 3 : 4) void k_sweep_x(SweepIO 
   // REMAP of cell p (M3:1600-1686): upwind flux through face p|p+1 from
   // cells p-1..p+2, the flux of face p-1|p from the lane below
   const double W1 = dxl;
-  const double W0 = sh_up(W1), W2 = sh_dn(W1), W3 = sh_dn(W2);
+  const double W0 = sh_up(W1), W2 = sh_dn(W1);
   const double vadt = va * dt;
   const bool up = !(vadt <= 0.0);
-  const double u4n = sh_dn(Q[4]), u0n = sh_dn(Q[0]);
-  const double u4 = up ? Q[4] : u4n, u0 = up ? Q[0] : u0n;
   const double depend = up ? 0.5 * (W1 - vadt) * A.facdep : 0.5 * (W2 + vadt) * A.facdep;
-  const R rdxm = (R)(up ? W0 : W1), rdx0 = (R)(up ? W1 : W2), rdxp = (R)(up ? W2 : W3);
-  const bool rmm = use_minmod_r<R>(u4, u0);
-  const R rdep = (R)depend;
   const bool own = lane >= 6 && lane < 6 + XSCELLS && p <= n;
   const double dxE = own ? xe[p + 1] - xe[p] : 1.0;
   double Qn[15];
-#pragma unroll
-  for (int v = 0; v < 15; ++v) {
-    const double q0 = sh_up(Q[v]), q1 = Q[v], q2 = sh_dn(Q[v]), q3 = sh_dn(q2);
-    const R gr = vslope<R>(up ? q0 : q1, up ? q1 : q2, up ? q2 : q3, rdxm, rdx0, rdxp, rmm);
-    const double qu = up ? q1 : q2;
-    double face;
-    if constexpr (Ar<R>::strict) face = up ? qu + depend * gr : qu - depend * gr;
-    else face = up ? qu + (double)(rdep * gr) : qu - (double)(rdep * gr);
-    const double F = -(vadt * face);
-    const double Fl = sh_up(F);
-    if constexpr (Ar<R>::strict) Qn[v] = (q1 * W1 + F - Fl) / dxE;
-    else Qn[v] = (q1 * W1 + F - Fl) * (1.0 / dxE);
-  }
+  x_remap<R>(Q, W0, W1, W2, vadt, up, depend, dxE, Qn);
   if (!own) return;
   // primitives (M3:1291-1321)
   double rr = dmax(1.27 * A.rmin, Qn[0]);
@@ -2134,33 +2093,15 @@ __global__ __launch_bounds__(256) void k_remap_x(SweepIO A, Geo g, double dt) {
 #pragma unroll
   for (int v = 0; v < 15; ++v) Q[v] = remap_field(A, v)[c];
   const double W1 = A.dxlagM[c];
-  const double W0 = sh_up(W1), W2 = sh_dn(W1), W3 = sh_dn(W2);
+  const double W0 = sh_up(W1), W2 = sh_dn(W1);
   // upwind linear flux through face p|p+1 (M3:1600-1640)
   const double vadt = A.va[ix3s(g, min(max(p, 0), n), j, k)] * dt;
   const bool up = !(vadt <= 0.0);
-  const double u4n = sh_dn(Q[4]), u0n = sh_dn(Q[0]);
-  const double u4 = up ? Q[4] : u4n, u0 = up ? Q[0] : u0n;
   const double depend = up ? 0.5 * (W1 - vadt) * A.facdep : 0.5 * (W2 + vadt) * A.facdep;
-  const R dxm = (R)(up ? W0 : W1), dx0 = (R)(up ? W1 : W2), dxp = (R)(up ? W2 : W3);
-  const bool mm = use_minmod_r<R>(u4, u0);
-  const R rdep = (R)depend;
   const bool own = lane >= 2 && lane < 2 + XRCELLS && p <= n;
   const double dxE = own ? A.xe[p + 1] - A.xe[p] : 1.0;
   double Qn[15];
-#pragma unroll
-  for (int v = 0; v < 15; ++v) {
-    const double q0 = sh_up(Q[v]), q1 = Q[v], q2 = sh_dn(Q[v]), q3 = sh_dn(q2);
-    const R gr = vslope<R>(up ? q0 : q1, up ? q1 : q2, up ? q2 : q3, dxm, dx0, dxp, mm);
-    const double qu = up ? q1 : q2;
-    double face;
-    if constexpr (Ar<R>::strict) face = up ? qu + depend * gr : qu - depend * gr;
-    else face = up ? qu + (double)(rdep * gr) : qu - (double)(rdep * gr);
-    const double F = -(vadt * face);
-    const double Fl = sh_up(F);
-    // remapped conserved state (M3:1645-1686)
-    if constexpr (Ar<R>::strict) Qn[v] = (q1 * W1 + F - Fl) / dxE;
-    else Qn[v] = (q1 * W1 + F - Fl) * (1.0 / dxE);
-  }
+  x_remap<R>(Q, W0, W1, W2, vadt, up, depend, dxE, Qn);
   if (!own) return;
   // primitives (M3:1291-1321)
   const double bn = A.bcc[0][c];

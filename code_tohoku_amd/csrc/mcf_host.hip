@@ -731,6 +731,24 @@ static int do_cc4(mcf_ctx *x) {
   return fillOT(x, 7, 2, OT_BCC);
 }
 
+// Planes per workgroup of k_ct_march over np planes of nb workgroups each.
+// Two workgroups share a CU (204 / 256 registers); a workgroup of z planes
+// costs z + 1 (its first z slopes), and the launch's uneven end about half a
+// round: (workgroups / (2 CUs) + 1/2) (z + 1), within 5% of the times over z
+// = 1..32 at 64^3 to 256^3.  It takes 20 planes at 256^3 (634 us mixed, 1282
+// FP64; 16 planes 653 / 1343, 64 planes 743 / 1520), 6 at 128^3 (102; 16
+// planes 132), 3 at 64^3 (20; 16 planes 52), 1 at 64 x 8 x 8 (11; 51).
+static int ct_zseg(const mcf_ctx *x, int np, long nb) {
+  int best = 1;
+  double cost = 0.0;
+  for (int ns = 1; ns <= np; ++ns) {
+    const int z = (np + ns - 1) / ns;
+    const double c = ((double)(nb * ((np + z - 1) / z)) / (2.0 * x->ncu) + 0.5) * (z + 1);
+    if (ns == 1 || c < cost) { cost = c; best = z; }
+  }
+  return best;
+}
+
 // CT (M3:638-649)
 static int do_ct(mcf_ctx *x, double dt) {
   StageScope scope(x, "ct");
@@ -756,15 +774,14 @@ static int do_ct(mcf_ctx *x, double dt) {
   // the three edge orientations in one launch over (1..n+1)^3: reads rho, p,
   // Vfc(3), face B(3), writes EMF(3)
   {
-    // z march over 61-cell rows, CTM_ROWS rows and CTM_ZSEG planes per
-    // block.  A variant with full 64-cell tiles (the tile's outer
-    // neighbours loaded by the edge lanes, the 257th column per cell) was
-    // slower: 1.08 / 2.11 ms against 1.00 / 1.77 (mixed / FP64), its extra
-    // registers cost more than the idle lanes of the fifth tile.
-    dim3 gr((unsigned)((n[0] + 1 + CTM_OUT - 1) / CTM_OUT), (unsigned)((n[1] + 1 + CTM_ROWS - 1) / CTM_ROWS),
-            (unsigned)((n[2] + 1 + CTM_ZSEG - 1) / CTM_ZSEG));
-    if (x->mixed) KLAUNCH_N("k_ct_march_mixed", k_ct_march_mixed, gr, dim3(64 * CTM_ROWS), 8.0 * boxsize(b1) * 11, A, x->g, dt);
-    else KLAUNCH_N("k_ct_march", k_ct_march<double>, gr, dim3(64 * CTM_ROWS), 8.0 * boxsize(b1) * 11, A, x->g, dt);
+    // z march; waves over the rows 1..ny+1 in memory order
+    const long span = (long)n[1] * x->g.st[1] + n[0] + 2; // memory positions 2 .. span hold the edges
+    const long waves = (span - 1 + CTM_OUT - 1) / CTM_OUT;
+    const long nb = (waves + CTM_WAVES - 1) / CTM_WAVES;
+    A.zseg = ct_zseg(x, n[2] + 1, nb);
+    dim3 gr((unsigned)nb, (unsigned)((n[2] + 1 + A.zseg - 1) / A.zseg));
+    if (x->mixed) KLAUNCH_N("k_ct_march", k_ct_march<float>, gr, dim3(64 * CTM_WAVES), 8.0 * boxsize(b1) * 11, A, x->g, dt);
+    else KLAUNCH_N("k_ct_march", k_ct_march<double>, gr, dim3(64 * CTM_WAVES), 8.0 * boxsize(b1) * 11, A, x->g, dt);
   }
   KLAUNCH512(k_cc3, boxsize(b1), 9, A, x->g, b1, dt);
   return do_cc4(x);

@@ -130,6 +130,7 @@ struct CtArgs {
   double *emf[3];
   const double *gdx[3]; // dx arrays, dx(i) at [i+1]
   double facdep;
+  int zseg; // planes per block of k_ct_march
 };
 
 struct SrcArgs {
@@ -195,11 +196,8 @@ __global__ void k_fill_yz(FillList L, Geo g, int nol);
 __global__ void k_fill_xrule(XFill X, Geo g, int nol);
 __global__ void k_cc1(CtArgs A, Geo g, Box b);
 template <class R> __global__ void k_ct_march(CtArgs A, Geo g, double dt);
-__global__ void k_ct_march_mixed(CtArgs A, Geo g, double dt); // the FP32 march at three waves per SIMD
-// k_ct_march: EMF cells per wave along x, rows (waves) per block, planes
-// per block (16, 32 and 64 planes measured 1.01 / 1.04 / 1.11 ms, mixed,
-// 256^3; 2 and 8 rows no faster than 4)
-constexpr int CTM_OUT = 61, CTM_ROWS = 4, CTM_ZSEG = 16;
+// k_ct_march: EMF cells per wave, waves per block
+constexpr int CTM_OUT = 61, CTM_WAVES = 4;
 __global__ void k_cc3(CtArgs A, Geo g, Box b, double dt);
 __global__ void k_cc4(CtArgs A, Geo g, Box b);
 // CHEM: the chemistry-network Fcool (R = double only) instead of the KI one

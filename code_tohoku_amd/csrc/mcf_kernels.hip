@@ -211,14 +211,15 @@ template <class R> __device__ __forceinline__ double cct_core(const EdgeIn<R> &E
     R a2p = vy + by * dsqinv;
     R da2p = (E.dq1[u2] + E.dq3[u2] * dsqinv) * facm;
     R t;
+    const QuotR<R> o1((R)1.0 - da1p * da2m * dt * dt), o2((R)1.0 - da1m * da2p * dt * dt);
     t = a1p + da1p * dyv * S1 - da1p * (a2m + da2m * dxv * S2) * dt;
-    C1p[cs] = Q::div(t, (R)1.0 - da1p * da2m * dt * dt);
+    C1p[cs] = o1(t);
     t = a2m + da2m * dxv * S2 - da2m * (a1p + da1p * dyv * S1) * dt;
-    C2m[cs] = Q::div(t, (R)1.0 - da1p * da2m * dt * dt);
+    C2m[cs] = o1(t);
     t = a1m + da1m * dyv * S1 - da1m * (a2p + da2p * dxv * S2) * dt;
-    C1m[cs] = Q::div(t, (R)1.0 - da1m * da2p * dt * dt);
+    C1m[cs] = o2(t);
     t = a2p + da2p * dxv * S2 - da2p * (a1m + da1m * dyv * S1) * dt;
-    C2p[cs] = Q::div(t, (R)1.0 - da1m * da2p * dt * dt);
+    C2p[cs] = o2(t);
   }
   const R z = (R)0.0;
   int f0[4], f1[4];
@@ -261,128 +262,126 @@ template <class R> __device__ __forceinline__ double cct_core(const EdgeIn<R> &E
 }
 
 // CCT for the whole box (1..n+1)^3 as a march along z, every transverse
-// slope formed once per cell.  A wave holds 64 consecutive cells of one
-// (j, k) row, lane l at x = ib - 2 + l, and writes the EMFs of lanes 2..62
-// (61 cells: the x slopes at i and i-1 need the values at i-2..i+1).  Per
-// plane k each lane forms, with its own cell's limiter switch:
+// slope formed once per cell.  Lanes follow the memory order of the plane's
+// rows j = 1..ny+1, ghosts included: a wave holds 64 consecutive cells of
+// that order and writes the EMFs of lanes 2..62 (the x slopes at i and i-1
+// need the values at i-2..i+1, which are the neighbouring lanes: a row has
+// two ghost cells at each end, so no written cell's stencil crosses into
+// another row).  61-cell tiles of single rows left the last tile of each row
+// nearly empty (22% more waves at 256^3, 79% at 64^3).  Per plane k each lane
+// forms, with its own cell's limiter switch:
 //   along x: V_y, B_y, V_z, B_z from its neighbours' values (lane shuffles);
 //            the slopes at i-1 then come from the left lane;
 //   along y: V_x, B_x, V_z, B_z at rows j and j-1 (rows j-2..j+1 loaded;
-//            the slope at j-1 is also formed by the wave of row j-1);
+//            the slope at j-1 is also formed by the lane of row j-1);
 //   along z: V_x, B_x, V_y, B_y at plane k (planes k-1, k+1 in registers),
 //            the slopes at k-1 kept from the previous plane.
-// The three edges of the cell then go through cct_core.  Against a kernel
-// with one thread per cell that formed all 24 slopes its three edges use
-// (each slope twice), the march took 1.00 / 1.77 ms instead of 1.12 / 1.93
-// (mixed / FP64, 256^3) with bit-identical EMFs; sharing the row-(j-1)
-// slopes through LDS instead of forming them in each wave needs a barrier
-// per plane and took 1.29 / 1.94.
-template <class R> __device__ __forceinline__ void ct_march(const CtArgs &A, const Geo &g, double dt_d) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+// The spacing along y and z is one number (INITIA, M3:255-298); along x it
+// may differ between the two halves of the box.  The three edges of the cell
+// then go through cct_core.
+//
+// Bound by instruction issue.  256^3, mixed / FP64: 1.00 / 1.78 ms with row
+// tiles and both slope candidates' operands selected per slope, 0.63 / 1.28
+// now, the same EMFs.  FP32 takes 204 registers, two waves per SIMD: capped
+// at 168 for three it spills 108 bytes a lane and takes 0.87; FP64 at two
+// waves spills 68 bytes a lane (its 272 registers would leave one).
+template <class R>
+__global__ __launch_bounds__(64 * CTM_WAVES, 2) void k_ct_march(CtArgs A, Geo g, double dt_d) {
   const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
-  const int j = 1 + CTM_ROWS * (int)blockIdx.y + w;
-  if (j > ny + 1) return; // whole waves; no barrier in this kernel
-  const int ib = 1 + CTM_OUT * (int)blockIdx.x;
-  const int i = ib - 2 + lane;
-  const int ic = min(i, nx + 2); // lanes past the last ghost read the last ghost
-  const bool outx = lane >= 2 && lane <= 62 && i <= nx + 1;
-  const int k0 = 1 + CTM_ZSEG * (int)blockIdx.z;
-  const int k1 = min(nz + 1, k0 + CTM_ZSEG - 1);
   const int sy = g.st[1], sz = g.st[2];
+  const int lane = threadIdx.x & 63;
+  const long wave = (long)CTM_WAVES * blockIdx.x + (threadIdx.x >> 6);
+  const long last = (long)(ny + 1) * sy - 1; // the last ghost of row ny+1
+  if (CTM_OUT * wave + 2 > last) return;     // whole waves; no barrier in this kernel
+  const int f = (int)min(CTM_OUT * wave + lane, last);
+  const int j = 1 + f / sy, i = f % sy - 1;
+  const bool out = lane >= 2 && lane <= 62 && CTM_OUT * wave + lane <= last && i >= 1 && i <= nx + 1;
+  const int k0 = 1 + A.zseg * (int)blockIdx.y;
+  const int k1 = min(nz + 1, k0 + A.zseg - 1);
   const double *Vx = A.vfc[0], *Vy = A.vfc[1], *Vz = A.vfc[2];
   const double *Bx = A.U[5], *By = A.U[6], *Bz = A.U[7], *rh = A.U[0], *pp = A.U[4];
   // widths: x at the lane's cell (indices clamped to the dx array for the
-  // halo lanes, whose slopes are not used), y at row j
-  const double *gx = A.gdx[0], *gy = A.gdx[1], *gz = A.gdx[2];
-  const int ix0 = max(0, min(ic, nx + 3)), ix1 = min(ic + 1, nx + 3), ix2 = min(ic + 2, nx + 3);
+  // halo lanes, whose slopes are not used)
+  const double *gx = A.gdx[0];
+  const int ix0 = max(0, i), ix1 = min(i + 1, nx + 3), ix2 = min(i + 2, nx + 3);
   const R xw0 = (R)gx[ix0], xw1 = (R)gx[ix1], xw2 = (R)gx[ix2];
-  const R yw_m = (R)gy[j - 1], yw0 = (R)gy[j], yw1 = (R)gy[j + 1], yw2 = (R)gy[j + 2];
+  const R yw = (R)A.gdx[1][1], zw = (R)A.gdx[2][1];
   // z window of the own column: V_x, B_x, V_y, B_y at planes k-1 and k,
   // their z slopes at k-1, and rho at k-1 in rows j and j-1
-  int c = ix3(g, ic, j, k0 - 1);
-  double wVx0 = Vx[c], wBx0 = Bx[c], wVy0 = Vy[c], wBy0 = By[c];
-  double wVx1 = Vx[c + sz], wBx1 = Bx[c + sz], wVy1 = Vy[c + sz], wBy1 = By[c + sz];
+  int c = 2 * sy + f + k0 * sz; // (i, j, k0-1)
+  double w0[4] = {Vx[c], Bx[c], Vy[c], By[c]};
+  double w1[4] = {Vx[c + sz], Bx[c + sz], Vy[c + sz], By[c + sz]};
   double rho_km = rh[c], rhoJ_km = rh[c - sy];
-  R zVx0, zBx0, zVy0, zBy0;
+  R z0[4];
   {
-    const bool mm = use_minmod_r<R>(pp[c], rh[c]);
-    const R z0 = (R)gz[k0 - 1], z1 = (R)gz[k0], z2 = (R)gz[k0 + 1];
     const int cm = c - sz;
-    zVx0 = vslope<R>(Vx[cm], wVx0, wVx1, z0, z1, z2, mm);
-    zBx0 = vslope<R>(Bx[cm], wBx0, wBx1, z0, z1, z2, mm);
-    zVy0 = vslope<R>(Vy[cm], wVy0, wVy1, z0, z1, z2, mm);
-    zBy0 = vslope<R>(By[cm], wBy0, wBy1, z0, z1, z2, mm);
+    const double wm[4] = {Vx[cm], Bx[cm], Vy[cm], By[cm]};
+    cell_slopes<R, 4>(wm, w0, w1, zw, zw, zw, use_minmod_r<R>(pp[c], rh[c]), z0);
   }
   for (int k = k0; k <= k1; ++k) {
-    c += sz; // (ic, j, k)
+    c += sz; // (i, j, k)
     // loads: own column at k+1 (z window) and k; rows j-1, j-2, j+1 at k
-    const double nVx = Vx[c + sz], nBx = Bx[c + sz], nVy = Vy[c + sz], nBy = By[c + sz];
+    const double wn[4] = {Vx[c + sz], Bx[c + sz], Vy[c + sz], By[c + sz]};
     const double vz = Vz[c], bz = Bz[c], rho = rh[c], p = pp[c];
     const int cJ = c - sy, cJJ = c - 2 * sy, cP = c + sy;
-    const double VxJ = Vx[cJ], BxJ = Bx[cJ], VzJ = Vz[cJ], BzJ = Bz[cJ], rhoJ = rh[cJ], pJ = pp[cJ];
-    const double VxJJ = Vx[cJJ], BxJJ = Bx[cJJ], VzJJ = Vz[cJJ], BzJJ = Bz[cJJ];
-    const double VxP = Vx[cP], BxP = Bx[cP], VzP = Vz[cP], BzP = Bz[cP];
+    const double rhoJ = rh[cJ], pJ = pp[cJ];
+    const double qJJ[4] = {Vx[cJJ], Bx[cJJ], Vz[cJJ], Bz[cJJ]};
+    const double qJ[4] = {Vx[cJ], Bx[cJ], Vz[cJ], Bz[cJ]};
+    const double qP[4] = {Vx[cP], Bx[cP], Vz[cP], Bz[cP]};
+    const double q0[4] = {w1[0], w1[1], vz, bz};
     const bool mm0 = use_minmod_r<R>(p, rho);
     const bool mmJ = use_minmod_r<R>(pJ, rhoJ);
-    const R zw0 = (R)gz[k], zw1 = (R)gz[k + 1], zw2 = (R)gz[k + 2];
-    // along z at k
-    const R zVx1 = vslope<R>(wVx0, wVx1, nVx, zw0, zw1, zw2, mm0);
-    const R zBx1 = vslope<R>(wBx0, wBx1, nBx, zw0, zw1, zw2, mm0);
-    const R zVy1 = vslope<R>(wVy0, wVy1, nVy, zw0, zw1, zw2, mm0);
-    const R zBy1 = vslope<R>(wBy0, wBy1, nBy, zw0, zw1, zw2, mm0);
-    // along y at j and j-1
-    const R yVx1 = vslope<R>(VxJ, wVx1, VxP, yw0, yw1, yw2, mm0);
-    const R yBx1 = vslope<R>(BxJ, wBx1, BxP, yw0, yw1, yw2, mm0);
-    const R yVz1 = vslope<R>(VzJ, vz, VzP, yw0, yw1, yw2, mm0);
-    const R yBz1 = vslope<R>(BzJ, bz, BzP, yw0, yw1, yw2, mm0);
-    const R yVx0 = vslope<R>(VxJJ, VxJ, wVx1, yw_m, yw0, yw1, mmJ);
-    const R yBx0 = vslope<R>(BxJJ, BxJ, wBx1, yw_m, yw0, yw1, mmJ);
-    const R yVz0 = vslope<R>(VzJJ, VzJ, vz, yw_m, yw0, yw1, mmJ);
-    const R yBz0 = vslope<R>(BzJJ, BzJ, bz, yw_m, yw0, yw1, mmJ);
-    // along x at i (neighbour values from the adjacent lanes), then at i-1
-    const double VyL = __shfl_up(wVy1, 1, 64), VyR = __shfl_down(wVy1, 1, 64);
-    const double ByL = __shfl_up(wBy1, 1, 64), ByR = __shfl_down(wBy1, 1, 64);
-    const double VzL = __shfl_up(vz, 1, 64), VzR = __shfl_down(vz, 1, 64);
-    const double BzL = __shfl_up(bz, 1, 64), BzR = __shfl_down(bz, 1, 64);
-    const R xVy1 = vslope<R>(VyL, wVy1, VyR, xw0, xw1, xw2, mm0);
-    const R xBy1 = vslope<R>(ByL, wBy1, ByR, xw0, xw1, xw2, mm0);
-    const R xVz1 = vslope<R>(VzL, vz, VzR, xw0, xw1, xw2, mm0);
-    const R xBz1 = vslope<R>(BzL, bz, BzR, xw0, xw1, xw2, mm0);
-    const R xVy0 = __shfl_up(xVy1, 1, 64), xBy0 = __shfl_up(xBy1, 1, 64);
-    const R xVz0 = __shfl_up(xVz1, 1, 64), xBz0 = __shfl_up(xBz1, 1, 64);
+    // along x at i (neighbour values from the adjacent lanes)
+    const double qx[4] = {w1[2], w1[3], vz, bz}; // V_y, B_y, V_z, B_z
+    double qL[4], qR[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) { qL[v] = __shfl_up(qx[v], 1, 64); qR[v] = __shfl_down(qx[v], 1, 64); }
+    R z1[4], y1[4], x1[4], y0[4], x0[4];
+    if (mm0) { // the three directions of the own cell in one branch
+      cell_slopes<R, 4>(w0, w1, wn, zw, zw, zw, true, z1);
+      cell_slopes<R, 4>(qJ, q0, qP, yw, yw, yw, true, y1);
+      cell_slopes<R, 4>(qL, qx, qR, xw0, xw1, xw2, true, x1);
+    } else {
+      cell_slopes<R, 4>(w0, w1, wn, zw, zw, zw, false, z1);
+      cell_slopes<R, 4>(qJ, q0, qP, yw, yw, yw, false, y1);
+      cell_slopes<R, 4>(qL, qx, qR, xw0, xw1, xw2, false, x1);
+    }
+    cell_slopes<R, 4>(qJJ, qJ, q0, yw, yw, yw, mmJ, y0); // along y at j-1
+#pragma unroll
+    for (int v = 0; v < 4; ++v) x0[v] = __shfl_up(x1[v], 1, 64); // along x at i-1
     const double rhoL = __shfl_up(rho, 1, 64), rhoJL = __shfl_up(rhoJ, 1, 64), rhoKL = __shfl_up(rho_km, 1, 64);
-    if (outx) {
+    if (out) {
       double e0 = 0.0, e1 = 0.0, e2 = 0.0;
       if (k <= nz) { // edge along z: (d1, d2) = (x, y)
         EdgeIn<R> E;
-        E.v1[0] = (R)VxJ; E.b1[0] = (R)BxJ; E.v1[1] = (R)wVx1; E.b1[1] = (R)wBx1;
-        E.v2[0] = (R)VyL; E.b2[0] = (R)ByL; E.v2[1] = (R)wVy1; E.b2[1] = (R)wBy1;
-        E.dq0[0] = yVx0; E.dq2[0] = yBx0; E.dq0[1] = yVx1; E.dq2[1] = yBx1;
-        E.dq1[0] = xVy0; E.dq3[0] = xBy0; E.dq1[1] = xVy1; E.dq3[1] = xBy1;
-        E.dy[0] = yw0; E.dy[1] = yw1;
+        E.v1[0] = (R)qJ[0]; E.b1[0] = (R)qJ[1]; E.v1[1] = (R)w1[0]; E.b1[1] = (R)w1[1];
+        E.v2[0] = (R)qL[0]; E.b2[0] = (R)qL[1]; E.v2[1] = (R)w1[2]; E.b2[1] = (R)w1[3];
+        E.dq0[0] = y0[0]; E.dq2[0] = y0[1]; E.dq0[1] = y1[0]; E.dq2[1] = y1[1];
+        E.dq1[0] = x0[0]; E.dq3[0] = x0[1]; E.dq1[1] = x1[0]; E.dq3[1] = x1[1];
+        E.dy[0] = yw; E.dy[1] = yw;
         E.dx[0] = xw0; E.dx[1] = xw1;
         E.dnc = 0.25 * (rho + rhoL + rhoJ + rhoJL);
         e0 = cct_core<R>(E, A.facdep, dt_d);
       }
       if (i <= nx) { // edge along x: (d1, d2) = (y, z)
         EdgeIn<R> E;
-        E.v1[0] = (R)wVy0; E.b1[0] = (R)wBy0; E.v1[1] = (R)wVy1; E.b1[1] = (R)wBy1;
-        E.v2[0] = (R)VzJ; E.b2[0] = (R)BzJ; E.v2[1] = (R)vz; E.b2[1] = (R)bz;
-        E.dq0[0] = zVy0; E.dq2[0] = zBy0; E.dq0[1] = zVy1; E.dq2[1] = zBy1;
-        E.dq1[0] = yVz0; E.dq3[0] = yBz0; E.dq1[1] = yVz1; E.dq3[1] = yBz1;
-        E.dy[0] = zw0; E.dy[1] = zw1;
-        E.dx[0] = yw0; E.dx[1] = yw1;
+        E.v1[0] = (R)w0[2]; E.b1[0] = (R)w0[3]; E.v1[1] = (R)w1[2]; E.b1[1] = (R)w1[3];
+        E.v2[0] = (R)qJ[2]; E.b2[0] = (R)qJ[3]; E.v2[1] = (R)vz; E.b2[1] = (R)bz;
+        E.dq0[0] = z0[2]; E.dq2[0] = z0[3]; E.dq0[1] = z1[2]; E.dq2[1] = z1[3];
+        E.dq1[0] = y0[2]; E.dq3[0] = y0[3]; E.dq1[1] = y1[2]; E.dq3[1] = y1[3];
+        E.dy[0] = zw; E.dy[1] = zw;
+        E.dx[0] = yw; E.dx[1] = yw;
         E.dnc = 0.25 * (rho + rhoJ + rho_km + rhoJ_km);
         e1 = cct_core<R>(E, A.facdep, dt_d);
       }
       if (j <= ny) { // edge along y: (d1, d2) = (z, x)
         EdgeIn<R> E;
-        E.v1[0] = (R)VzL; E.b1[0] = (R)BzL; E.v1[1] = (R)vz; E.b1[1] = (R)bz;
-        E.v2[0] = (R)wVx0; E.b2[0] = (R)wBx0; E.v2[1] = (R)wVx1; E.b2[1] = (R)wBx1;
-        E.dq0[0] = xVz0; E.dq2[0] = xBz0; E.dq0[1] = xVz1; E.dq2[1] = xBz1;
-        E.dq1[0] = zVx0; E.dq3[0] = zBx0; E.dq1[1] = zVx1; E.dq3[1] = zBx1;
+        E.v1[0] = (R)qL[2]; E.b1[0] = (R)qL[3]; E.v1[1] = (R)vz; E.b1[1] = (R)bz;
+        E.v2[0] = (R)w0[0]; E.b2[0] = (R)w0[1]; E.v2[1] = (R)w1[0]; E.b2[1] = (R)w1[1];
+        E.dq0[0] = x0[2]; E.dq2[0] = x0[3]; E.dq0[1] = x1[2]; E.dq2[1] = x1[3];
+        E.dq1[0] = z0[0]; E.dq3[0] = z0[1]; E.dq1[1] = z1[0]; E.dq3[1] = z1[1];
         E.dy[0] = xw0; E.dy[1] = xw1;
-        E.dx[0] = zw0; E.dx[1] = zw1;
+        E.dx[0] = zw; E.dx[1] = zw;
         E.dnc = 0.25 * (rho + rhoL + rho_km + rhoKL);
         e2 = cct_core<R>(E, A.facdep, dt_d);
       }
@@ -391,23 +390,13 @@ template <class R> __device__ __forceinline__ void ct_march(const CtArgs &A, con
       if (j <= ny) A.emf[1][c] = e2;
     }
     // advance the z window
-    wVx0 = wVx1; wBx0 = wBx1; wVy0 = wVy1; wBy0 = wBy1;
-    wVx1 = nVx; wBx1 = nBx; wVy1 = nVy; wBy1 = nBy;
-    zVx0 = zVx1; zBx0 = zBx1; zVy0 = zVy1; zBy0 = zBy1;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) { w0[v] = w1[v]; w1[v] = wn[v]; z0[v] = z1[v]; }
     rho_km = rho; rhoJ_km = rhoJ;
   }
 }
-template <class R>
-__global__ __launch_bounds__(64 * CTM_ROWS) void k_ct_march(CtArgs A, Geo g, double dt_d) {
-  ct_march<R>(A, g, dt_d);
-}
 template __global__ void k_ct_march<double>(CtArgs, Geo, double);
-// The FP32 (mixed) march capped at 168 registers, three waves per SIMD
-// instead of two (36 bytes of scratch spill): 0.99-1.02 against 1.03 ms at
-// 256^3, the same EMFs.  The FP64 march would spill 348 bytes at that cap.
-__global__ __launch_bounds__(64 * CTM_ROWS, 3) void k_ct_march_mixed(CtArgs A, Geo g, double dt_d) {
-  ct_march<float>(A, g, dt_d);
-}
+template __global__ void k_ct_march<float>(CtArgs, Geo, double);
 
 // CC(3): face-B induction (M3:2159-2169).  A variant fused with CC(4),
 // out of place over the whole box (each thread also forming the new faces

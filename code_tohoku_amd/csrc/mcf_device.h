@@ -98,7 +98,8 @@ __device__ __forceinline__ void chareq(double vyp, double Byp, double rl, double
 // Koyama-Inutsuka net cooling (1DMHDKIcool/1DMHDwCC3KIcool.f90:1165-1171)
 // with N = rho/1.27 (3DMHD-feedback/MCF3DSGincfca3-feedback.f90:3586).
 __device__ __forceinline__ double fcool_ki(double rho, double T) {
-  double N = rho / 1.27;
+  const Quot o127(1.27); // the reciprocal is a constant
+  double N = o127(rho);
   double Laml = 1.0e7 * exp(-1.184e5 / (T * 1.0e3 + 1.0e3));
   Laml = dmin(Laml, 5.0e3);
   double Lamc = 1.4e-2 * sqrt(T * 1.0e3) * exp(-9.2e1 / (T * 1.0e3));

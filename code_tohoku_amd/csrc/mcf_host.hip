@@ -831,6 +831,17 @@ static int do_source(mcf_ctx *x, double dt) {
   return MCF_OK;
 }
 
+// Planes per workgroup of k_src_col: as many as leave two workgroups for
+// every CU, at most zmax (each march reads two planes of its neighbours).
+// zmax = 64 mixed, 32 FP64: the best at 256^3 (265 / 424 us; 8 planes 299 /
+// 438).  With zmax everywhere a launch took 108 us at 64^3 and 120 us at
+// 128^3 (mixed); 11 us with 1 plane and 34 us with 8.
+static int src_zseg(const mcf_ctx *x, const Box &b, int zmax) {
+  const long tiles = (long)((b.cnt[0] + 63) / 64) * ((b.cnt[1] + SRC_ROWS - 1) / SRC_ROWS);
+  const long segs = std::max(1L, (2L * x->ncu + tiles - 1) / tiles); // wanted
+  return (int)std::min<long>(zmax, std::max<long>(1, b.cnt[2] / segs));
+}
+
 // The thermal part of SOURCE (M3:2477-2572): two-stage cooling +
 // saturated conduction
 static int do_thermal(mcf_ctx *x, double dt) {
@@ -883,7 +894,8 @@ static int do_thermal(mcf_ctx *x, double dt) {
     {
       // the chemistry Fcool always runs in FP64
       const bool f32 = x->mixed && !x->chem;
-      const int zseg = f32 ? SRC_ZSEG_F32 : SRC_ZSEG_F64;
+      const int zseg = src_zseg(x, b, f32 ? 64 : 32);
+      A.zseg = zseg;
       dim3 gr((unsigned)((b.cnt[0] + 63) / 64), (unsigned)((b.cnt[1] + SRC_ROWS - 1) / SRC_ROWS), (unsigned)((b.cnt[2] + zseg - 1) / zseg));
       if (x->chem) KLAUNCH_N("k_src_col", (k_src_col<double, true>), gr, dim3(64 * SRC_ROWS), 8.0 * (double)boxsize(b) * 19, A, x->g, b, dt, stage);
       else if (f32) KLAUNCH_N("k_src_col", (k_src_col<float, false>), gr, dim3(64 * SRC_ROWS), 8.0 * (double)boxsize(b) * 9, A, x->g, b, dt, stage);

@@ -141,6 +141,7 @@ struct SrcArgs {
   const double *sp[8];
   const double *gdx[3];
   double pmin, pmax;
+  int zseg; // planes per block of k_src_col
   // cooling surrogate (sur != 0): packed MLP operands, FP32 weights and the
   // counters {backward-Euler cells, IMC fallbacks}
   // and the queue of backward-Euler cells with their conduction increments
@@ -202,8 +203,6 @@ __global__ void k_cc3(CtArgs A, Geo g, Box b, double dt);
 __global__ void k_cc4(CtArgs A, Geo g, Box b);
 // CHEM: the chemistry-network Fcool (R = double only) instead of the KI one
 template <class R, bool CHEM = false> __global__ void k_src_col(SrcArgs A, Geo g, Box b, double dt, int stage);
-// planes per block of k_src_col: FP32 rates (mixed) 64, FP64 32
-constexpr int SRC_ZSEG_F32 = 64, SRC_ZSEG_F64 = 32;
 constexpr int SRC_ROWS = 8;  // x rows (waves) per block of k_src_col
 __global__ void k_shell_copy(const double *__restrict__ src, double *__restrict__ dst, Geo g);
 __global__ void k_src_stiff(SrcArgs A, double dt, int stage);

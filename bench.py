@@ -136,9 +136,9 @@ def kernel_stage(name):
         return "sweep_z"
     if name in ("k_cc1", "k_ct_march", "k_cc3", "k_cc4"):
         return "ct"
-    if name in ("k_src_col", "k_shell_copy", "k_src_stiff", "k_src_imc", "k_shield", "k_chem"):
+    if name in ("k_src_col", "k_src_stiff", "k_src_imc", "k_shield", "k_chem"):
         return "source"
-    if name in ("k_dtmin", "k_dtfinal"):
+    if name == "k_dtmin":
         return "dt"
     if name in ("k_dissip_div", "k_dissip_upd"):
         return "dissip"

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -98,7 +99,8 @@ struct mcf_ctx {
   int ncu = 256; // compute units of the device
   double time = 0.0;
   int ifevo = 1;
-  double *hred = nullptr; // pinned 2 doubles
+  double *hred = nullptr; // host memory the device writes: the two dt minima, then the number of the launch
+  unsigned long long dtseq = 0;
   // per-kernel event timing (mcf_profile)
   bool prof = false;
   bool mixed = false; // MCF_PREC_MIXED: FP32 reconstruction / Riemann / EMF
@@ -229,8 +231,8 @@ static void setup_constants(mcf_ctx *x) {
 // launch helpers
 // ----------------------------------------------------------------------------
 static const int TPB = 256;
-// blocks of the dt reduction's first pass (one partial min pair each)
-static const int DT_BLOCKS = 8192;
+// most blocks of the dt reduction (one partial min pair each)
+static const int DT_BLOCKS = 512;
 
 static Box mkbox(int x0, int x1, int y0, int y1, int z0, int z1) {
   Box b;
@@ -326,42 +328,7 @@ static int col_seg(const mcf_ctx *x, int n, long ncol) {
 // ----------------------------------------------------------------------------
 // ghost fills
 // ----------------------------------------------------------------------------
-// The y and z periodic passes of one fill in one launch (k_fill_yz); dm[f]
-// says which of the two passes field f takes (bit 0: y, bit 1: z).
-static int fill_yz(mcf_ctx *x, double *const *a, const int *dm, int nf, int nol) {
-  FillList L{};
-  L.nf = nf;
-  for (int f = 0; f < nf; ++f) { L.a[f] = a[f]; L.dm[f] = dm[f]; }
-  const long m0 = x->g.n[0] + 4, m1 = x->g.n[1] + 4, m2 = x->g.n[2] + 4;
-  const long nt = 2L * nol * m0 * m2 + 2L * nol * m0 * (m1 - 2 * nol);
-  KLAUNCH(k_fill_yz, nt, 2 * nf, L, x->g, nol);
-  return MCF_OK;
-}
-
 static bool x_inflow(const mcf_ctx *x) { return x->cfg.bcx1 == 4 || x->cfg.bcx2 == 4; }
-
-static int launch_xfill(mcf_ctx *x, XFill &X, int nol) {
-  X.rho = x->U[F_RHO];
-  X.bcc1 = x->bcc[0];
-  X.blg1 = x->blg[0];
-  X.blg2 = x->blg[1];
-  if (x->dtfd) {
-    // the boundary ranks' dx(0) and L = dx(0)*Ncellx*NSPLTx (M3:821-822, 857-858)
-    const int cx = x->g.n[0] / x->nsp[0], nsx = x->nsp[0];
-    X.dtf.f = x->dtfd;
-    X.dtf.xe = x->gx[0];
-    X.dtf.t = x->time;
-    for (int s = 0; s < 2; ++s) {
-      const double dx0 = x->hdx[0][(s == 0 ? 0 : (nsx - 1) * cx) + 1];
-      X.dtf.dx0[s] = dx0;
-      X.dtf.L[s] = dx0 * (double)cx * (double)nsx;
-      X.dtf.v[s] = x->bbrv[2][1][s + 1];
-    }
-  }
-  long nt = (long)(x->g.n[1] + 4) * (x->g.n[2] + 4) * 2 * nol;
-  KLAUNCH(k_fill_xrule, nt, 2 * X.nf, X, x->g, nol);
-  return MCF_OK;
-}
 
 enum { OT_DXLAG = 1, OT_BCC, OT_BLG, OT_VFC, OT_SPECIES };
 
@@ -379,33 +346,27 @@ static int ot_fields(mcf_ctx *x, int what, int d, double **a) {
   return nf;
 }
 
-// Fills that run back to back, gathered into one x launch (the x rules or
-// the periodic copy, fields in call order) and one y/z launch.  Equal to the
-// calls in sequence when no x rule reads, at a y or z ghost row, a field an
-// earlier call fills: the rules that read other fields are the species rule
-// (interior rows only) and the mode-2 momentum and energy rules, which are
-// never gathered with another call.
+// Fills that run back to back, gathered into one launch (k_fill).  Equal to
+// the calls in sequence when no x rule reads, at a y or z ghost row, a field
+// an earlier call fills other than rho: the rules that read other fields are
+// the species rule (interior rows only) and the mode-2 momentum and energy
+// rules, which are never gathered with another call.
 struct FillPlan {
   int nol;
-  XFill X{};
-  double *yz[16];
-  int dm[16];
-  int nyz = 0;
-  bool over = false; // more than 16 fields in a pass
+  Fill F{};
+  bool over = false; // more fields than a launch takes
   explicit FillPlan(int n) : nol(n) {}
-  int add_x() {
-    if (X.nf == 16) { over = true; return 15; }
-    return X.nf++;
+  int field(double *p) {
+    for (int q = 0; q < F.nf; ++q)
+      if (F.a[q] == p) return q;
+    if (F.nf == FILL_MAXF) { over = true; return FILL_MAXF - 1; }
+    const int q = F.nf++;
+    F.a[q] = p;
+    F.rule[q][0] = F.rule[q][1] = XR_NONE;
+    return q;
   }
-  void add_yz(double *p, int bits) {
-    int q = 0;
-    while (q < nyz && yz[q] != p) ++q;
-    if (q == nyz) {
-      if (nyz == 16) { over = true; return; }
-      yz[nyz] = p; dm[nyz] = 0; ++nyz;
-    }
-    dm[q] |= bits;
-  }
+  int add_x(double *p) { F.anyx = 1; return field(p); }
+  void add_yz(double *p, int bits) { F.anyyz = 1; F.dm[field(p)] |= bits; }
 };
 
 // BC_MPI(nol, mode) for the 1-based U components in list (M3:800-926)
@@ -415,9 +376,8 @@ static void planU(mcf_ctx *x, FillPlan &P, int dmask, int mode, const int *list,
     const int K = list[t];
     double *a = x->U[K - 1];
     if (dmask & 1) {
-      XFill &X = P.X;
-      const int u = P.add_x();
-      X.a[u] = a;
+      Fill &X = P.F;
+      const int u = P.add_x(a);
       for (int s = 0; s < 2; ++s) {
         int side = s + 1;
         if (bc[s] == 1) { // outflow: zero-gradient copy; face B_x as the inflow rule
@@ -445,10 +405,9 @@ static void planOT(mcf_ctx *x, FillPlan &P, int dmask, int what) {
   double *a[16];
   if (dmask & 1) {
     const int nf = ot_fields(x, what, 0, a);
-    XFill &X = P.X;
+    Fill &X = P.F;
     for (int t = 0; t < nf; ++t) {
-      const int u = P.add_x();
-      X.a[u] = a[t];
+      const int u = P.add_x(a[t]);
       for (int s = 0; s < 2; ++s) {
         int side = s + 1;
         if (bc[s] == 1) { X.rule[u][s] = XR_COPY; X.src[u][s] = s == 0 ? 1 : nx; continue; }
@@ -469,15 +428,38 @@ static void planOT(mcf_ctx *x, FillPlan &P, int dmask, int what) {
   for (int d = 1; d <= 2; ++d) {
     if (!(dmask & (1 << d))) continue;
     const int nf = ot_fields(x, what, d, a);
-    for (int t = 0; t < nf; ++t) P.add_yz(a[t], d);
+    for (int t = 0; t < nf; ++t) P.add_yz(a[t], d); // d = 1: bit 0 (y), d = 2: bit 1 (z)
   }
 }
 
-// the x launch, then the y/z launch
 static int flush(mcf_ctx *x, FillPlan &P) {
-  if (P.over) { g_err = "internal: a fill plan holds more than 16 fields"; return MCF_E_STATE; }
-  if (P.X.nf > 0) CHK(launch_xfill(x, P.X, P.nol));
-  if (P.nyz > 0) CHK(fill_yz(x, P.yz, P.dm, P.nyz, P.nol));
+  if (P.over) { g_err = "internal: a fill plan holds more fields than a launch takes"; return MCF_E_STATE; }
+  Fill &F = P.F;
+  if (F.nf == 0) return MCF_OK;
+  F.rho = x->U[F_RHO];
+  F.bcc1 = x->bcc[0];
+  F.blg1 = x->blg[0];
+  F.blg2 = x->blg[1];
+  F.rho_f = -1;
+  for (int q = 0; q < F.nf; ++q)
+    if (F.a[q] == F.rho && F.rule[q][0] != XR_NONE) F.rho_f = q;
+  if (x->dtfd) {
+    // the boundary ranks' dx(0) and L = dx(0)*Ncellx*NSPLTx (M3:821-822, 857-858)
+    const int cx = x->g.n[0] / x->nsp[0], nsx = x->nsp[0];
+    F.dtf.f = x->dtfd;
+    F.dtf.xe = x->gx[0];
+    F.dtf.t = x->time;
+    for (int s = 0; s < 2; ++s) {
+      const double dx0 = x->hdx[0][(s == 0 ? 0 : (nsx - 1) * cx) + 1];
+      F.dtf.dx0[s] = dx0;
+      F.dtf.L[s] = dx0 * (double)cx * (double)nsx;
+      F.dtf.v[s] = x->bbrv[2][1][s + 1];
+    }
+  }
+  const long m0 = x->g.n[0] + 4, m1 = x->g.n[1] + 4, m2 = x->g.n[2] + 4, l2 = 2L * P.nol;
+  const long w = F.anyx ? m0 - l2 : m0;
+  const long nt = (F.anyx ? l2 * m1 * m2 : 0) + (F.anyyz ? l2 * w * m2 + l2 * w * (m1 - l2) : 0);
+  KLAUNCH_G(k_fill, dim3(nblocks(nt), (unsigned)F.nf), dim3(TPB), 16.0 * (double)nt * F.nf, F, x->g, P.nol);
   return MCF_OK;
 }
 
@@ -878,13 +860,15 @@ static int do_thermal(mcf_ctx *x, double dt) {
     } else {
       // ghosts of the predictor (the fill works on U[F_P])
       x->U[F_P] = Q; x->Ub[F_P] = P;
-      CHK(fillU(x, 7, 1, 1, l5, 1));
+      {
+        FillPlan G(1);
+        planU(x, G, 7, 1, l5, 1);
+        G.F.mirror = P; // P's first ghost layer takes the predictor's
+        CHK(flush(x, G));
+      }
       x->U[F_P] = P; x->Ub[F_P] = Q;
-      // corrector: T from the predictor, result written over P; P's first
-      // ghost layer takes the predictor's
+      // corrector: T from the predictor, result written over P
       A.Tp = Q; A.Pn = P; A.Pout = P;
-      const long a0 = nx + 2, a1 = ny + 2;
-      KLAUNCH(k_shell_copy, 2 * (a0 * a1 + a0 * nz + (long)ny * nz), 2, Q, P, x->g);
     }
     const Box &b = bc;
     // queue counters: cool_cnt[2] and cool_cnt[3] (two u32 each), zero at
@@ -1384,7 +1368,7 @@ extern "C" int mcf_init(const mcf_config *cfg, mcf_ctx **out) {
   for (int c = 0; c < 3; ++c) { x->emf[c] = p; p += nc; }
   x->divv = p; p += ndivv;
   for (int d = 0; d < 3; ++d) { x->gx[d] = p; p += n[d] + 4; x->gdx[d] = p; p += n[d] + 4; }
-  x->red = p; p += 16 + 2 * DT_BLOCKS;
+  x->red = p; p += 16 + 2 * DT_BLOCKS; // block counter, then the partial minima
   if (x->has_cols) {
     for (int q = 0; q < 10; ++q) { x->col[q] = p; p += nc; }
     x->ctemp = p; p += nc;
@@ -1414,7 +1398,8 @@ extern "C" int mcf_init(const mcf_config *cfg, mcf_ctx **out) {
     INITCHK(hipMemcpyAsync(x->gx[d], x->hx[d].data(), (n[d] + 4) * sizeof(double), hipMemcpyHostToDevice, x->stream));
     INITCHK(hipMemcpyAsync(x->gdx[d], x->hdx[d].data(), (n[d] + 4) * sizeof(double), hipMemcpyHostToDevice, x->stream));
   }
-  INITCHK(hipHostMalloc((void **)&x->hred, 2 * sizeof(double), hipHostMallocDefault));
+  INITCHK(hipHostMalloc((void **)&x->hred, 4 * sizeof(double), hipHostMallocCoherent));
+  std::memset(x->hred, 0, 4 * sizeof(double));
   INITCHK(hipMalloc(&x->mlp, 4 * MLP_NP * sizeof(float)));
   INITCHK(hipMalloc(&x->mlp_pk, MLP_NPK * sizeof(__bf16)));
   INITCHK(hipMalloc(&x->cool_cnt, 4 * sizeof(unsigned long long)));
@@ -1551,16 +1536,33 @@ extern "C" int mcf_timestep(mcf_ctx *x, double tsave, double *dt_out, int *tag) 
   DtArgs A{};
   for (int f = 0; f < 8; ++f) { A.U[f] = x->U[f]; A.sp[f] = x->sp[f]; }
   for (int c = 0; c < 3; ++c) { A.bcc[c] = x->bcc[c]; A.gdx[c] = x->gdx[c]; }
-  A.out = x->red;
+  A.done = reinterpret_cast<unsigned *>(x->red);
+  A.part = x->red + 16;
+  A.out = x->hred;
+  A.stamp = reinterpret_cast<unsigned long long *>(x->hred + 2);
+  A.seq = ++x->dtseq;
   A.tfinal = x->cfg.tfinal;
   A.cols = chem_cols(x);
-  long rows = (long)x->g.n[1] * x->g.n[2];
-  unsigned nb = (unsigned)(rows < DT_BLOCKS ? rows : DT_BLOCKS);
-  if (x->chem) KLAUNCH_N("k_dtmin", k_dtmin<true>, dim3(nb), dim3(256), 184.0 * (double)rows * x->g.n[0], A, x->g, x->red + 16);
-  else KLAUNCH_N("k_dtmin", k_dtmin<false>, dim3(nb), dim3(256), 104.0 * (double)rows * x->g.n[0], A, x->g, x->red + 16);
-  KLAUNCH_G(k_dtfinal, dim3(1), dim3(256), 16.0 * nb, x->red + 16, (int)nb, x->red, x->cfg.tfinal);
-  HIPCHK(hipMemcpyAsync(x->hred, x->red, 2 * sizeof(double), hipMemcpyDeviceToHost, x->stream));
-  HIPCHK(hipStreamSynchronize(x->stream));
+  const long cells = (long)x->g.n[0] * x->g.n[1] * x->g.n[2];
+  const long tiles = (long)((x->g.n[0] + 63) / 64) * x->g.n[1] * x->g.n[2];
+  const unsigned nb = (unsigned)std::min<long>((tiles + DT_WAVES - 1) / DT_WAVES, DT_BLOCKS);
+  if (x->chem) KLAUNCH_N("k_dtmin", k_dtmin<true>, dim3(nb), dim3(64 * DT_WAVES), 184.0 * (double)cells, A, x->g);
+  else KLAUNCH_N("k_dtmin", k_dtmin<false>, dim3(nb), dim3(64 * DT_WAVES), 104.0 * (double)cells, A, x->g);
+  // The minima arrive with the launch's number; waiting for that instead of
+  // the stream saves the copy and the wake-up (about 15 us a step).  A step
+  // longer than the spin waits for the stream, which also reports errors.
+  {
+    volatile unsigned long long *stamp = A.stamp;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(4);
+    for (unsigned n = 1; __atomic_load_n(stamp, __ATOMIC_ACQUIRE) != A.seq; ++n) {
+      if ((n & 63u) == 0 && std::chrono::steady_clock::now() > until) {
+        HIPCHK(hipStreamSynchronize(x->stream));
+        if (__atomic_load_n(stamp, __ATOMIC_ACQUIRE) == A.seq) break;
+        g_err = "the dt reduction did not finish";
+        return MCF_E_HIP;
+      }
+    }
+  }
   double tCFL = x->hred[0], tLMT = x->hred[1];
   double tfinal = x->cfg.tfinal;
   double dt = tfinal;

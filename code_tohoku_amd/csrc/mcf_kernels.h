@@ -41,13 +41,7 @@ __device__ __forceinline__ void xcd_tile(int &bx, int &by, int &bz) {
   bz = (int)(t / (gx * gy));
 }
 
-struct FillList {
-  double *a[16];
-  int nf;
-  int dm[16]; // k_fill_yz: the passes of each field (bit 0: y, bit 1: z)
-};
-
-enum XRule { XR_PERIODIC = 0, XR_CONST, XR_COPY, XR_FACE, XR_MOM, XR_ENERGY, XR_SPECIES, XR_DTF };
+enum XRule { XR_NONE = -1, XR_PERIODIC = 0, XR_CONST, XR_COPY, XR_FACE, XR_MOM, XR_ENERGY, XR_SPECIES, XR_DTF };
 
 // Inflow density read from the DTF field shifted by -v t and wrapped in x
 // (XR_DTF): the field (float, the (-1:N+2)^3 box), the simulation time, the
@@ -60,13 +54,20 @@ struct DtfShift {
   double v[2], dx0[2], L[2];
 };
 
-// x-direction fill with the inflow (BC=4) rules of BC_MPI / BC_MPI_OT
-struct XFill {
-  double *a[16];
-  int rule[16][2];   // per field and side (0 = left ghosts 1-nol..0, 1 = right N+1..N+nol)
-  double val[16][2];
-  int src[16][2];
+// One ghost fill (k_fill): per field its x rule on each side (BC_MPI /
+// BC_MPI_OT; XR_NONE: no x pass) and its periodic passes (dm, bit 0: y,
+// bit 1: z)
+constexpr int FILL_MAXF = 16;
+struct Fill {
+  double *a[FILL_MAXF];
+  int rule[FILL_MAXF][2]; // per side (0 = left ghosts 1-nol..0, 1 = right N+1..N+nol)
+  double val[FILL_MAXF][2];
+  int src[FILL_MAXF][2];
+  int dm[FILL_MAXF];
   int nf;
+  int rho_f; // the field that is rho, when this fill has an x pass of it, else -1
+  int anyx, anyyz;
+  double *mirror; // if set, field 0's first ghost layer is written here too
   const double *rho, *bcc1, *blg1, *blg2;
   double val2[2];
   DtfShift dtf;
@@ -161,7 +162,11 @@ struct DtArgs {
   const double *sp[8];
   const double *bcc[3];
   const double *gdx[3];
-  double *out;
+  double *part;              // one pair of partial minima per block
+  unsigned *done;            // blocks finished, zero between launches
+  double *out;               // host memory: the two minima ...
+  unsigned long long *stamp; // ... and the launch's number, written after them
+  unsigned long long seq;
   double tfinal;
   ChemCols cols; // column densities the chemistry Fcool reads
 };
@@ -193,8 +198,7 @@ struct DisArgs {
   double *divv;
 };
 
-__global__ void k_fill_yz(FillList L, Geo g, int nol);
-__global__ void k_fill_xrule(XFill X, Geo g, int nol);
+__global__ void k_fill(Fill F, Geo g, int nol);
 __global__ void k_cc1(CtArgs A, Geo g, Box b);
 template <class R> __global__ void k_ct_march(CtArgs A, Geo g, double dt);
 // k_ct_march: EMF cells per wave, waves per block
@@ -204,12 +208,13 @@ __global__ void k_cc4(CtArgs A, Geo g, Box b);
 // CHEM: the chemistry-network Fcool (R = double only) instead of the KI one
 template <class R, bool CHEM = false> __global__ void k_src_col(SrcArgs A, Geo g, Box b, double dt, int stage);
 constexpr int SRC_ROWS = 8;  // x rows (waves) per block of k_src_col
-__global__ void k_shell_copy(const double *__restrict__ src, double *__restrict__ dst, Geo g);
 __global__ void k_src_stiff(SrcArgs A, double dt, int stage);
 template <bool CHEM = false> __global__ void k_src_imc(SrcArgs A, double dt, int stage, int which);
 __global__ void k_zero_u32x2(unsigned *p);
-template <bool CHEM = false> __global__ void k_dtmin(DtArgs A, Geo g, double *part);
-__global__ void k_dtfinal(const double *part, int nb, double *out, double tfinal);
+template <bool CHEM = false> __global__ void k_dtmin(DtArgs A, Geo g);
+// waves per block of k_dtmin: the blocks' counts meet at one address, so few
+// large blocks (256 of 16 waves at 64^3 instead of 1024 of 4)
+constexpr int DT_WAVES = 16;
 __global__ void k_dissip_div(DisArgs A, Geo g, int e0);
 __global__ void k_dissip_upd(DisArgs A, Geo g, int e0);
 __global__ void k_copy(const double *__restrict__ a, double *__restrict__ b, long n);

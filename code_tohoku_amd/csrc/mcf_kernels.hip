@@ -43,106 +43,132 @@ __device__ __forceinline__ double gammi1_of(const double *const *sp, int c) {
 // ---------------------------------------------------------------------------
 // ghost fills
 // ---------------------------------------------------------------------------
-// The periodic y pass and then the periodic z pass of a fill in one launch.
-// Done in sequence, the passes leave at a ghost point (i, j, k) the value of
-// (i, jw, kw), where jw = j -+ n1 if the point's field has a y pass and j is
-// one of its nol ghost layers (else jw = j), and kw likewise along z; no
-// such source point is written by either pass, so every point can copy its
-// source directly.  Points: the y ghost layers over all (i, k), then the z
-// ghost layers over all i and the j outside the y ghost layers.
-__global__ void k_fill_yz(FillList L, Geo g, int nol) {
-  const int m0 = g.n[0] + 4, m1 = g.n[1] + 4, m2 = g.n[2] + 4, n1 = g.n[1], n2 = g.n[2];
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long ra = 2L * nol * m0 * m2, rb = 2L * nol * m0 * (m1 - 2 * nol);
+// x-ghost value of field f at grid point (i, j, k), i in the ghost layers of
+// `side`: the rules of BC_MPI / BC_MPI_OT (M3:818-884, 948-1092) or the
+// periodic copy.  False where the rule leaves the point as it is.
+__device__ __forceinline__ bool fill_x(const Fill &F, const Geo &g, int f, int side, int i, int j, int k, double &v);
+
+// rho at the same ghost point after the x pass
+__device__ __forceinline__ double fill_rho(const Fill &F, const Geo &g, int side, int i, int j, int k) {
+  double r;
+  if (F.rho_f >= 0 && fill_x(F, g, F.rho_f, side, i, j, k, r)) return r;
+  return F.rho[ix3(g, i, j, k)];
+}
+
+__device__ __forceinline__ bool fill_x(const Fill &F, const Geo &g, int f, int side, int i, int j, int k, double &v) {
+  const int nx = g.n[0];
+  const double *a = F.a[f];
+  switch (F.rule[f][side]) {
+  case XR_PERIODIC: v = a[ix3(g, side == 0 ? i + nx : i - nx, j, k)]; return true;
+  case XR_CONST: v = F.val[f][side]; return true;
+  case XR_COPY: v = a[ix3(g, F.src[f][side], j, k)]; return true;
+  case XR_FACE: // U(:,:,:,6): left copies face 1, right only N+2 copies face N+1
+    if (side == 1 && i < nx + 2) return false;
+    v = a[ix3(g, side == 0 ? 1 : nx + 1, j, k)];
+    return true;
+  case XR_DTF: { // M3:818-826 (left), 854-861 (right), in the reference's operation order
+    const DtfShift &D = F.dtf;
+    const double dx0 = D.dx0[side], L = D.L[side];
+    double xp;
+    int nn;
+    if (side == 0) {
+      xp = D.xe[1] - 0.5 * dx0 + (double)i * dx0 - D.t * D.v[0];
+      nn = (int)(fabs(xp) / L) + 1;
+      xp = xp + L * (double)nn;
+    } else {
+      xp = 0.5 * (D.xe[i] + D.xe[i + 1]) - D.t * D.v[1];
+      nn = (int)(fabs(xp) / L);
+      xp = xp - L * (double)nn;
+    }
+    const int ii = (int)(xp / dx0) + 1;
+    v = (double)D.f[ix3(g, ii, j, k)];
+    return true;
+  }
+  }
+  return false;
+}
+
+// A fill: the x pass on every row, then the periodic y and z passes, in one
+// launch with one thread per ghost point and field.  In sequence the passes
+// leave at a ghost point (i, j, k) the x pass's value at (i, jw, kw), where
+// jw is the periodic image of j if the field has a y pass and j is one of its
+// nol ghost layers (else j itself), kw likewise along z.  No point a thread
+// reads is written in the same launch: sources are interior along every
+// wrapped axis, and along x the rules read interior cells; the rules that
+// read another field at the ghost point read arrays this launch does not
+// fill, or, for rho, form its value again (fill_rho).
+// Points: the x ghost layers over all rows (if any field has an x pass, the
+// layers of a row on adjacent threads), then the y ghost layers over the
+// other i and all k, then the z ghost layers over the other i and the j
+// outside the y ghost layers.  Two launches whose threads ran over the
+// fields in a loop, one load after the other, took 5.7 + 4.7 us at 64^3 (a
+// SOURCE fill of 10 fields); 4.9 us now, 28 us at 256^3 (34 before).
+__global__ void k_fill(Fill F, Geo g, int nol) {
+  const int f = blockIdx.y;
+  const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2], m0 = n0 + 4, m1 = n1 + 4, m2 = n2 + 4;
+  const int w = F.anyx ? m0 - 2 * nol : m0; // positions along x of the y and z ghosts
+  const unsigned ra = F.anyx ? 2u * nol * m1 * m2 : 0u; // all counts are below 4/8 of the grid's 2^31
+  const unsigned rb = F.anyyz ? 2u * nol * w * m2 : 0u, rc = F.anyyz ? 2u * nol * w * (m1 - 2 * nol) : 0u;
+  unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
   int i, j, k; // memory positions (index + 1)
+  // position q of the ones outside the ghost layers, of an axis of n cells
+  auto skip = [&](int q, int n) { return q < 2 - nol ? q : (q < 2 - nol + n ? q + nol : q + 2 * nol); };
   if (t < ra) {
-    i = (int)(t % m0);
-    long r = t / m0;
-    k = (int)(r % m2);
-    const int layer = (int)(r / m2);
-    j = layer < nol ? 2 - nol + layer : n1 + 2 + (layer - nol);
+    const int layer = (int)(t % (2u * nol));
+    const unsigned r = t / (2u * nol);
+    j = (int)(r % (unsigned)m1);
+    k = (int)(r / (unsigned)m1);
+    i = layer < nol ? 2 - nol + layer : n0 + 2 + (layer - nol);
   } else if ((t -= ra) < rb) {
-    i = (int)(t % m0);
-    long r = t / m0;
-    const int q = (int)(r % (m1 - 2 * nol));
-    const int layer = (int)(r / (m1 - 2 * nol));
-    j = q < 2 - nol ? q : (q < 2 - nol + n1 ? q + nol : q + 2 * nol);
+    const unsigned r = t / (unsigned)w;
+    i = (int)(t - r * w);
+    k = (int)(r % (unsigned)m2);
+    const int layer = (int)(r / (unsigned)m2);
+    j = layer < nol ? 2 - nol + layer : n1 + 2 + (layer - nol);
+    if (F.anyx) i = skip(i, n0);
+  } else if ((t -= rb) < rc) {
+    const unsigned r = t / (unsigned)w;
+    i = (int)(t - r * w);
+    j = skip((int)(r % (unsigned)(m1 - 2 * nol)), n1);
+    const int layer = (int)(r / (unsigned)(m1 - 2 * nol));
     k = layer < nol ? 2 - nol + layer : n2 + 2 + (layer - nol);
+    if (F.anyx) i = skip(i, n0);
   } else {
     return;
   }
   // ghost layers within nol: memory positions 2-nol..1 and n+2..n+1+nol
-  const bool yg = (j >= 2 - nol && j <= 1) || (j >= n1 + 2 && j <= n1 + 1 + nol);
-  const bool zg = (k >= 2 - nol && k <= 1) || (k >= n2 + 2 && k <= n2 + 1 + nol);
-  const int jw = j <= 1 ? j + n1 : j - n1, kw = k <= 1 ? k + n2 : k - n2;
+  auto in = [&](int q, int n) { return (q >= 2 - nol && q <= 1) || (q >= n + 2 && q <= n + 1 + nol); };
+  const bool wy = (F.dm[f] & 1) && in(j, n1), wz = (F.dm[f] & 2) && in(k, n2);
+  const int side = i <= 1 ? 0 : 1;
+  const int rule = in(i, n0) ? F.rule[f][side] : (int)XR_NONE;
+  if (rule == XR_NONE && !wy && !wz) return;
+  const int js = wy ? (j <= 1 ? j + n1 : j - n1) : j, ks = wz ? (k <= 1 ? k + n2 : k - n2) : k;
+  double *a = F.a[f];
+  const int gi = i - 1, gj = js - 1, gk = ks - 1;
+  double v;
+  bool ok = false;
+  if (rule == XR_MOM) {
+    v = fill_rho(F, g, side, gi, gj, gk) * F.val[f][side];
+    ok = true;
+  } else if (rule == XR_ENERGY) {
+    const double u = F.val2[side], r = fill_rho(F, g, side, gi, gj, gk);
+    const int c = ix3(g, gi, gj, gk);
+    v = F.val[f][side] * 1.5 + 0.5 * (r * (u * u) + F.bcc1[c] * F.bcc1[c] + F.blg1[c] * F.blg1[c] + F.blg2[c] * F.blg2[c]);
+    ok = true;
+  } else if (rule == XR_SPECIES) {
+    ok = gj >= 1 && gj <= n1 && gk >= 1 && gk <= n2; // interior rows only
+    if (ok) v = F.val[f][side] * fill_rho(F, g, side, gi, gj, gk);
+  } else if (rule != XR_NONE) {
+    ok = fill_x(F, g, f, side, gi, gj, gk, v);
+  }
+  if (!ok) {
+    if (!wy && !wz) return;
+    v = a[ix3(g, gi, gj, gk)];
+  }
   const int c = i + j * g.st[1] + k * g.st[2];
-  for (int f = 0; f < L.nf; ++f) {
-    const bool wy = yg && (L.dm[f] & 1), wz = zg && (L.dm[f] & 2);
-    if (!wy && !wz) continue;
-    L.a[f][c] = L.a[f][i + (wy ? jw : j) * g.st[1] + (wz ? kw : k) * g.st[2]];
-  }
-}
-
-// x-ghost rules of BC_MPI / BC_MPI_OT, the periodic copy (XR_PERIODIC) or
-// an inflow (BC=4) end's rules
-// (M3:818-884, 948-1092).  One thread per ghost point and side, the ghost
-// layers of a row on adjacent threads (adjacent in memory); the fields are
-// processed in list order, as the reference's K loop does.  A thread reads
-// only its own ghost point and interior points, so the order of the points
-// does not matter.
-__global__ void k_fill_xrule(XFill X, Geo g, int nol) {
-  int ny4 = g.n[1] + 4, nz4 = g.n[2] + 4, nx = g.n[0];
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long tot = (long)ny4 * nz4 * (2 * nol);
-  if (t >= tot) return;
-  int layer = (int)(t % (2 * nol));
-  long r = t / (2 * nol);
-  int j = (int)(r % ny4) - 1;
-  int k = (int)(r / ny4) - 1;
-  int side = layer < nol ? 0 : 1;
-  int i = side == 0 ? 1 - nol + layer : nx + 1 + (layer - nol);
-  int c = ix3(g, i, j, k);
-  bool inner = (j >= 1 && j <= g.n[1] && k >= 1 && k <= g.n[2]);
-  for (int f = 0; f < X.nf; ++f) {
-    double *a = X.a[f];
-    switch (X.rule[f][side]) {
-    case XR_PERIODIC: a[c] = a[ix3(g, side == 0 ? i + nx : i - nx, j, k)]; break;
-    case XR_CONST: a[c] = X.val[f][side]; break;
-    case XR_COPY: a[c] = a[ix3(g, X.src[f][side], j, k)]; break;
-    case XR_FACE: // U(:,:,:,6): left copies face 1, right only N+2 copies face N+1
-      if (side == 0) a[c] = a[ix3(g, 1, j, k)];
-      else if (i >= nx + 2) a[c] = a[ix3(g, nx + 1, j, k)];
-      break;
-    case XR_MOM: a[c] = X.rho[c] * X.val[f][side]; break;
-    case XR_ENERGY: {
-      double v = X.val2[side];
-      a[c] = X.val[f][side] * 1.5 + 0.5 * (X.rho[c] * (v * v) + X.bcc1[c] * X.bcc1[c] +
-                                          X.blg1[c] * X.blg1[c] + X.blg2[c] * X.blg2[c]);
-      break;
-    }
-    case XR_SPECIES:
-      if (inner) a[c] = X.val[f][side] * X.rho[c];
-      break;
-    case XR_DTF: { // M3:818-826 (left), 854-861 (right), in the reference's operation order
-      const DtfShift &D = X.dtf;
-      const double dx0 = D.dx0[side], L = D.L[side];
-      double xp;
-      int nn;
-      if (side == 0) {
-        xp = D.xe[1] - 0.5 * dx0 + (double)i * dx0 - D.t * D.v[0];
-        nn = (int)(fabs(xp) / L) + 1;
-        xp = xp + L * (double)nn;
-      } else {
-        xp = 0.5 * (D.xe[i] + D.xe[i + 1]) - D.t * D.v[1];
-        nn = (int)(fabs(xp) / L);
-        xp = xp - L * (double)nn;
-      }
-      const int ii = (int)(xp / dx0) + 1;
-      a[c] = (double)D.f[ix3(g, ii, j, k)];
-      break;
-    }
-    }
-  }
+  a[c] = v;
+  // the mirror takes the first ghost layer (the x pass runs on the outer rows too)
+  if (F.mirror && f == 0 && i >= 1 && i <= n0 + 2 && j >= 1 && j <= n1 + 2 && k >= 1 && k <= n2 + 2) F.mirror[c] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -449,7 +475,7 @@ __device__ __forceinline__ double qflux(double Tc, double Tcs, double dxi, doubl
 // A.Pout.  Stage 1 (corrector, dt): T from the predictor (A.Tp), P_old =
 // A.Pn, result written over A.Pn (= A.Pout; each cell reads only its own
 // P_old there).  Both stages cover the interior; the corrector's first
-// ghost layer takes the predictor's ghost values (k_shell_copy), as the
+// ghost layer takes the predictor's ghost values (the fill's mirror), as the
 // reference leaves them.
 // The backward-Euler cells (dt > 0.2*t_cool) are not solved here: they are
 // queued with their conduction increment for k_src_stiff (the surrogate) or
@@ -654,27 +680,6 @@ template __global__ void k_src_col<double, false>(SrcArgs, Geo, Box, double, int
 template __global__ void k_src_col<float, false>(SrcArgs, Geo, Box, double, int);
 template __global__ void k_src_col<double, true>(SrcArgs, Geo, Box, double, int);
 
-// Copy of the first ghost layer around the interior, src -> dst: the faces
-// k = 0 and n2+1 with their edges and corners, then j = 0 and n1+1 over
-// k = 1..n2, then i = 0 and n0+1 over the interior (j, k).
-__global__ void k_shell_copy(const double *__restrict__ src, double *__restrict__ dst, Geo g) {
-  const long a0 = g.n[0] + 2, a1 = g.n[1] + 2, n1 = g.n[1], n2 = g.n[2];
-  const long fz = a0 * a1, fy = a0 * n2, fx = n1 * n2;
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  int i, j, k;
-  if (t < 2 * fz) {
-    i = (int)(t % a0); j = (int)((t / a0) % a1); k = t < fz ? 0 : g.n[2] + 1;
-  } else if ((t -= 2 * fz) < 2 * fy) {
-    i = (int)(t % a0); k = 1 + (int)((t / a0) % n2); j = t < fy ? 0 : g.n[1] + 1;
-  } else if ((t -= 2 * fy) < 2 * fx) {
-    j = 1 + (int)(t % n1); k = 1 + (int)((t / n1) % n2); i = t < fx ? 0 : g.n[0] + 1;
-  } else {
-    return;
-  }
-  const int c = ix3(g, i, j, k);
-  dst[c] = src[c];
-}
-
 // The queued backward-Euler cells of one SOURCE stage, 64 per wave: the
 // surrogate predicts, Newton steps refine, the residual test accepts; the
 // cell's conduction increment and the pressure clamps are then applied as
@@ -756,83 +761,89 @@ __device__ __forceinline__ double wave_min(double v) {
   return v;
 }
 
-// Two-pass min: each block strides over (j,k) rows and writes one pair of
-// partial minima; k_dtfinal folds them.  min is exact, so the result does
-// not depend on the order.
-template <bool CHEM> __global__ void k_dtmin(DtArgs A, Geo g, double *part) {
-  __shared__ double s0[16], s1[16];
-  const int nx = g.n[0];
-  const long rows = (long)g.n[1] * g.n[2];
+// Min in one launch: each wave strides over 64-cell tiles of rows, each
+// block writes one pair of partial minima, and the last block to finish
+// folds them (min is exact, so the result does not depend on the order) and
+// writes them to host memory, then the launch's number, which the host waits
+// for.  Bound by HBM at 256^3: 0.35 ms for 1.74 GB, 4.9 TB/s.  At 64^3 the
+// launch takes 16 us; a block of 256 threads per row, a second launch and a
+// copy to the host took 16 + 6 + 2 us and two gaps between launches.
+template <bool CHEM> __global__ __launch_bounds__(64 * DT_WAVES) void k_dtmin(DtArgs A, Geo g) {
+  __shared__ double s0[DT_WAVES], s1[DT_WAVES];
+  __shared__ bool lastb;
+  const int nx = g.n[0], lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int nt = (nx + 63) >> 6;
+  const int tiles = nt * g.n[1] * g.n[2];
   const double *const *sp = A.sp;
   double tc = A.tfinal, tl = A.tfinal;
-  for (long r = blockIdx.x; r < rows; r += gridDim.x) {
-    int j = 1 + (int)(r % g.n[1]), k = 1 + (int)(r / g.n[1]);
-    double dyj = A.gdx[1][j + 1], dzk = A.gdx[2][k + 1];
-    for (int i = 1 + threadIdx.x; i <= nx; i += blockDim.x) {
-      int c = ix3(g, i, j, k);
-      double rho = A.U[0][c], p = A.U[4][c];
-      double bx = A.bcc[0][c], by = A.bcc[1][c], bz = A.bcc[2][c];
-      double gamma = gam_of(sp, c);
-      double c2 = (gamma * p + bx * bx + by * by + bz * bz) / rho;
-      double dxi = A.gdx[0][i + 1];
-      double cf = sqrt(c2);
-      double t = dxi / (cf + fabs(A.U[1][c]));
-      tc = dmin(tc, t);
-      t = dyj / (cf + fabs(A.U[2][c]));
-      tc = dmin(tc, t);
-      t = dzk / (cf + fabs(A.U[3][c]));
-      tc = dmin(tc, t);
-      double Nn = sp[1][c] + sp[0][c] + sp[2][c] + sp[3][c] + sp[4][c];
-      double Tn = p / (KB * Nn);
-      double dl = dmin(dxi, dyj);
-      dl = dmin(dl, dzk);
-      double gi = gammi1_of(sp, c);
-      double alpha = gi * KCOND * sqrt(dmin(Tn, 15.0));
-      alpha = 0.4 * Nn * KB / alpha * (dl * dl);
-      double CooL;
-      if constexpr (CHEM) CooL = ch_fcool(ch_fc_setup(sp, A.cols, c), Tn);
-      else CooL = fcool_ki(rho, Tn);
-      double tauC = p / gi / fabs(CooL);
-      tauC = dmax(0.2 * tauC, 2.5e-4);
-      tl = dmin(tl, tauC);
-      tl = dmin(tl, alpha);
-    }
+  for (int w = __builtin_amdgcn_readfirstlane(DT_WAVES * (int)blockIdx.x + wid); w < tiles; w += DT_WAVES * (int)gridDim.x) {
+    const int r = w / nt, i = 1 + 64 * (w - r * nt) + lane;
+    const int j = 1 + r % g.n[1], k = 1 + r / g.n[1];
+    const double dyj = A.gdx[1][j + 1], dzk = A.gdx[2][k + 1];
+    if (i > nx) continue;
+    int c = ix3(g, i, j, k);
+    double rho = A.U[0][c], p = A.U[4][c];
+    double bx = A.bcc[0][c], by = A.bcc[1][c], bz = A.bcc[2][c];
+    double gamma = gam_of(sp, c);
+    double c2 = (gamma * p + bx * bx + by * by + bz * bz) / rho;
+    double dxi = A.gdx[0][i + 1];
+    double cf = sqrt(c2);
+    double t = dxi / (cf + fabs(A.U[1][c]));
+    tc = dmin(tc, t);
+    t = dyj / (cf + fabs(A.U[2][c]));
+    tc = dmin(tc, t);
+    t = dzk / (cf + fabs(A.U[3][c]));
+    tc = dmin(tc, t);
+    double Nn = sp[1][c] + sp[0][c] + sp[2][c] + sp[3][c] + sp[4][c];
+    double Tn = p / (KB * Nn);
+    double dl = dmin(dxi, dyj);
+    dl = dmin(dl, dzk);
+    double gi = gammi1_of(sp, c);
+    double alpha = gi * KCOND * sqrt(dmin(Tn, 15.0));
+    alpha = 0.4 * Nn * KB / alpha * (dl * dl);
+    double CooL;
+    if constexpr (CHEM) CooL = ch_fcool(ch_fc_setup(sp, A.cols, c), Tn);
+    else CooL = fcool_ki(rho, Tn);
+    double tauC = p / gi / fabs(CooL);
+    tauC = dmax(0.2 * tauC, 2.5e-4);
+    tl = dmin(tl, tauC);
+    tl = dmin(tl, alpha);
   }
   tc = wave_min(tc);
   tl = wave_min(tl);
-  int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if (lane == 0) { s0[wid] = tc; s1[wid] = tl; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    int nw = (blockDim.x + 63) >> 6;
-    for (int w = 1; w < nw; ++w) { tc = fmin(tc, s0[w]); tl = fmin(tl, s1[w]); }
-    part[2 * blockIdx.x] = tc;
-    part[2 * blockIdx.x + 1] = tl;
+    for (int w = 1; w < DT_WAVES; ++w) { tc = fmin(tc, s0[w]); tl = fmin(tl, s1[w]); }
+    // device-scope stores (past the XCD's L2), acknowledged before the count:
+    // a release fence per block would write back the whole L2 each time
+    // (0.45 against 0.34 ms at 256^3)
+    __hip_atomic_store(A.part + 2 * blockIdx.x, tc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(A.part + 2 * blockIdx.x + 1, tl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lastb = __hip_atomic_fetch_add(A.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
   }
-}
-
-template __global__ void k_dtmin<false>(DtArgs, Geo, double *);
-template __global__ void k_dtmin<true>(DtArgs, Geo, double *);
-
-__global__ void k_dtfinal(const double *part, int nb, double *out, double tfinal) {
-  __shared__ double s0[16], s1[16];
-  double tc = tfinal, tl = tfinal;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-    tc = fmin(tc, part[2 * b]);
-    tl = fmin(tl, part[2 * b + 1]);
+  __syncthreads();
+  if (!lastb) return;
+  tc = tl = A.tfinal;
+  for (int b = threadIdx.x; b < (int)gridDim.x; b += 64 * DT_WAVES) {
+    tc = fmin(tc, __hip_atomic_load(A.part + 2 * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    tl = fmin(tl, __hip_atomic_load(A.part + 2 * b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   }
   tc = wave_min(tc);
   tl = wave_min(tl);
-  int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if (lane == 0) { s0[wid] = tc; s1[wid] = tl; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    int nw = (blockDim.x + 63) >> 6;
-    for (int w = 1; w < nw; ++w) { tc = fmin(tc, s0[w]); tl = fmin(tl, s1[w]); }
-    out[0] = tc;
-    out[1] = tl;
+    for (int w = 1; w < DT_WAVES; ++w) { tc = fmin(tc, s0[w]); tl = fmin(tl, s1[w]); }
+    __hip_atomic_store(A.done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(A.out, tc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(A.out + 1, tl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(A.stamp, A.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
+template __global__ void k_dtmin<false>(DtArgs, Geo);
+template __global__ void k_dtmin<true>(DtArgs, Geo);
 
 // ---------------------------------------------------------------------------
 // DISSIP (M3:3143-3173)

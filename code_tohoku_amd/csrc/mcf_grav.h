@@ -44,7 +44,7 @@ struct GravGeo {
 };
 
 struct GravBuf {
-  double *phi2, *rho2, *res2, *rhs2; // split levels
+  double *phi2, *rho2, *rhs2;        // split levels
   double *phi1, *rho1, *res1, *rhs1; // whole-domain levels, need1+1 entries (1-based)
   double *bphi1;                     // 2 x (needb1+1), 1-based
   double *bphi2;
@@ -74,16 +74,16 @@ struct PbArgs {
 
 __global__ void k_grav_zero(double *a, long n);
 __global__ void k_grav_rhs(GravGeo G, const double *rho, Geo g, double *rhs2);
-__global__ void k_grav_rstrct(GravGeo G, double *uc2, const double *uf2, int lc, int mode);
+__global__ void k_grav_rstrct(GravGeo G, double *uc2, const double *uf2, int lc);
 __global__ void k_grav_exchange(GravGeo G, double *u2, int l, int flags);
 __global__ void k_grav_relax(GravGeo G, double *phi2, const double *rhs2, int l);
 template <int PP, int LMAX, int D, bool PL>
 __global__ void k_grav_relax_col(GravGeo G, double *phi2, const double *rhs2, int l, const double *Ein, double *Eout,
                                  long EP);
-__global__ void k_grav_resid(GravGeo G, double *res2, const double *phi2, const double *rhs2, int l);
-__global__ void k_grav_prolong(GravGeo G, double *uf2, const double *uc2, int lf, int mode, const double *bphi2);
-__global__ void k_grav_add(GravGeo G, double *uf2, const double *res2, int l);
+__global__ void k_grav_down(GravGeo G, double *phi2, double *rhs2, int lc);
+__global__ void k_grav_prolong(GravGeo G, double *phi2, int lf, int mode, const double *bphi2);
 __global__ void k_grav_collect(GravGeo G, double *u1, const double *u2);
+__global__ void k_grav_collect_resid(GravGeo G, double *phi1, double *res1, const double *phi2, const double *rhs2);
 __global__ void k_grav_divide(GravGeo G, double *u2, const double *u1);
 // the whole-domain part of the solve as one workgroup (prog: 0 set-up,
 // 1 FMG stage j < NGcr, 2 FMG stage NGcr before the split levels, 3 the

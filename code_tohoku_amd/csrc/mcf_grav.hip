@@ -115,9 +115,8 @@ __global__ void k_grav_rhs(GravGeo G, const double *rho, Geo g, double *rhs2) {
 // rstrctMPI (SG8:385-456) into split level lc from lc+1, coarse nodes
 // 1..nc of every rank: the first node of the first rank and the last node
 // of the last rank along an axis are copied, the other inner nodes take
-// 1/2 + 6 x 1/12; mode 1 zeroes the x-end nodes.  The exchange follows as
-// its own launch.
-__global__ void k_grav_rstrct(GravGeo G, double *uc2, const double *uf2, int lc, int mode) {
+// 1/2 + 6 x 1/12.  The exchange follows as its own launch.
+__global__ void k_grav_rstrct(GravGeo G, double *uc2, const double *uf2, int lc) {
   const int *nc = G.n[lc], *nf = G.n[lc + 1];
   const long cnt = (long)nc[0] * nc[1] * nc[2], t = g_tid();
   if (t >= cnt * G.npe) return;
@@ -146,10 +145,6 @@ __global__ void k_grav_rstrct(GravGeo G, double *uc2, const double *uf2, int lc,
     v = 0.5 * uf[p] + w * (uf[p + sx] + uf[p - sx] + uf[p + sy] + uf[p - sy] + uf[p + sz] + uf[p - sz]);
   } else {
     write = false;
-  }
-  if (mode == 1 && ((c[0] == 0 && ic[0] == 1) || (c[0] == G.S[0] - 1 && ic[0] == nc[0]))) {
-    v = 0.0;
-    write = true;
   }
   if (write) uc[g_idx(nc, ic[0], ic[1], ic[2])] = v;
 }
@@ -411,30 +406,57 @@ template __global__ void k_grav_relax_col<1, 1156, GRAV_RELAX_D1, false>(GravGeo
 template __global__ void k_grav_relax_col<4, 4356, GRAV_RELAX_D4, true>(GravGeo, double *, const double *, int,
                                                                         const double *, double *, long);
 
-// residMPI (SG8:918-952): nodes 1..n-1, then zero at the x-end nodes
-// (nodes in g_node's order, so that neighbouring threads touch neighbouring
-// addresses of the skewed layout)
-__global__ void k_grav_resid(GravGeo G, double *res2, const double *phi2, const double *rhs2, int l) {
+// residMPI (SG8:918-952) and its exchange at one node of split level l: node
+// (i,j,k) of rank c, a ghost taken to the node it is a copy of (whose
+// neighbours, ghosts included, are in its own block); zero at the x-end nodes.
+__device__ __forceinline__ double g_resid(const GravGeo &G, const double *phi2, const double *rhs2, int l, const int c_[3],
+                                          int i, int j, int k) {
   const int *n = G.n[l];
-  const long cnt = (long)n[0] * n[1] * n[2], t = g_tid();
-  if (t >= cnt * G.npe) return;
-  const int r = (int)(t / cnt);
-  int i, j, k;
-  g_node(n, t - r * cnt, i, j, k);
-  int c[3];
-  g_rank(G, r, c);
-  const long base = G.off[l] + r * G.bsz[l], p = g_idx(n, i, j, k);
-  if ((c[0] == 0 && i == 1) || (c[0] == G.S[0] - 1 && i == n[0])) {
-    res2[base + p] = 0.0;
-    return;
-  }
-  if (i > n[0] - 1 || j > n[1] - 1 || k > n[2] - 1) return;
-  const double *u = phi2 + base;
+  int c[3] = {c_[0], c_[1], c_[2]};
+  g_resolve(G, n, c, i, j, k, 63);
+  if ((c[0] == 0 && i <= 1) || (c[0] == G.S[0] - 1 && i == n[0])) return 0.0;
+  const long p = G.off[l] + g_rid(G, c[0], c[1], c[2]) * G.bsz[l] + g_idx(n, i, j, k);
+  const double *u = phi2 + p;
   const double h = G.Lbox / (double)((n[0] - 1) * G.S[0]);
   const double h2i = 1.0 / (h * h);
   const long J = n[1] + 1, JK = J * (n[2] + 1), sx = JK, sy = 1 + JK, sz = J + JK;
-  res2[base + p] =
-      -h2i * (u[p + sx] + u[p - sx] + u[p + sy] + u[p - sy] + u[p + sz] + u[p - sz] - 6.0 * u[p]) + rhs2[base + p];
+  return -h2i * (u[sx] + u[-sx] + u[sy] + u[-sy] + u[sz] + u[-sz] - 6.0 * u[0]) + rhs2[p];
+}
+
+// The way down from split level lc+1 to lc: residual, its restriction
+// (rstrctMPI, mode 1) into the right-hand side of lc at the nodes 1..n-1
+// (the only ones read there), and the potential of lc set to zero.  The
+// residual is formed where the restriction reads it (7 points per coarse
+// node, 7/8 of a pass over the fine nodes), so it is neither stored nor
+// exchanged: one launch instead of residual, exchange, restriction, exchange
+// and zeroing (20 ways down a solve; 256^3 on 8x8x8: 0.69 against 1.9 ms).
+__global__ void k_grav_down(GravGeo G, double *phi2, double *rhs2, int lc) {
+  const int *nc = G.n[lc];
+  const int m[3] = {nc[0] - 1, nc[1] - 1, nc[2] - 1};
+  const long cnt = (long)m[0] * m[1] * m[2], t = g_tid();
+  const long nz = G.bsz[lc] * G.npe, all = (long)gridDim.x * blockDim.x;
+  for (long q = t; q < nz; q += all) phi2[G.off[lc] + q] = 0.0;
+  if (t >= cnt * G.npe) return;
+  const int r = (int)(t / cnt);
+  int ic[3];
+  g_node(m, t - r * cnt, ic[0], ic[1], ic[2]);
+  int c[3];
+  g_rank(G, r, c);
+  bool copy = false;
+  for (int d = 0; d < 3; ++d)
+    if (c[d] == 0 && ic[d] == 1) copy = true;
+  const int fi = 2 * ic[0] - 1, fj = 2 * ic[1] - 1, fk = 2 * ic[2] - 1, lf = lc + 1;
+  double v = 0.0;
+  if (!(c[0] == 0 && ic[0] == 1)) {
+    auto R = [&](int i, int j, int k) { return g_resid(G, phi2, rhs2, lf, c, i, j, k); };
+    v = R(fi, fj, fk);
+    if (!copy) {
+      const double w = 1.0 / 12.0;
+      v = 0.5 * v + w * (R(fi + 1, fj, fk) + R(fi - 1, fj, fk) + R(fi, fj + 1, fk) + R(fi, fj - 1, fk) +
+                         R(fi, fj, fk + 1) + R(fi, fj, fk - 1));
+    }
+  }
+  rhs2[G.off[lc] + r * G.bsz[lc] + g_idx(nc, ic[0], ic[1], ic[2])] = v;
 }
 
 // Prolongation of interpMPI / interp (SG8:500-599): injection at odd
@@ -454,42 +476,48 @@ __device__ __forceinline__ double pro_node(const F &C, int i, int j, int k) {
   return (k & 1) ? pro_v(C, i, j, k) : .5 * (pro_v(C, i, j, k + 1) + pro_v(C, i, j, k - 1));
 }
 
-// interpMPI into split level lf (nodes 1..nf of every rank); mode 1 puts
-// the end-plane potential on the x-end nodes.  The exchange (low ghosts
-// only) follows as its own launch.
-__global__ void k_grav_prolong(GravGeo G, double *uf2, const double *uc2, int lf, int mode, const double *bphi2) {
+// interpMPI into split level lf with its exchange of the low ghosts: nodes
+// 0..nf of every rank, a low ghost taken to the node it is a copy of and
+// formed from that rank's coarse block (node 0 of the first x rank stays).
+// Mode 1 writes the potential, with the end-plane potential on the x-end
+// nodes; mode 0 adds to it (addintMPI, SG8:602-624; the interpolant is
+// neither stored nor exchanged).  An odd coordinate's two coarse nodes are
+// one and the same, and 0.5 (c + c) = c, so every node takes eight loads and
+// no branch.
+__global__ void k_grav_prolong(GravGeo G, double *phi2, int lf, int mode, const double *bphi2) {
   const int *nf = G.n[lf], *nc = G.n[lf - 1];
-  const long cnt = (long)nf[0] * nf[1] * nf[2], t = g_tid();
+  const int m[3] = {nf[0] + 1, nf[1] + 1, nf[2] + 1};
+  const long cnt = (long)m[0] * m[1] * m[2], t = g_tid();
   if (t >= cnt * G.npe) return;
   const int r = (int)(t / cnt);
   int i, j, k;
-  g_node(nf, t - r * cnt, i, j, k);
+  g_node(m, t - r * cnt, i, j, k);
+  --i; --j; --k;
   int c[3];
   g_rank(G, r, c);
-  const double *uc = uc2 + G.off[lf - 1] + r * G.bsz[lf - 1];
+  if (c[0] == 0 && i == 0) return;
+  const long out = G.off[lf] + r * G.bsz[lf] + g_idx(nf, i, j, k);
+  int rs = r;
+  if (i == 0 || j == 0 || k == 0) {
+    g_resolve(G, nf, c, i, j, k, 1 | 4 | 16);
+    rs = g_rid(G, c[0], c[1], c[2]);
+  }
   double v;
   const int side = (c[0] == 0 && i == 1) ? 0 : ((c[0] == G.S[0] - 1 && i == nf[0]) ? 1 : -1);
   if (mode == 1 && side >= 0) {
-    v = bphi2[G.boff[lf] + (2L * r + side) * (long)(nf[1] + 1) * (nf[2] + 1) + j + (long)(nf[1] + 1) * k];
+    v = bphi2[G.boff[lf] + (2L * rs + side) * (long)(nf[1] + 1) * (nf[2] + 1) + j + (long)(nf[1] + 1) * k];
   } else {
-    auto C = [&](int a, int b, int e) { return uc[g_idx(nc, (a + 1) / 2, (b + 1) / 2, (e + 1) / 2)]; };
-    v = pro_node(C, i, j, k);
+    const long J = nc[1] + 1, JK = J * (nc[2] + 1);
+    const double *u = phi2 + G.off[lf - 1] + rs * G.bsz[lf - 1] + g_idx(nc, (i + 2) / 2, (j + 2) / 2, (k + 2) / 2);
+    // the upper coarse node of each axis is (f+2)/2; the lower one f/2 at an
+    // even coordinate, the same node at an odd one
+    const long sx = (i & 1) ? 0 : JK, sy = (j & 1) ? 0 : 1 + JK, sz = (k & 1) ? 0 : J + JK;
+    auto w = [&](long o) { return .5 * (u[-o] + u[-o - sx]); };
+    auto vv = [&](long o) { return .5 * (w(o) + w(o + sy)); };
+    v = .5 * (vv(0) + vv(sz));
   }
-  uf2[G.off[lf] + r * G.bsz[lf] + g_idx(nf, i, j, k)] = v;
-}
-
-// addintMPI's update (SG8:602-624): every node 0..n, uf += res
-// (over the slots of the skewed layout, the unused ones skipped: a third of
-// the slots are nodes)
-__global__ void k_grav_add(GravGeo G, double *uf2, const double *res2, int l) {
-  const int *n = G.n[l];
-  const long n_ = G.bsz[l] * G.npe, t = g_tid();
-  if (t >= n_) return;
-  const int J = n[1] + 1, K = n[2] + 1;
-  const int s = (int)(t % G.bsz[l]);
-  const int j = s % J, k = (s / J) % K, i = s / (J * K) - j - k;
-  if (i < 0 || i > n[0]) return;
-  uf2[G.off[l] + t] = uf2[G.off[l] + t] + res2[G.off[l] + t];
+  if (mode == 1) phi2[out] = v;
+  else phi2[out] = phi2[out] + v;
 }
 
 // collect (SG8:339-366): the level-NGcr rank blocks into the whole-domain
@@ -508,6 +536,23 @@ __global__ void k_grav_collect(GravGeo G, double *u1, const double *u2) {
   }
   const int r = g_rid(G, c[0], c[1], c[2]);
   u1[G.p1[L] + t] = u2[G.off[L] + r * G.bsz[L] + g_idx(m, lo[0], lo[1], lo[2])];
+}
+
+// collect of the potential and of the residual at split level NGcr (the
+// residual formed where it is read)
+__global__ void k_grav_collect_resid(GravGeo G, double *phi1, double *res1, const double *phi2, const double *rhs2) {
+  const int L = G.NGcr, N1 = (1 << L) + 1;
+  const int *m = G.n[L];
+  const long t = g_tid();
+  if (t >= (long)N1 * N1 * N1) return;
+  const int g3[3] = {1 + (int)(t % N1), 1 + (int)((t / N1) % N1), 1 + (int)(t / ((long)N1 * N1))};
+  int c[3], lo[3];
+  for (int d = 0; d < 3; ++d) {
+    c[d] = min((g3[d] - 1) / (m[d] - 1), G.S[d] - 1);
+    lo[d] = g3[d] - c[d] * (m[d] - 1);
+  }
+  phi1[G.p1[L] + t] = phi2[G.off[L] + g_rid(G, c[0], c[1], c[2]) * G.bsz[L] + g_idx(m, lo[0], lo[1], lo[2])];
+  res1[G.p1[L] + t] = g_resid(G, phi2, rhs2, L, c, lo[0], lo[1], lo[2]);
 }
 
 // divide (SG8:369-382): whole-domain level NGcr into the rank blocks, the

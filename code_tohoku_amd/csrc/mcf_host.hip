@@ -1005,7 +1005,7 @@ static int grav_setup(mcf_ctx *x) {
   // every segment starts at an even double (16-byte alignment for double2)
   auto ev = [](long c) { return (c + 1) & ~1L; };
   const long n1 = ev(G.need1 + 1), nb1 = ev(2 * (G.needb1 + 1));
-  const long nz = 4 * ev(tot2) + 4 * n1 + nb1 + ev(totb); // cleared at every solve
+  const long nz = 3 * ev(tot2) + 4 * n1 + nb1 + ev(totb); // cleared at every solve
   const long nZ = 2L * npl * nn2 * H, nS = 2L * npl * nn2, nD = 2L * 2 * nn2 * H, nSD = 2L * 2 * nn2;
   const long ntab = 4L * (q4 + 2);
   // boundary planes of consecutive sweeps: 6 per rank block, two sets
@@ -1021,7 +1021,6 @@ static int grav_setup(mcf_ctx *x) {
   auto take = [&](long c) { double *r = p; p += ev(c); return r; };
   x->gb.phi2 = take(tot2);
   x->gb.rho2 = take(tot2);
-  x->gb.res2 = take(tot2);
   x->gb.rhs2 = take(tot2);
   x->gb.phi1 = take(n1);
   x->gb.rho1 = take(n1);
@@ -1085,7 +1084,7 @@ static int grav_exchange(mcf_ctx *x, double *u2, int l, int flags) {
   KLAUNCH_N(k_exchange_names[l], k_grav_exchange, dim3(gblocks(per * G.npe)), dim3(TPB), 16.0 * per * G.npe, G, u2, l, flags);
   return MCF_OK;
 }
-static const int XALL = 63, XLOW = 1 | 4 | 16;
+static const int XALL = 63;
 
 // per-level names of the relaxation launches (mcf_profile)
 static const char *const k_relax_names[GRAV_MAXL] = {
@@ -1157,7 +1156,7 @@ static int do_grav_solve(mcf_ctx *x) {
   // every array starts the solve at zero, as in the reference's fixture
   // build; the finest split level needs no clearing: what a solve reads
   // there before writing it (node 0 of the first x rank) is never written
-  for (double *a : {B.phi2, B.rho2, B.res2, B.rhs2}) CHK(grav_zero(x, a, G.off[G.NGL]));
+  for (double *a : {B.phi2, B.rho2, B.rhs2}) CHK(grav_zero(x, a, G.off[G.NGL]));
   CHK(grav_zero(x, B.phi1, x->gpool_n - (B.phi1 - x->gpool)));
   // PB
   const int nn1 = P.nn1, nn2 = P.nn2, H = nn1 / 2, NGL = G.NGL, NGcr = G.NGcr;
@@ -1197,9 +1196,9 @@ static int do_grav_solve(mcf_ctx *x) {
     const long nr = (long)(G.n[NGL][0] + 1) * (G.n[NGL][1] + 1) * (G.n[NGL][2] + 1) * G.npe;
     KLAUNCH_N("k_grav_rhs", k_grav_rhs, dim3(gblocks(nr)), dim3(TPB), 16.0 * nr, G, x->U[F_RHO], x->g, B.rhs2);
   }
-  auto rstrct = [&](double *uc, const double *uf, int lc, int mode) -> int {
+  auto rstrct = [&](double *uc, const double *uf, int lc) -> int {
     const long nr = (long)G.n[lc][0] * G.n[lc][1] * G.n[lc][2] * G.npe;
-    KLAUNCH_N("k_grav_rstrct", k_grav_rstrct, dim3(gblocks(nr)), dim3(TPB), 64.0 * nr, G, uc, uf, lc, mode);
+    KLAUNCH_N("k_grav_rstrct", k_grav_rstrct, dim3(gblocks(nr)), dim3(TPB), 64.0 * nr, G, uc, uf, lc);
     return grav_exchange(x, uc, lc, XALL);
   };
   auto collect = [&](double *u1, const double *u2) {
@@ -1221,13 +1220,13 @@ static int do_grav_solve(mcf_ctx *x) {
     KLAUNCH_N("k_copy", k_copy, dim3(gblocks(nr)), dim3(TPB), 16.0 * nr, src + G.off[l], dst + G.off[l], nr);
     return MCF_OK;
   };
-  auto prolong = [&](double *uf, const double *uc, int lf, int mode) -> int {
-    const long nr = (long)G.n[lf][0] * G.n[lf][1] * G.n[lf][2] * G.npe;
-    KLAUNCH_N("k_grav_prolong", k_grav_prolong, dim3(gblocks(nr)), dim3(TPB), 16.0 * nr, G, uf, uc, lf, mode, B.bphi2);
-    return grav_exchange(x, uf, lf, XLOW);
+  auto prolong = [&](int lf, int mode) -> int {
+    const long nr = (long)(G.n[lf][0] + 1) * (G.n[lf][1] + 1) * (G.n[lf][2] + 1) * G.npe;
+    KLAUNCH_N("k_grav_prolong", k_grav_prolong, dim3(gblocks(nr)), dim3(TPB), 24.0 * nr, G, B.phi2, lf, mode, B.bphi2);
+    return MCF_OK;
   };
-  CHK(rstrct(B.rho2, B.rhs2, NGL - 1, 0));
-  for (int l = NGL - 2; l >= NGcr; --l) CHK(rstrct(B.rho2, B.rho2, l, 0));
+  CHK(rstrct(B.rho2, B.rhs2, NGL - 1));
+  for (int l = NGL - 2; l >= NGcr; --l) CHK(rstrct(B.rho2, B.rho2, l));
   CHK(collect(B.rho1, B.rho2));
   CHK(coarse(0, 0));
   for (int j = 2; j <= NGL; ++j) {
@@ -1240,34 +1239,28 @@ static int do_grav_solve(mcf_ctx *x) {
       CHK(divide());
       CHK(copy_level(B.rhs2, B.rho2, NGcr));
     } else {
-      CHK(prolong(B.phi2, B.phi2, j, 1));
+      CHK(prolong(j, 1));
       if (j != NGL) CHK(copy_level(B.rhs2, B.rho2, j));
     }
     for (int cyc = 0; cyc < 2; ++cyc) {
       for (int jj = j; jj >= NGcr; --jj) {
         CHK(grav_relax(x, jj, j >= NGL ? 2 : 5));
-        {
-          const int *m = G.n[jj];
-          const long nr = (long)m[0] * m[1] * m[2] * G.npe;
-          KLAUNCH_N("k_grav_resid", k_grav_resid, dim3(gblocks(nr)), dim3(TPB), 24.0 * nr, G, B.res2, B.phi2,
-                    B.rhs2, jj);
-          CHK(grav_exchange(x, B.res2, jj, XALL));
-        }
         if (jj == NGcr) {
-          CHK(collect(B.phi1, B.phi2));
-          CHK(collect(B.res1, B.res2));
+          const long N1 = (1L << NGcr) + 1;
+          KLAUNCH_N("k_grav_collect_resid", k_grav_collect_resid, dim3(gblocks(N1 * N1 * N1)), dim3(TPB),
+                    40.0 * N1 * N1 * N1, G, B.phi1, B.res1, B.phi2, B.rhs2);
         } else {
-          CHK(rstrct(B.rhs2, B.res2, jj - 1, 1));
-          CHK(grav_zero(x, B.phi2 + G.off[jj - 1], G.bsz[jj - 1] * G.npe));
+          const int *m = G.n[jj - 1];
+          const long nr = (long)(m[0] - 1) * (m[1] - 1) * (m[2] - 1) * G.npe;
+          KLAUNCH_N("k_grav_down", k_grav_down, dim3(gblocks(nr)), dim3(TPB), 16.0 * 8.0 * nr + 8.0 * nr, G, B.phi2,
+                    B.rhs2, jj - 1);
         }
       }
       CHK(coarse(3, j));
       CHK(divide());
       CHK(grav_relax(x, NGcr, 5));
       for (int jj = NGcr + 1; jj <= j; ++jj) {
-        CHK(prolong(B.res2, B.phi2, jj, 0));
-        const long nr = G.bsz[jj] * G.npe;
-        KLAUNCH_N("k_grav_add", k_grav_add, dim3(gblocks(nr)), dim3(TPB), 24.0 * nr, G, B.phi2, B.res2, jj);
+        CHK(prolong(jj, 0));
         CHK(grav_relax(x, jj, j >= NGL ? 2 : 5));
       }
     }

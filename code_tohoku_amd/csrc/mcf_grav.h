@@ -24,8 +24,10 @@ constexpr int GRAV_MAX_NGCR = 4;
 constexpr int GRAV_NEED1_MAX = 5795;
 constexpr int GRAV_COARSE_THREADS = 1024;
 constexpr int GRAV_RELAX_THREADS = 1024;
-// planes of loads in flight in k_grav_relax_col with 1 and 4 columns per thread
-constexpr int GRAV_RELAX_D1 = 4, GRAV_RELAX_D4 = 1;
+constexpr int GRAV_LDS_NODES = 18 * 18 * 18; // k_grav_relax_lds: most nodes of a block, ghosts included
+constexpr int GRAV_LDS_THREADS = 512;
+// planes of loads in flight in k_grav_relax_col and k_grav_relax_col4
+constexpr int GRAV_RELAX_D = 4, GRAV_RELAX_D4 = 1;
 constexpr int GRAV_FFT_MAXL = 1024; // longest FFT line (nn1/2 and nn2)
 // 4 pi G (M3:35: G = 1.11142d-4, G4pi = 12.56637d0*G)
 constexpr double GRAV_G4PI = 12.56637 * 1.11142e-4;
@@ -44,11 +46,10 @@ struct GravGeo {
 };
 
 struct GravBuf {
-  double *phi2, *rho2, *rhs2;        // split levels
+  double *phi2[2], *rho2, *rhs2;     // split levels; the potential in two copies (a sweep writes the other one)
   double *phi1, *rho1, *res1, *rhs1; // whole-domain levels, need1+1 entries (1-based)
   double *bphi1;                     // 2 x (needb1+1), 1-based
   double *bphi2;
-  double *ex[2]; // boundary planes of consecutive sweeps (k_grav_relax_col), 6 per rank block
 };
 
 // threads of an exchange per rank block at a split level of nodes 0..n
@@ -77,11 +78,13 @@ __global__ void k_grav_rhs(GravGeo G, const double *rho, Geo g, double *rhs2);
 __global__ void k_grav_rstrct(GravGeo G, double *uc2, const double *uf2, int lc);
 __global__ void k_grav_exchange(GravGeo G, double *u2, int l, int flags);
 __global__ void k_grav_relax(GravGeo G, double *phi2, const double *rhs2, int l);
-template <int PP, int LMAX, int D, bool PL>
-__global__ void k_grav_relax_col(GravGeo G, double *phi2, const double *rhs2, int l, const double *Ein, double *Eout,
-                                 long EP);
-__global__ void k_grav_down(GravGeo G, double *phi2, double *rhs2, int lc);
-__global__ void k_grav_prolong(GravGeo G, double *phi2, int lf, int mode, const double *bphi2);
+__global__ void k_grav_relax_lds(GravGeo G, const double *src, double *dst, const double *rhs2, int l);
+template <int LMAX, int D>
+__global__ void k_grav_relax_col(GravGeo G, const double *src, double *dst, const double *rhs2, int l);
+template <int PP, int LMAX, int D>
+__global__ void k_grav_relax_col4(GravGeo G, const double *src, double *dst, const double *rhs2, int l);
+__global__ void k_grav_down(GravGeo G, const double *phif, double *phic, double *rhs2, int lc);
+__global__ void k_grav_prolong(GravGeo G, double *phif, const double *phic, int lf, int mode, const double *bphi2);
 __global__ void k_grav_collect(GravGeo G, double *u1, const double *u2);
 __global__ void k_grav_collect_resid(GravGeo G, double *phi1, double *res1, const double *phi2, const double *rhs2);
 __global__ void k_grav_divide(GravGeo G, double *u2, const double *u1);

@@ -254,114 +254,340 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The same sweep with each thread owning fixed (j,k) columns of the block
-// (PP of them) and walking i = t-j-k along them: the node's lower x
-// neighbour is the thread's own result of the previous plane (a register),
-// its lower y and z neighbours are the neighbouring columns' results of the
-// previous plane (LDS, two buffers by plane parity) or, on the j = 0 and
-// k = 0 faces, fixed ghost values staged in LDS at the start.  Everything
-// else a node reads is a value from before the sweep -- its upper
-// neighbours, the right-hand side, and its own old value (the upper x
-// neighbour loaded one plane earlier) -- and is loaded D planes ahead into a
-// ring of registers, so that D planes of loads are in flight behind the
-// plane being computed: a node on plane t+D+1 is written only after the
-// barrier that ends plane t+D, by which time its old value has arrived.
-// LMAX bounds (n1+1)(n2+1), (n0+1)(n2+1) and (n0+1)(n1+1).
-//
-// Sweeps in a row exchange halos through boundary planes instead of a
-// separate launch: with Eout, every node the sweep computes on the six
-// planes next to the block's faces (node 1 or n-1 along an axis) is also
-// written there; with Ein, the ghost nodes are first set from the
-// neighbours' planes of the previous sweep, resolved as BCsgr_MPI would
-// resolve them (a source at a closed x end, never written, is read from the
-// neighbour's block itself).  Plane layout per block: 6 planes of EP values
-// (x planes indexed by (j,k), y by (i,k), z by (i,j)); the instances with
-// PL false have no plane code.
-__device__ __forceinline__ long g_plane_at(const int *n, long EP, int i, int j, int k) {
-  if (i == 1) return 0 * EP + j + (long)(n[1] + 1) * k;
-  if (i == n[0] - 1) return 1 * EP + j + (long)(n[1] + 1) * k;
-  if (j == 1) return 2 * EP + i + (long)(n[0] + 1) * k;
-  if (j == n[1] - 1) return 3 * EP + i + (long)(n[0] + 1) * k;
-  if (k == 1) return 4 * EP + i + (long)(n[0] + 1) * j;
-  return 5 * EP + i + (long)(n[0] + 1) * j;
-}
+// ---------------------------------------------------------------------------
+// Sweeps from one copy of the level into another: a block reads its nodes and
+// ghosts from src and writes the swept nodes to dst, then puts those next to
+// its faces into the ghosts of the blocks that hold copies of them (in dst,
+// which no block reads in this launch), so the level is exchanged when the
+// launch ends, and no separate exchange is needed between sweeps or after
+// them.  BCsgr_MPI's six phases give a ghost the value of the node that is
+// its image along every axis on which it is a ghost (x: only inside the
+// domain); seen from that node, it goes out along every combination of the
+// axes on which it lies next to a face.  The boundary node n of the last x
+// rank is carried along with its y and z images.  Node 0 of the first x rank
+// is never written, in either copy.
+// ---------------------------------------------------------------------------
+struct GPush {
+  const GravGeo &G;
+  double *level; // dst of the level
+  const int *n;
+  int c[3];
+  long bsz;
+  __device__ __forceinline__ int axis(int d, int q) const { return q == 1 ? -1 : (q == n[d] - 1 ? 1 : 0); }
+  __device__ __forceinline__ void put(int dx, int dy, int dz, int i, int j, int k, double v) const {
+    int a = c[0] + dx, b = c[1] + dy, e = c[2] + dz;
+    b = b < 0 ? G.S[1] - 1 : (b == G.S[1] ? 0 : b);
+    e = e < 0 ? G.S[2] - 1 : (e == G.S[2] ? 0 : e);
+    if (dx) i = dx < 0 ? n[0] : 0;
+    if (dy) j = dy < 0 ? n[1] : 0;
+    if (dz) k = dz < 0 ? n[2] : 0;
+    level[g_rid(G, a, b, e) * bsz + g_idx(n, i, j, k)] = v;
+  }
+  // the images of all nodes next to a face; val(i, j, k) is the node's new
+  // value.  Combinations with x over the x faces, with y but not x over the
+  // y faces, z alone over the z faces.
+  template <class F> __device__ __forceinline__ void all(F val) const {
+    const int m0 = n[0] - 1, m1 = n[1] - 1, m2 = n[2] - 1;
+    const int me = c[0] == G.S[0] - 1 ? n[0] : m0; // last node along x carried
+    for (int q = threadIdx.x; q < 2 * m1 * m2; q += blockDim.x) {
+      const int s = q >= m1 * m2, r = q - s * m1 * m2, j = 1 + r % m1, k = 1 + r / m1, i = s ? m0 : 1, dx = s ? 1 : -1;
+      if (c[0] + dx < 0 || c[0] + dx >= G.S[0]) continue;
+      const int dy = axis(1, j), dz = axis(2, k);
+      const double v = val(i, j, k);
+      put(dx, 0, 0, i, j, k, v);
+      if (dy) put(dx, dy, 0, i, j, k, v);
+      if (dz) put(dx, 0, dz, i, j, k, v);
+      if (dy && dz) put(dx, dy, dz, i, j, k, v);
+    }
+    for (int q = threadIdx.x; q < 2 * me * m2; q += blockDim.x) {
+      const int s = q >= me * m2, r = q - s * me * m2, i = 1 + r % me, k = 1 + r / me, j = s ? m1 : 1, dy = s ? 1 : -1;
+      const int dz = axis(2, k);
+      const double v = val(i, j, k);
+      put(0, dy, 0, i, j, k, v);
+      if (dz) put(0, dy, dz, i, j, k, v);
+    }
+    // (i+j, j) with j fastest: neighbouring slots, here and at the image
+    const int zn = (me + m1 - 1) * m1;
+    for (int q = threadIdx.x; q < 2 * zn; q += blockDim.x) {
+      const int s = q >= zn, r = q - s * zn, j = 1 + r % m1, i = 2 + r / m1 - j, k = s ? m2 : 1;
+      if (i >= 1 && i <= me) put(0, 0, s ? 1 : -1, i, j, k, val(i, j, k));
+    }
+  }
+};
 
-template <int PP, int LMAX, int D, bool PL>
-__global__ __launch_bounds__(GRAV_RELAX_THREADS) void k_grav_relax_col(GravGeo G, double *phi2, const double *rhs2,
-                                                                       int l, const double *Ein, double *Eout, long EP) {
-  // two plane buffers, then the fixed ghost faces j = 0 and k = 0
-  __shared__ double lds[4 * LMAX];
+// A sweep of blocks that fit in LDS (at most GRAV_LDS_NODES nodes, ghosts
+// included, at most 256 (j,k) columns): the block is loaded whole, swept
+// plane by plane with one thread per column (a node's lower x neighbour is
+// the thread's last result, the others come from LDS), and written out.  The
+// right-hand side is loaded RD planes ahead by every lane, so the loads sit in
+// no branch and the compiler can count them.  Bound by the chain of planes
+// (an LDS round trip and nine dependent FP64 operations each).
+typedef unsigned g_u2 __attribute__((ext_vector_type(2)));
+constexpr int RD = 4;
+__global__ __launch_bounds__(GRAV_LDS_THREADS) void k_grav_relax_lds(GravGeo G, const double *src, double *dst,
+                                                                     const double *rhs2, int l) {
+  __shared__ double U[GRAV_LDS_NODES];
   const int r = blockIdx.x;
   const int *n = G.n[l];
   int c[3];
   g_rank(G, r, c);
-  double *u = phi2 + G.off[l] + r * G.bsz[l];
-  const double *rhs = rhs2 + G.off[l] + r * G.bsz[l];
-  if (PL && Ein) {
-    const int ng = (int)grav_nghost(n);
-    for (int q = threadIdx.x; q < ng; q += blockDim.x) {
-      int i, j, k, cc[3] = {c[0], c[1], c[2]};
-      if (!g_ghost(n, q, i, j, k)) continue;
-      int si = i, sj = j, sk = k;
-      if (!g_resolve(G, n, cc, si, sj, sk, 63)) continue;
-      const int rs = g_rid(G, cc[0], cc[1], cc[2]);
-      u[g_idx(n, i, j, k)] = (si == 0 || si == n[0]) ? phi2[G.off[l] + rs * G.bsz[l] + g_idx(n, si, sj, sk)]
-                                                     : Ein[rs * 6 * EP + g_plane_at(n, EP, si, sj, sk)];
+  const long base = G.off[l] + r * G.bsz[l];
+  const double *u = src + base, *rhs = rhs2 + base;
+  const double w = 1.0 / 6.0;
+  const double h = G.Lbox / (double)((n[0] - 1) * G.S[0]);
+  const double h2 = h * h;
+  const int li = c[0] == 0 ? 1 : 0;
+  const int n0 = n[0], m0 = n[0] - 1, m1 = n[1] - 1, m2 = n[2] - 1, T = m0 + m1 + m2;
+  const int I = n[0] + 1, J = n[1] + 1, JK = J * (n[2] + 1), IJ = I * J;
+  // load: hyperplanes, contiguous over their (j,k) columns, dealt out to the
+  // waves 64 columns at a time; a column without a node on a plane loads
+  // nothing (the buffer resource drops its offset).  Sixteen loads in flight
+  // per wave.
+  const int TM = n[0] + n[1] + n[2], wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const __amdgpu_buffer_rsrc_t ub = __builtin_amdgcn_make_buffer_rsrc((void *)u, 0, (int)(8 * G.bsz[l]), 0x00020000);
+  for (int q0 = 0; q0 < JK; q0 += 128) {
+    int p0[2], jk[2], q[2];
+#pragma unroll
+    for (int h_ = 0; h_ < 2; ++h_) {
+      q[h_] = q0 + 64 * h_ + (int)(threadIdx.x & 63);
+      jk[h_] = q[h_] < JK ? q[h_] % J + q[h_] / J : 1 << 20;
+      p0[h_] = I * q[h_];
     }
-    __syncthreads();
+    for (int t0 = wave; t0 <= TM; t0 += 8 * nw) {
+      double a[2][8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int h_ = 0; h_ < 2; ++h_) {
+          const int t = t0 + s * nw;
+          const bool ok = (unsigned)(t - jk[h_]) <= (unsigned)n0;
+          a[h_][s] = __builtin_bit_cast(
+              double, __builtin_amdgcn_raw_buffer_load_b64(ub, ok ? 8u * (unsigned)(q[h_] + JK * t) : 0xffffff00u, 0, 0));
+        }
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int h_ = 0; h_ < 2; ++h_) {
+          const int i = t0 + s * nw - jk[h_];
+          if ((unsigned)i <= (unsigned)n0) U[p0[h_] + i] = a[h_][s];
+        }
+    }
   }
+  __syncthreads();
+  const int q = min((int)threadIdx.x, m1 * m2 - 1), j = 1 + q % m1, k = 1 + q / m1, p0 = I * (j + J * k);
+  const bool on = (int)threadIdx.x < m1 * m2; // further waves only load and store
+  const double *rc = rhs + j + J * k;
+  auto rat = [&](int t) { return rc[(long)JK * min(t, T)]; };
+  double prev = U[p0], rr[RD];
+#pragma unroll
+  for (int s = 0; s < RD; ++s) rr[s] = rat(3 + s);
+  for (int tb = 3; tb <= T; tb += RD) {
+#pragma unroll
+    for (int s = 0; s < RD; ++s) {
+      const int i = tb + s - j - k, p = p0 + min(max(i, 1), m0);
+      const double sum = U[p + 1] + prev + U[p + I] + U[p - I] + U[p + IJ] + U[p - IJ] - h2 * rr[s];
+      const double v = (li && i == 1) ? U[p] : w * sum;
+      rr[s] = rat(tb + s + RD);
+      if (on && i >= 1 && i <= m0) {
+        U[p] = v;
+        prev = v;
+      }
+      lds_barrier();
+    }
+  }
+  // write back nodes 1..m0 (to n0 on the last x rank), then the images
+  const int me = c[0] == G.S[0] - 1 ? n0 : m0;
+  double *d = dst + base + j + J * k;
+  if (on)
+    for (int t = 3; t <= T + 1; ++t) {
+      const int i = t - j - k;
+      if (i >= 1 && i <= me) d[(long)JK * t] = U[p0 + i];
+    }
+  const GPush P{G, dst + G.off[l], n, {c[0], c[1], c[2]}, G.bsz[l]};
+  P.all([&](int a, int b, int e) { return U[a + I * (b + J * e)]; });
+}
+
+// A sweep of larger blocks, streamed: each thread owns one (j,k) column and
+// walks i = t-j-k along it.  The node's lower x neighbour is the thread's own
+// last result (a register), its lower y and z neighbours are the neighbouring
+// columns' results of the previous plane (LDS, two buffers by plane parity).
+// Its upper neighbours are values from before the sweep: along x the one
+// loaded for this plane, along y and z the ones the neighbouring columns
+// loaded for it (u(i,j+1,k) is the upper x neighbour of their node on the same
+// plane), passed on through LDS one plane ahead.  Ghosts on the four j and k
+// faces are staged in LDS at the start.  So a plane takes two loads per
+// column (upper x neighbour, right-hand side), issued D planes ahead into a
+// ring of registers: memory answers in about 2.4 us, four times a plane.
+// Loads and stores go through buffer resources, which drop the offsets of idle
+// lanes: with loads or stores inside a branch the compiler cannot count how
+// many are in flight and waits for all of them.  A wave runs only the planes on which one of its
+// columns, or a column next to them, has a node, and waits at the barriers of
+// the others.
+template <int LMAX, int D>
+__global__ __launch_bounds__(GRAV_RELAX_THREADS) void k_grav_relax_col(GravGeo G, const double *src, double *dst,
+                                                                       const double *rhs2, int l) {
+  // two planes of results (0, 1), two of old values (2, 3), the ghost faces
+  // j = 0, k = 0, j = n1, k = n2 (4 .. 7); idle lanes read up to 128 entries
+  // past either end of a face
+  constexpr int PAD = 128;
+  __shared__ double lds[8 * LMAX + PAD];
+  const int r = blockIdx.x;
+  const int *n = G.n[l];
+  int c[3];
+  g_rank(G, r, c);
+  const long base = G.off[l] + r * G.bsz[l];
+  const double *u = src + base, *rhs = rhs2 + base;
+  double *d = dst + base;
+  const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(d, 0, (int)(8 * G.bsz[l]), 0x00020000);
   const double w = 1.0 / 6.0;
   const double h = G.Lbox / (double)((n[0] - 1) * G.S[0]);
   const double h2 = h * h;
   const int li = c[0] == 0 ? 1 : 0;
   const int m0 = n[0] - 1, m1 = n[1] - 1, m2 = n[2] - 1, LJ = n[1] + 1, T = m0 + m1 + m2, I1 = n[0] + 1;
-  const long J = n[1] + 1, JK = J * (n[2] + 1), sx = JK, sy = 1 + JK, sz = J + JK;
+  const int JK = LJ * (n[2] + 1);
+  for (int q = threadIdx.x; q < I1 * (n[2] + 1); q += blockDim.x) {
+    lds[4 * LMAX + q] = u[g_idx(n, q % I1, 0, q / I1)];
+    lds[6 * LMAX + q] = u[g_idx(n, q % I1, n[1], q / I1)];
+  }
+  for (int q = threadIdx.x; q < I1 * (n[1] + 1); q += blockDim.x) {
+    lds[5 * LMAX + q] = u[g_idx(n, q % I1, q / I1, 0)];
+    lds[7 * LMAX + q] = u[g_idx(n, q % I1, q / I1, n[2])];
+  }
+  const int q = min((int)threadIdx.x, m1 * m2 - 1), j = 1 + q % m1, k = 1 + q / m1, jk = j + k, cell = j + LJ * k;
+  // threads past the last column run it once more (the same values) and store nothing
+  const bool on = (int)threadIdx.x < m1 * m2;
+  double prev = u[cell + JK * jk];
+  const double u1 = u[cell + JK * (jk + 1)]; // nodes 0 and 1 before the sweep
+  // planes of this wave: from two before its first column's first node (the
+  // old value a neighbour needs, passed on one plane ahead) to its last one
+  const int q0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u)), q1 = min(q0 + 63, m1 * m2 - 1);
+  const bool row = q0 / m1 == q1 / m1;
+  const int t0 = (row ? 1 + q0 % m1 : 1) + 1 + q0 / m1 - 1;
+  const int len = (m0 + (row ? 1 + q1 % m1 : m1) + 1 + q1 / m1 - t0 + 1 + D - 1) / D * D;
+  const int NB = T + 2 * D; // barriers every wave reaches, planes 1 .. NB
+  // Positions in lds of the neighbours read on plane t0 + s, s even (e) and
+  // odd (o): fixed in the plane buffers, moving with i on a ghost face.
+  // A face has row length I1; positions of idle lanes stay within PAD of it.
+  const int pe = t0 & 1, i0 = t0 - jk; // parity of plane t0; i there (>= -m1 - 1, below m0 + m1 + D)
+  auto pos = [&](bool face, int f, int fq, int plane, int off) { return face ? f * LMAX + fq + i0 : plane * LMAX + cell + off; };
+  int ym[2], zm[2], yp[2], zp[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    ym[s] = pos(j == 1, 4, I1 * k + s, pe ^ s ^ 1, -1);
+    zm[s] = pos(k == 1, 5, I1 * j + s, pe ^ s ^ 1, -LJ);
+    yp[s] = pos(j == m1, 6, I1 * k + s, 2 + (pe ^ s), 1);
+    zp[s] = pos(k == m2, 7, I1 * j + s, 2 + (pe ^ s), LJ);
+  }
+  const int ay = j == 1 ? 2 : 0, az = k == 1 ? 2 : 0, by = j == m1 ? 2 : 0, bz = k == m2 ? 2 : 0;
+  const int wc[2] = {pe * LMAX + cell, (pe ^ 1) * LMAX + cell};                   // own result on an even / odd plane
+  const int wx[2] = {(2 + (pe ^ 1)) * LMAX + cell, (2 + pe) * LMAX + cell};       // old value for the next plane
+  unsigned so = 8u * (unsigned)(cell + JK * t0);
+  double rx[D], rr[D];
+  const __amdgpu_buffer_rsrc_t ub = __builtin_amdgcn_make_buffer_rsrc((void *)u, 0, (int)(8 * G.bsz[l]), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)rhs, 0, (int)(8 * G.bsz[l]), 0x00020000);
+  auto fetch = [&](int s, int i, unsigned off) { // node i of the column, at byte offset off
+    const unsigned o = (unsigned)i <= (unsigned)m0 ? off : 0xffffff00u;
+    rx[s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ub, o, 8 * JK, 0));
+    rr[s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rb, o, 0, 0));
+  };
+  const unsigned sk = 8u * (unsigned)JK;
+#pragma unroll
+  for (int s = 0; s < D; ++s) fetch(s, i0 + s, so + (unsigned)s * sk);
+  __syncthreads();
+  for (int b = 1; b < t0; ++b) lds_barrier();
+  int i = i0;
+  for (int tb = t0; tb < t0 + len; tb += D) {
+#pragma unroll
+    for (int s = 0; s < D; ++s) {
+      const int e = s & 1;
+      const double vyp = lds[yp[e]], vym = lds[ym[e]], vzp = lds[zp[e]], vzm = lds[zm[e]];
+      const double sum = rx[s] + prev + vyp + vym + vzp + vzm - h2 * rr[s];
+      const double v = (li && i == 1) ? u1 : w * sum;
+      const bool act = (unsigned)(i - 1) < (unsigned)m0;
+      lds[wc[e]] = v; // read only by the columns that have this i on the next plane
+      lds[wx[e]] = rx[(s + 1) % D];
+      prev = act ? v : prev;
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(g_u2, v), db, act && on ? so : 0xffffffffu, 0, 0);
+      fetch(s, i + D, so + D * sk);
+      ym[e] += ay;
+      zm[e] += az;
+      yp[e] += by;
+      zp[e] += bz;
+      so += sk;
+      ++i;
+      lds_barrier();
+    }
+  }
+  for (int b = t0 + len; b <= NB; ++b) lds_barrier();
+  if (c[0] == G.S[0] - 1) // the boundary nodes of the last x rank
+    for (int e = threadIdx.x; e < m1 * m2; e += blockDim.x) {
+      const long p = g_idx(n, n[0], 1 + e % m1, 1 + e / m1);
+      d[p] = u[p];
+    }
+  __syncthreads(); // the block's stores, before they are read again
+  const GPush P{G, dst + G.off[l], n, {c[0], c[1], c[2]}, G.bsz[l]};
+  P.all([&](int a, int b, int e) { return d[g_idx(n, a, b, e)]; });
+}
+template __global__ void k_grav_relax_col<1156, GRAV_RELAX_D>(GravGeo, const double *, double *, const double *, int);
+
+// The same for blocks of up to four columns per thread, whose faces and old
+// values do not fit LDS: the upper y and z neighbours are loaded, the faces
+// j = 0 and k = 0 staged.
+template <int PP, int LMAX, int D>
+__global__ __launch_bounds__(GRAV_RELAX_THREADS) void k_grav_relax_col4(GravGeo G, const double *src, double *dst,
+                                                                       const double *rhs2, int l) {
+  // two plane buffers, then the ghost faces j = 0 and k = 0
+  __shared__ double lds[4 * LMAX];
+  const int r = blockIdx.x;
+  const int *n = G.n[l];
+  int c[3];
+  g_rank(G, r, c);
+  const long base = G.off[l] + r * G.bsz[l];
+  const double *u = src + base, *rhs = rhs2 + base;
+  double *d = dst + base;
+  const __amdgpu_buffer_rsrc_t db = __builtin_amdgcn_make_buffer_rsrc(d, 0, (int)(8 * G.bsz[l]), 0x00020000);
+  const double w = 1.0 / 6.0;
+  const double h = G.Lbox / (double)((n[0] - 1) * G.S[0]);
+  const double h2 = h * h;
+  const int li = c[0] == 0 ? 1 : 0;
+  const int m0 = n[0] - 1, m1 = n[1] - 1, m2 = n[2] - 1, LJ = n[1] + 1, T = m0 + m1 + m2, I1 = n[0] + 1;
+  const int JK = LJ * (n[2] + 1);
   double *gyf = lds + 2 * LMAX, *gzf = lds + 3 * LMAX;
   for (int q = threadIdx.x; q < I1 * (n[2] + 1); q += blockDim.x) gyf[q] = u[g_idx(n, q % I1, 0, q / I1)];
   for (int q = threadIdx.x; q < I1 * (n[1] + 1); q += blockDim.x) gzf[q] = u[g_idx(n, q % I1, q / I1, 0)];
-  __syncthreads();
   int pj[PP], pk[PP];
   bool on[PP];
-  // per column: the lower x neighbour (the ghost u(0,j,k), then the last
-  // result) and the old value of the node to compute (u(1,j,k) at first)
-  double prev[PP], fon[PP];
-  // ring slot s: the loads of the node on plane t = 3 + s (mod D)
+  double prev[PP], u1[PP]; // the lower x neighbour; node 1 before the sweep
+  // ring slot s: the loads of the node on plane t = t0 + s (mod D)
   double rx[D][PP], ry[D][PP], rz[D][PP], rr[D][PP];
 #pragma unroll
   for (int p = 0; p < PP; ++p) {
-    const int q = threadIdx.x + p * blockDim.x;
-    on[p] = q < m1 * m2;
-    pj[p] = on[p] ? 1 + q % m1 : 1;
-    pk[p] = on[p] ? 1 + q / m1 : 1;
+    // columns past the last one run it once more (the same values) and store nothing
+    const int q = min((int)(threadIdx.x + p * blockDim.x), m1 * m2 - 1);
+    on[p] = (int)(threadIdx.x + p * blockDim.x) < m1 * m2;
+    pj[p] = 1 + q % m1;
+    pk[p] = 1 + q / m1;
     const long q1 = g_idx(n, 1, pj[p], pk[p]);
-    prev[p] = u[q1 - sx];
-    fon[p] = u[q1];
+    prev[p] = u[q1 - JK];
+    u1[p] = u[q1];
   }
   // 32-bit byte offsets from the block's (uniform) base: one register per address
-  const unsigned bx = 8u * (unsigned)sx, by = 8u * (unsigned)sy, bz = 8u * (unsigned)sz;
-  auto at = [](const double *base, unsigned off) { return *(const double *)((const char *)base + off); };
-  auto fetch = [&](int s, int p, int i) {
-    // with one column per thread only the columns whose node i exists load
-    // (the sweep is bound by the instructions its waves issue more than by
-    // the latency of these loads); with four, every column loads, a column
-    // off its nodes at an unused slot of the plane (held to 3..T) on the
-    // same cache lines as the others
-    if (PP == 1 && (!on[p] || i < 1 || i > m0)) return;
-    const int tq = min(i + pj[p] + pk[p], T);
-    const unsigned q = 8u * (unsigned)(pj[p] + LJ * (pk[p] + (n[2] + 1) * tq));
+  auto at = [](const double *b, unsigned off) { return *(const double *)((const char *)b + off); };
+  const unsigned bx = 8u * (unsigned)JK, by = bx + 8u, bz = bx + 8u * (unsigned)LJ;
+  auto fetch = [&](int s, int p, int t) {
+    const unsigned q = 8u * (unsigned)(pj[p] + LJ * pk[p] + JK * min(t, T));
     rx[s][p] = at(u, q + bx);
     ry[s][p] = at(u, q + by);
     rz[s][p] = at(u, q + bz);
     rr[s][p] = at(rhs, q);
   };
+  const int t0 = 3, len = (T - 2 + D - 1) / D * D;
 #pragma unroll
   for (int s = 0; s < D; ++s)
 #pragma unroll
-    for (int p = 0; p < PP; ++p) fetch(s, p, 3 + s - pj[p] - pk[p]);
-  // whole groups of D planes: on the planes past T every column's node is
-  // past its end (i > n0-1), so they only wait at the barrier, and the loop
-  // body has one shape
-  for (int tb = 3; tb <= T; tb += D) {
+    for (int p = 0; p < PP; ++p) fetch(s, p, t0 + s);
+  __syncthreads();
+  for (int tb = t0; tb < t0 + len; tb += D) {
 #pragma unroll
     for (int s = 0; s < D; ++s) {
       const int t = tb + s;
@@ -369,42 +595,30 @@ __global__ __launch_bounds__(GRAV_RELAX_THREADS) void k_grav_relax_col(GravGeo G
       const double *Lp = lds + ((t + 1) & 1) * LMAX;
 #pragma unroll
       for (int p = 0; p < PP; ++p) {
-        const int i = t - pj[p] - pk[p];
-        if (on[p] && i >= 1 && i <= m0) {
-          const double ym = pj[p] == 1 ? gyf[i + I1 * pk[p]] : Lp[(pj[p] - 1) + LJ * pk[p]];
-          const double zm = pk[p] == 1 ? gzf[i + I1 * pj[p]] : Lp[pj[p] + LJ * (pk[p] - 1)];
-          const int ifl = li * (1 / i);
-          const double sum = rx[s][p] + prev[p] + ry[s][p] + ym + rz[s][p] + zm - h2 * rr[s][p];
-          const double v = w * sum * (double)(1 - ifl) + (0.5 + copysign(0.5, (double)ifl - 0.5)) * fon[p];
-          u[g_idx(n, i, pj[p], pk[p])] = v;
-          Lc[pj[p] + LJ * pk[p]] = v;
-          prev[p] = v;
-          if (PL && Eout) {
-            double *E = Eout + r * 6 * EP;
-            if (i == 1) E[0 * EP + pj[p] + LJ * pk[p]] = v;
-            if (i == m0) E[1 * EP + pj[p] + LJ * pk[p]] = v;
-            if (pj[p] == 1) E[2 * EP + i + (long)(n[0] + 1) * pk[p]] = v;
-            if (pj[p] == m1) E[3 * EP + i + (long)(n[0] + 1) * pk[p]] = v;
-            if (pk[p] == 1) E[4 * EP + i + (long)(n[0] + 1) * pj[p]] = v;
-            if (pk[p] == m2) E[5 * EP + i + (long)(n[0] + 1) * pj[p]] = v;
-          }
-        }
-        if (i >= 1) fon[p] = rx[s][p];
-        fetch(s, p, i + D);
+        const int i = t - pj[p] - pk[p], ic = min(max(i, 1), m0), cell = pj[p] + LJ * pk[p];
+        const double ym = *(pj[p] == 1 ? gyf + ic + I1 * pk[p] : Lp + cell - 1);
+        const double zm = *(pk[p] == 1 ? gzf + ic + I1 * pj[p] : Lp + cell - LJ);
+        const double sum = rx[s][p] + prev[p] + ry[s][p] + ym + rz[s][p] + zm - h2 * rr[s][p];
+        const double v = (li && i == 1) ? u1[p] : w * sum;
+        const bool act = i >= 1 && i <= m0;
+        Lc[cell] = v; // read only by the columns that have this i on the next plane
+        prev[p] = act ? v : prev[p];
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(g_u2, v), db, act && on[p] ? 8u * (unsigned)(cell + JK * t) : 0xffffffffu, 0, 0);
+        fetch(s, p, t + D);
       }
       lds_barrier();
     }
   }
+  if (c[0] == G.S[0] - 1) // the boundary nodes of the last x rank
+    for (int q = threadIdx.x; q < m1 * m2; q += blockDim.x) {
+      const long p = g_idx(n, n[0], 1 + q % m1, 1 + q / m1);
+      d[p] = u[p];
+    }
+  __syncthreads(); // the block's stores, before they are read again
+  const GPush P{G, dst + G.off[l], n, {c[0], c[1], c[2]}, G.bsz[l]};
+  P.all([&](int a, int b, int e) { return d[g_idx(n, a, b, e)]; });
 }
-template __global__ void k_grav_relax_col<1, 1156, GRAV_RELAX_D1, true>(GravGeo, double *, const double *, int,
-                                                                        const double *, double *, long);
-template __global__ void k_grav_relax_col<1, 1156, GRAV_RELAX_D1, false>(GravGeo, double *, const double *, int,
-                                                                         const double *, double *, long);
-// (four columns per thread: the instance with the plane code, called
-// without planes, measured faster than the one without: 605 against 660 us
-// per sweep on 65^3-node blocks)
-template __global__ void k_grav_relax_col<4, 4356, GRAV_RELAX_D4, true>(GravGeo, double *, const double *, int,
-                                                                        const double *, double *, long);
+template __global__ void k_grav_relax_col4<4, 4356, GRAV_RELAX_D4>(GravGeo, const double *, double *, const double *, int);
 
 // residMPI (SG8:918-952) and its exchange at one node of split level l: node
 // (i,j,k) of rank c, a ghost taken to the node it is a copy of (whose
@@ -430,12 +644,12 @@ __device__ __forceinline__ double g_resid(const GravGeo &G, const double *phi2, 
 // node, 7/8 of a pass over the fine nodes), so it is neither stored nor
 // exchanged: one launch instead of residual, exchange, restriction, exchange
 // and zeroing (20 ways down a solve; 256^3 on 8x8x8: 0.69 against 1.9 ms).
-__global__ void k_grav_down(GravGeo G, double *phi2, double *rhs2, int lc) {
+__global__ void k_grav_down(GravGeo G, const double *phif, double *phic, double *rhs2, int lc) {
   const int *nc = G.n[lc];
   const int m[3] = {nc[0] - 1, nc[1] - 1, nc[2] - 1};
   const long cnt = (long)m[0] * m[1] * m[2], t = g_tid();
   const long nz = G.bsz[lc] * G.npe, all = (long)gridDim.x * blockDim.x;
-  for (long q = t; q < nz; q += all) phi2[G.off[lc] + q] = 0.0;
+  for (long q = t; q < nz; q += all) phic[G.off[lc] + q] = 0.0;
   if (t >= cnt * G.npe) return;
   const int r = (int)(t / cnt);
   int ic[3];
@@ -448,7 +662,7 @@ __global__ void k_grav_down(GravGeo G, double *phi2, double *rhs2, int lc) {
   const int fi = 2 * ic[0] - 1, fj = 2 * ic[1] - 1, fk = 2 * ic[2] - 1, lf = lc + 1;
   double v = 0.0;
   if (!(c[0] == 0 && ic[0] == 1)) {
-    auto R = [&](int i, int j, int k) { return g_resid(G, phi2, rhs2, lf, c, i, j, k); };
+    auto R = [&](int i, int j, int k) { return g_resid(G, phif, rhs2, lf, c, i, j, k); };
     v = R(fi, fj, fk);
     if (!copy) {
       const double w = 1.0 / 12.0;
@@ -484,7 +698,7 @@ __device__ __forceinline__ double pro_node(const F &C, int i, int j, int k) {
 // neither stored nor exchanged).  An odd coordinate's two coarse nodes are
 // one and the same, and 0.5 (c + c) = c, so every node takes eight loads and
 // no branch.
-__global__ void k_grav_prolong(GravGeo G, double *phi2, int lf, int mode, const double *bphi2) {
+__global__ void k_grav_prolong(GravGeo G, double *phif, const double *phic, int lf, int mode, const double *bphi2) {
   const int *nf = G.n[lf], *nc = G.n[lf - 1];
   const int m[3] = {nf[0] + 1, nf[1] + 1, nf[2] + 1};
   const long cnt = (long)m[0] * m[1] * m[2], t = g_tid();
@@ -508,7 +722,7 @@ __global__ void k_grav_prolong(GravGeo G, double *phi2, int lf, int mode, const 
     v = bphi2[G.boff[lf] + (2L * rs + side) * (long)(nf[1] + 1) * (nf[2] + 1) + j + (long)(nf[1] + 1) * k];
   } else {
     const long J = nc[1] + 1, JK = J * (nc[2] + 1);
-    const double *u = phi2 + G.off[lf - 1] + rs * G.bsz[lf - 1] + g_idx(nc, (i + 2) / 2, (j + 2) / 2, (k + 2) / 2);
+    const double *u = phic + G.off[lf - 1] + rs * G.bsz[lf - 1] + g_idx(nc, (i + 2) / 2, (j + 2) / 2, (k + 2) / 2);
     // the upper coarse node of each axis is (f+2)/2; the lower one f/2 at an
     // even coordinate, the same node at an odd one
     const long sx = (i & 1) ? 0 : JK, sy = (j & 1) ? 0 : 1 + JK, sz = (k & 1) ? 0 : J + JK;
@@ -516,8 +730,8 @@ __global__ void k_grav_prolong(GravGeo G, double *phi2, int lf, int mode, const 
     auto vv = [&](long o) { return .5 * (w(o) + w(o + sy)); };
     v = .5 * (vv(0) + vv(sz));
   }
-  if (mode == 1) phi2[out] = v;
-  else phi2[out] = phi2[out] + v;
+  if (mode == 1) phif[out] = v;
+  else phif[out] = phif[out] + v;
 }
 
 // collect (SG8:339-366): the level-NGcr rank blocks into the whole-domain

@@ -131,6 +131,7 @@ struct mcf_ctx {
   PbArgs pb{};
   double *gpool = nullptr; // one allocation for all of it
   long gpool_n = 0;        // doubles in gpool cleared at each solve
+  int gcur[GRAV_MAXL]{}; // per split level: the copy that holds the potential
   double *phi = nullptr;
   double2 *pbZ = nullptr, *pbS = nullptr, *pbD = nullptr, *pbSD = nullptr;
 };
@@ -1005,21 +1006,15 @@ static int grav_setup(mcf_ctx *x) {
   // every segment starts at an even double (16-byte alignment for double2)
   auto ev = [](long c) { return (c + 1) & ~1L; };
   const long n1 = ev(G.need1 + 1), nb1 = ev(2 * (G.needb1 + 1));
-  const long nz = 3 * ev(tot2) + 4 * n1 + nb1 + ev(totb); // cleared at every solve
+  const long nz = 4 * ev(tot2) + 4 * n1 + nb1 + ev(totb); // cleared at every solve
   const long nZ = 2L * npl * nn2 * H, nS = 2L * npl * nn2, nD = 2L * 2 * nn2 * H, nSD = 2L * 2 * nn2;
   const long ntab = 4L * (q4 + 2);
-  // boundary planes of consecutive sweeps: 6 per rank block, two sets
-  long nex = 0;
-  for (int l = G.NGcr; l <= G.NGL; ++l) {
-    const int *m = G.n[l];
-    const long ep = std::max((long)(m[1] + 1) * (m[2] + 1), std::max((long)(m[0] + 1) * (m[2] + 1), (long)(m[0] + 1) * (m[1] + 1)));
-    nex = std::max(nex, 6L * G.npe * ep);
-  }
-  const long total = nz + ev((long)x->ncell) + nZ + nS + nD + nSD + ntab + 4 * ev(npl) + 2 * ev(nex) + 16;
+  const long total = nz + ev((long)x->ncell) + nZ + nS + nD + nSD + ntab + 4 * ev(npl) + 16;
   HIPCHK(hipMalloc(&x->gpool, total * sizeof(double)));
   double *p = x->gpool;
   auto take = [&](long c) { double *r = p; p += ev(c); return r; };
-  x->gb.phi2 = take(tot2);
+  x->gb.phi2[0] = take(tot2);
+  x->gb.phi2[1] = take(tot2);
   x->gb.rho2 = take(tot2);
   x->gb.rhs2 = take(tot2);
   x->gb.phi1 = take(n1);
@@ -1040,8 +1035,6 @@ static int grav_setup(mcf_ctx *x) {
   double *dzq = take(npl);
   double *dfg = take(npl);
   int *dgx = (int *)take(npl);
-  x->gb.ex[0] = take(nex);
-  x->gb.ex[1] = take(nex);
   if (p > x->gpool + total) { g_err = "self-gravity: pool layout"; return MCF_E_ARG; }
   HIPCHK(hipMemsetAsync(x->gpool, 0, total * sizeof(double), x->stream));
   HIPCHK(hipMemcpyAsync(wf, tw[0].data(), (q4 + 2) * sizeof(double2), hipMemcpyHostToDevice, x->stream));
@@ -1092,50 +1085,43 @@ static const char *const k_relax_names[GRAV_MAXL] = {
     "k_grav_relax<6>", "k_grav_relax<7>", "k_grav_relax<8>", "k_grav_relax<9>", "k_grav_relax<10>", "k_grav_relax<11>",
     "k_grav_relax<12>", "k_grav_relax<13>", "k_grav_relax<14>", "k_grav_relax<15>"};
 
-// Gauss-Seidel sweeps at split level l: the column kernel (k_grav_relax_col)
-// when the block's (j,k) columns fit 1 or 4 per thread of 1024 and its
-// y-z plane and ghost faces fit the kernel's LDS buffers, else the
-// plane-by-plane kernel
+// Gauss-Seidel sweeps at split level l, each from the current copy of the
+// level into the other one: blocks that fit in LDS whole (k_grav_relax_lds),
+// else the streaming kernel when the block's (j,k) columns fit 1 or 4 per
+// thread of 1024 and its planes and ghost faces fit the LDS buffers, else
+// (larger blocks) plane by plane in place with an exchange after each sweep.
 static int grav_relax(mcf_ctx *x, int l, int times) {
   const GravGeo &G = x->gg;
   const int *n = G.n[l];
   const long cols = (long)(n[1] - 1) * (n[2] - 1);
   const long plane = std::max((long)(n[1] + 1) * (n[2] + 1),
                               (long)(n[0] + 1) * std::max(n[1] + 1, n[2] + 1)); // the LDS planes and ghost faces
-  const double bytes = 8.0 * 8.0 * (double)(n[0] - 1) * cols * G.npe;
-  const unsigned tb = (unsigned)std::min<long>(GRAV_RELAX_THREADS, std::max<long>(64, (cols + 63) / 64 * 64));
-  const long ep = std::max(plane, std::max((long)(n[0] + 1) * (n[2] + 1), (long)(n[0] + 1) * (n[1] + 1)));
-  const int kind = (cols <= GRAV_RELAX_THREADS && plane <= 1156) ? 1
+  const double bytes = 8.0 * 3.0 * (double)(n[0] - 1) * cols * G.npe;
+  const long nodes = (long)(n[0] + 1) * (n[1] + 1) * (n[2] + 1);
+  const bool lds = cols <= 256 && nodes <= GRAV_LDS_NODES;
+  const int kind = lds ? 2 : (cols <= GRAV_RELAX_THREADS && plane <= 1156) ? 1
                    : (cols <= 4 * GRAV_RELAX_THREADS && plane <= 4356) ? 4 : 0;
-  if (kind == 0) {
-    for (int t = 0; t < times; ++t) {
-      KLAUNCH_N(k_relax_names[l], k_grav_relax, dim3(G.npe), dim3(GRAV_RELAX_THREADS), bytes, G, x->gb.phi2,
-                x->gb.rhs2, l);
-      CHK(grav_exchange(x, x->gb.phi2, l, XALL));
-    }
-    return MCF_OK;
-  }
-  // Blocks of at most 9 nodes per side pass the halo between the sweeps of
-  // the sequence through boundary planes and exchange once after the last
-  // one; larger blocks exchange after every sweep (256^3, 8x8x8: the planes
-  // saved 9 us of launch per sweep at 5^3-node blocks but cost 130 us per
-  // sweep at 33^3).
-  const bool planes = std::max(n[0], std::max(n[1], n[2])) <= 9;
+  const unsigned tb = (unsigned)((cols + 63) / 64 * 64);
+  // blocks in LDS: more waves than columns need, for the loads and stores
+  const unsigned tl = nodes > 2048 ? 512u : nodes > 256 ? 256u : 64u;
   for (int t = 0; t < times; ++t) {
-    const double *ein = planes && t > 0 ? x->gb.ex[(t - 1) & 1] : nullptr;
-    double *eout = planes && t < times - 1 ? x->gb.ex[t & 1] : nullptr;
-    if (!planes && t > 0) CHK(grav_exchange(x, x->gb.phi2, l, XALL));
-    if (kind == 1 && planes)
-      KLAUNCH_N(k_relax_names[l], (k_grav_relax_col<1, 1156, GRAV_RELAX_D1, true>), dim3(G.npe), dim3(tb), bytes, G,
-                x->gb.phi2, x->gb.rhs2, l, ein, eout, ep);
+    double *a = x->gb.phi2[x->gcur[l]], *b = x->gb.phi2[x->gcur[l] ^ 1];
+    if (kind == 2)
+      KLAUNCH_N(k_relax_names[l], k_grav_relax_lds, dim3(G.npe), dim3(tl), bytes, G, a, b, x->gb.rhs2, l);
     else if (kind == 1)
-      KLAUNCH_N(k_relax_names[l], (k_grav_relax_col<1, 1156, GRAV_RELAX_D1, false>), dim3(G.npe), dim3(tb), bytes, G,
-                x->gb.phi2, x->gb.rhs2, l, nullptr, nullptr, ep);
-    else
-      KLAUNCH_N(k_relax_names[l], (k_grav_relax_col<4, 4356, GRAV_RELAX_D4, true>), dim3(G.npe),
-                dim3(GRAV_RELAX_THREADS), bytes, G, x->gb.phi2, x->gb.rhs2, l, nullptr, nullptr, ep);
+      KLAUNCH_N(k_relax_names[l], (k_grav_relax_col<1156, GRAV_RELAX_D>), dim3(G.npe), dim3(tb), bytes, G, a, b,
+                x->gb.rhs2, l);
+    else if (kind == 4)
+      KLAUNCH_N(k_relax_names[l], (k_grav_relax_col4<4, 4356, GRAV_RELAX_D4>), dim3(G.npe), dim3(GRAV_RELAX_THREADS), bytes,
+                G, a, b, x->gb.rhs2, l);
+    if (kind != 0) {
+      x->gcur[l] ^= 1;
+      continue;
+    }
+    KLAUNCH_N(k_relax_names[l], k_grav_relax, dim3(G.npe), dim3(GRAV_RELAX_THREADS), bytes, G, a, x->gb.rhs2, l);
+    CHK(grav_exchange(x, a, l, XALL));
   }
-  return grav_exchange(x, x->gb.phi2, l, XALL);
+  return MCF_OK;
 }
 
 static int grav_zero(mcf_ctx *x, double *a, long n) {
@@ -1153,10 +1139,13 @@ static int do_grav_solve(mcf_ctx *x) {
   static const int l1[1] = {F_RHO};
   CHK(fillU(x, 7, 1, 1, l1, 1));
   CHK(fillU(x, 7, 2, 1, l1, 1));
+  // the potential's current copy of every level
+  auto cur = [&](int l) { return B.phi2[x->gcur[l]]; };
+  for (int l = 0; l < GRAV_MAXL; ++l) x->gcur[l] = 0;
   // every array starts the solve at zero, as in the reference's fixture
   // build; the finest split level needs no clearing: what a solve reads
   // there before writing it (node 0 of the first x rank) is never written
-  for (double *a : {B.phi2, B.rho2, B.rhs2}) CHK(grav_zero(x, a, G.off[G.NGL]));
+  for (double *a : {B.phi2[0], B.rho2, B.rhs2}) CHK(grav_zero(x, a, G.off[G.NGL]));
   CHK(grav_zero(x, B.phi1, x->gpool_n - (B.phi1 - x->gpool)));
   // PB
   const int nn1 = P.nn1, nn2 = P.nn2, H = nn1 / 2, NGL = G.NGL, NGcr = G.NGcr;
@@ -1212,7 +1201,7 @@ static int do_grav_solve(mcf_ctx *x) {
   };
   auto divide = [&]() {
     const long nr = (long)(G.n[NGcr][0] + 1) * (G.n[NGcr][1] + 1) * (G.n[NGcr][2] + 1) * G.npe;
-    KLAUNCH_N("k_grav_divide", k_grav_divide, dim3(gblocks(nr)), dim3(TPB), 16.0 * nr, G, B.phi2, B.phi1);
+    KLAUNCH_N("k_grav_divide", k_grav_divide, dim3(gblocks(nr)), dim3(TPB), 16.0 * nr, G, cur(NGcr), B.phi1);
     return MCF_OK;
   };
   auto copy_level = [&](double *dst, const double *src, int l) {
@@ -1222,7 +1211,8 @@ static int do_grav_solve(mcf_ctx *x) {
   };
   auto prolong = [&](int lf, int mode) -> int {
     const long nr = (long)(G.n[lf][0] + 1) * (G.n[lf][1] + 1) * (G.n[lf][2] + 1) * G.npe;
-    KLAUNCH_N("k_grav_prolong", k_grav_prolong, dim3(gblocks(nr)), dim3(TPB), 24.0 * nr, G, B.phi2, lf, mode, B.bphi2);
+    KLAUNCH_N("k_grav_prolong", k_grav_prolong, dim3(gblocks(nr)), dim3(TPB), 24.0 * nr, G, cur(lf), cur(lf - 1),
+              lf, mode, B.bphi2);
     return MCF_OK;
   };
   CHK(rstrct(B.rho2, B.rhs2, NGL - 1));
@@ -1248,12 +1238,12 @@ static int do_grav_solve(mcf_ctx *x) {
         if (jj == NGcr) {
           const long N1 = (1L << NGcr) + 1;
           KLAUNCH_N("k_grav_collect_resid", k_grav_collect_resid, dim3(gblocks(N1 * N1 * N1)), dim3(TPB),
-                    40.0 * N1 * N1 * N1, G, B.phi1, B.res1, B.phi2, B.rhs2);
+                    40.0 * N1 * N1 * N1, G, B.phi1, B.res1, cur(NGcr), B.rhs2);
         } else {
           const int *m = G.n[jj - 1];
           const long nr = (long)(m[0] - 1) * (m[1] - 1) * (m[2] - 1) * G.npe;
-          KLAUNCH_N("k_grav_down", k_grav_down, dim3(gblocks(nr)), dim3(TPB), 16.0 * 8.0 * nr + 8.0 * nr, G, B.phi2,
-                    B.rhs2, jj - 1);
+          KLAUNCH_N("k_grav_down", k_grav_down, dim3(gblocks(nr)), dim3(TPB), 16.0 * 8.0 * nr + 8.0 * nr, G, cur(jj),
+                    cur(jj - 1), B.rhs2, jj - 1);
         }
       }
       CHK(coarse(3, j));
@@ -1266,7 +1256,7 @@ static int do_grav_solve(mcf_ctx *x) {
     }
   }
   const long nc = (long)x->g.n[0] * x->g.n[1] * x->g.n[2];
-  KLAUNCH_N("k_grav_phi", k_grav_phi, dim3(gblocks(nc)), dim3(TPB), 16.0 * nc, G, B.phi2, x->phi, x->g);
+  KLAUNCH_N("k_grav_phi", k_grav_phi, dim3(gblocks(nc)), dim3(TPB), 16.0 * nc, G, cur(NGL), x->phi, x->g);
   const long ng = (long)x->g.n[1] * x->g.n[2] + (long)x->g.n[0] * x->g.n[2] + (long)x->g.n[0] * x->g.n[1];
   KLAUNCH_N("k_grav_phi_ghosts", k_grav_phi_ghosts, dim3(gblocks(ng)), dim3(TPB), 64.0 * ng, x->phi, x->g);
   return MCF_OK;

@@ -107,18 +107,22 @@ __device__ __forceinline__ double fcool_ki(double rho, double T) {
 }
 
 // IMC (M3:2898-2921): backward-Euler P + gammi1*Lambda(P)*dt = P_old by
-// bisection in log10 P on [1e-10, 1e10], at most 30 steps.
+// bisection in log10 P on [1e-10, 1e10], at most 30 steps.  The reference
+// keeps the bracket in P and takes log10 of both ends and a power of ten per
+// step; the bracket is kept in log10 P here.  Its upper end comes from
+// 2 Pm/(2 + 1e-10) where the root lies below Pm: log10 Pm - IMC_DU.
+constexpr double IMC_DU = 2.1714724094619722e-11; // log10(1 + 5e-11)
 __device__ __forceinline__ double imc(double P, double n, double dt, double rho, double gammi1) {
-  double Pu = 1.0e10, Pd = 1.0e-10, Pm = 1.0e1, Pmold = -1.0;
+  double lu = 10.0, ld = -10.0, lm = 1.0, Pm = 1.0e1, Pmold = -1.0;
   double nkbi = 1.0 / (KB * n);
   for (int it = 0; it < 30; ++it) {
     double T = Pm * nkbi;
     double CooL = fcool_ki(rho, T);
     double fev = Pm + CooL * dt * gammi1 - P;
-    double iud = copysign(1.0, fev);
-    Pd = dmax(-iud * Pm, Pd);
-    Pu = dmin(2.0 * Pm / (iud + 1.0 + 1.0e-10), Pu);
-    Pm = pow(1.0e1, 0.5 * (log10(Pu) + log10(Pd)));
+    if (signbit(fev)) ld = dmax(lm, ld);
+    else lu = dmin(lm - IMC_DU, lu);
+    lm = 0.5 * (lu + ld);
+    Pm = exp10(lm);
     if (fabs(Pm - Pmold) < 1.0e-5) break;
     Pmold = Pm;
   }

@@ -1924,6 +1924,13 @@ extern "C" int mcf_mlp_train(mcf_ctx *x, const mcf_train_opts *o, float *epoch_l
   return MCF_OK;
 }
 
+// Cells per block of k_cool_solve: two blocks per CU (as many as its registers
+// allow at once) while a block's cells fit its reject list
+static int cool_per(const mcf_ctx *x, int64_t n) {
+  const int64_t per = (n + 2 * x->ncu - 1) / (2 * x->ncu);
+  return (int)std::min<int64_t>(COOL_PER, (per + 255) / 256 * 256);
+}
+
 extern "C" int mcf_cool_solve(mcf_ctx *x, const double *P0, const double *nn, const double *dt, const double *rho,
                               const double *gammi1, int64_t n, int mode, double *P, int32_t *flag, double *ms) {
   if (!x || n <= 0 || !P0 || !nn || !dt || !rho || !gammi1 || !P || (mode != 0 && mode != 1)) {
@@ -1947,8 +1954,9 @@ extern "C" int mcf_cool_solve(mcf_ctx *x, const double *P0, const double *nn, co
   HIPCHK(hipEventCreate(&ea));
   HIPCHK(hipEventCreate(&eb));
   HIPCHK(hipEventRecord(ea, x->stream));
-  hipLaunchKernelGGL(k_cool_solve, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, x->stream, d0, d1, d2, d3, d4,
-                     (long)n, mode, x->mlp_pk, x->mlp, dP, df, nfb, fq);
+  const int per = cool_per(x, n);
+  hipLaunchKernelGGL(k_cool_solve, dim3((unsigned)((n + per - 1) / per)), dim3(256), 0, x->stream, d0, d1, d2, d3, d4,
+                     (long)n, per, mode, x->mlp_pk, x->mlp, dP, df, nfb, fq);
   if (mode == 1)
     hipLaunchKernelGGL(k_cool_fallback, dim3(256), dim3(256), 0, x->stream, d0, d1, d2, d3, d4, nfb, fq, dP);
   HIPCHK(hipGetLastError());
@@ -1984,8 +1992,9 @@ extern "C" int mcf_cool_solve_noalloc(mcf_ctx *x, const double *P0, const double
   unsigned *nfb = reinterpret_cast<unsigned *>(x->scratch);
   int *fq = reinterpret_cast<int *>(static_cast<unsigned char *>(x->scratch) + NOALLOC_HDR);
   hipLaunchKernelGGL(k_zero_u32x2, dim3(1), dim3(64), 0, x->stream, nfb);
-  hipLaunchKernelGGL(k_cool_solve, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, x->stream, P0, nn, dt, rho,
-                     gammi1, (long)n, mode, x->mlp_pk, x->mlp, P, flag, nfb, fq);
+  const int per = cool_per(x, n);
+  hipLaunchKernelGGL(k_cool_solve, dim3((unsigned)((n + per - 1) / per)), dim3(256), 0, x->stream, P0, nn, dt, rho,
+                     gammi1, (long)n, per, mode, x->mlp_pk, x->mlp, P, flag, nfb, fq);
   if (mode == 1)
     hipLaunchKernelGGL(k_cool_fallback, dim3(256), dim3(256), 0, x->stream, P0, nn, dt, rho, gammi1, nfb, fq, P);
   HIPCHK(hipGetLastError());

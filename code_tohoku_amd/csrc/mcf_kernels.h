@@ -229,8 +229,9 @@ __global__ void k_mlp_grad(const __bf16 *pk, const float *w, const float *X, con
                            float *grad, float *loss);
 __global__ void k_mlp_adam(float *w, float *m, float *v, const float *g, float lr, float b1t, float b2t);
 __global__ void k_fill_f32(float *a, int n, float v);
+constexpr int COOL_PER = 2048; // most cells of a block of k_cool_solve
 __global__ void k_cool_solve(const double *P0, const double *nn, const double *dt, const double *rho,
-                             const double *gi, long n, int mode, const __bf16 *pk, const float *w, double *Pout,
+                             const double *gi, long n, int per, int mode, const __bf16 *pk, const float *w, double *Pout,
                              int *flag, unsigned *nfb, int *fq);
 __global__ void k_cool_fallback(const double *P0, const double *nn, const double *dt, const double *rho,
                                 const double *gi, const unsigned *nfb, const int *fq, double *Pout);

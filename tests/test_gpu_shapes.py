@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import oracle
-from code_tohoku_amd import ics, mcf
+from code_tohoku_amd import ics, mcf, surrogate
 from code_tohoku_amd.restart import Input3D
 from helpers import interior, rel_linf, worst
 
@@ -90,3 +90,20 @@ def test_gravity_blocks_vs_oracle(n, nsplit):
     g.gravty(0.0, 2)
     np.testing.assert_array_equal(g.phi(), c)
     g.close()
+
+
+def test_cool_solve_batch_sizes():
+    """The stiff-cell solve on batches that end inside a wave, a block and a
+    block's share of cells: every cell's result and fallback flag are those of
+    the whole batch, bit for bit, in both modes (a cell's solve does not depend
+    on its place)."""
+    d = mcf.Domain(ics.converging_flow_input(16), nsplit=(1, 1, 1))
+    d.mlp_set_weights(surrogate.load_weights())
+    args = surrogate.stiff_batch(300001, 77)
+    for mode in (0, 1):
+        P, fl, _ = d.cool_solve(*args, mode)
+        for n in (1, 63, 257, 2048, 2049, 131073):
+            p, f, _ = d.cool_solve(*[a[:n] for a in args], mode)
+            np.testing.assert_array_equal(p, P[:n])
+            np.testing.assert_array_equal(f, fl[:n])
+    d.close()

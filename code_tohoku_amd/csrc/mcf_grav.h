@@ -28,6 +28,13 @@ constexpr int GRAV_LDS_NODES = 18 * 18 * 18; // k_grav_relax_lds: most nodes of 
 constexpr int GRAV_LDS_THREADS = 512;
 // planes of loads in flight in k_grav_relax_col and k_grav_relax_col4
 constexpr int GRAV_RELAX_D = 4, GRAV_RELAX_D4 = 1;
+// split levels held in LDS by k_grav_bottom: NGcr..4 (2 <= NGcr <= 4)
+constexpr int GRAV_BOT_TOP = 4;
+// NGcr = 4 takes the most: level 4 (Bot::size entries, three arrays), its four
+// ghost planes, the whole-domain levels 1..3 (882 entries, three arrays) and
+// 81 entries more of the potential
+constexpr int GRAV_BOT_LDS = 3 * (16 * 297) + 4 * 17 * 16 + 3 * 882 + 81;
+static_assert(GRAV_BOT_TOP >= GRAV_MAX_NGCR, "every split from 2 along an axis takes k_grav_bottom");
 constexpr int GRAV_FFT_MAXL = 1024; // longest FFT line (nn1/2 and nn2)
 // 4 pi G (M3:35: G = 1.11142d-4, G4pi = 12.56637d0*G)
 constexpr double GRAV_G4PI = 12.56637 * 1.11142e-4;
@@ -50,6 +57,7 @@ struct GravBuf {
   double *phi1, *rho1, *res1, *rhs1; // whole-domain levels, need1+1 entries (1-based)
   double *bphi1;                     // 2 x (needb1+1), 1-based
   double *bphi2;
+  double *flat; // potential of a level that k_grav_bottom took, whole
 };
 
 // threads of an exchange per rank block at a split level of nodes 0..n
@@ -84,7 +92,7 @@ __global__ void k_grav_relax_col(GravGeo G, const double *src, double *dst, cons
 template <int PP, int LMAX, int D>
 __global__ void k_grav_relax_col4(GravGeo G, const double *src, double *dst, const double *rhs2, int l);
 __global__ void k_grav_down(GravGeo G, const double *phif, double *phic, double *rhs2, int lc);
-__global__ void k_grav_prolong(GravGeo G, double *phif, const double *phic, int lf, int mode, const double *bphi2);
+__global__ void k_grav_prolong(GravGeo G, double *phif, const double *phic, int lf, int mode, const double *bphi2, int flat);
 __global__ void k_grav_collect(GravGeo G, double *u1, const double *u2);
 __global__ void k_grav_collect_resid(GravGeo G, double *phi1, double *res1, const double *phi2, const double *rhs2);
 __global__ void k_grav_divide(GravGeo G, double *u2, const double *u1);
@@ -92,6 +100,8 @@ __global__ void k_grav_divide(GravGeo G, double *u2, const double *u1);
 // 1 FMG stage j < NGcr, 2 FMG stage NGcr before the split levels, 3 the
 // bottom of a V-cycle below the coarsest split level)
 __global__ void k_grav_coarse(GravGeo G, GravBuf B, int prog, int j);
+// V-cycles of the split levels NGcr..top and of those below, one workgroup
+__global__ void k_grav_bottom(GravGeo G, GravBuf B, const double *phi, double *out, int top, int sweeps, int cycles);
 __global__ void k_pb_pack(PbArgs P, const double *rho, Geo g, double2 *Z);
 __global__ void k_pb_fft(double2 *Z, int L, long es, long inner_stride, long outer_stride, int ninner, int sign,
                          int lcw);

@@ -18,8 +18,11 @@
 // earlier planes, its upper neighbours on later ones, exactly as in the
 // sequential order.  One workgroup sweeps one block, a barrier per plane.
 //
-// The whole-domain levels 1..NGcr (at most 17^3 nodes) run as one
-// workgroup (k_grav_coarse) with the potential, right-hand side and
+// The split levels of at most 16^3 cells and all levels below them run whole
+// V-cycles in one workgroup's LDS (k_grav_bottom).
+//
+// The whole-domain levels 1..NGcr (at most 17^3 nodes) of the set-up, and of
+// an unsplit grid's V-cycles, run as one workgroup (k_grav_coarse) with the potential, right-hand side and
 // residual of all levels in LDS (3 x 45 KB), the reference's level-stacked
 // layout kept so that the residual's reads past a level's ends hit the same
 // neighbouring values.
@@ -31,6 +34,8 @@
 // column; the Green's-function weights and the sum over planes per mode;
 // the same unpacking and FFT backwards.
 #include "mcf_grav.h"
+
+#include <type_traits>
 
 namespace mcf {
 
@@ -254,6 +259,14 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Orders a wave's own LDS accesses (one lane's write before another's read):
+// the LDS serves them in the order issued, so only the compiler is held.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // ---------------------------------------------------------------------------
 // Sweeps from one copy of the level into another: a block reads its nodes and
 // ghosts from src and writes the swept nodes to dst, then puts those next to
@@ -378,20 +391,38 @@ __global__ __launch_bounds__(GRAV_LDS_THREADS) void k_grav_relax_lds(GravGeo G, 
   const bool on = (int)threadIdx.x < m1 * m2; // further waves only load and store
   const double *rc = rhs + j + J * k;
   auto rat = [&](int t) { return rc[(long)JK * min(t, T)]; };
+  const double u1 = U[p0 + 1];
   double prev = U[p0], rr[RD];
 #pragma unroll
   for (int s = 0; s < RD; ++s) rr[s] = rat(3 + s);
+  // the upper neighbours, values from before the sweep, are read a plane
+  // ahead, so that a plane's chain is the round trip of the two lower ones.
+  // Columns without a node on a plane read what lies there (i runs from 3-j-k
+  // to T+RD+1-j-k: inside the block's array, as a row is shorter than the rows
+  // before and behind it) and keep nothing.
+  double *col = U + p0 - j - k;
+  double xu = col[4], yu = col[3 + I], zu = col[3 + IJ];
+  const int lo = j + k + 1, cnt = on ? m0 : 0;
+  const bool idle = __builtin_amdgcn_readfirstlane((int)threadIdx.x) >= m1 * m2; // no column in this wave
   for (int tb = 3; tb <= T; tb += RD) {
+    if (idle) {
+#pragma unroll
+      for (int s = 0; s < RD; ++s) lds_barrier();
+      continue;
+    }
 #pragma unroll
     for (int s = 0; s < RD; ++s) {
-      const int i = tb + s - j - k, p = p0 + min(max(i, 1), m0);
-      const double sum = U[p + 1] + prev + U[p + I] + U[p - I] + U[p + IJ] + U[p - IJ] - h2 * rr[s];
-      const double v = (li && i == 1) ? U[p] : w * sum;
-      rr[s] = rat(tb + s + RD);
-      if (on && i >= 1 && i <= m0) {
-        U[p] = v;
-        prev = v;
-      }
+      const int t = tb + s;
+      const double ym = col[t - I], zm = col[t - IJ];
+      const double sum = xu + prev + yu + ym + zu + zm - h2 * rr[s];
+      xu = col[t + 2];
+      yu = col[t + 1 + I];
+      zu = col[t + 1 + IJ];
+      const double v = (li && t == lo) ? u1 : w * sum;
+      rr[s] = rat(t + RD);
+      const bool act = (unsigned)(t - lo) < (unsigned)cnt;
+      if (act) col[t] = v;
+      prev = act ? v : prev; // a use outside the branch keeps the loads and the sum out of it
       lds_barrier();
     }
   }
@@ -620,6 +651,12 @@ __global__ __launch_bounds__(GRAV_RELAX_THREADS) void k_grav_relax_col4(GravGeo 
 }
 template __global__ void k_grav_relax_col4<4, 4356, GRAV_RELAX_D4>(GravGeo, const double *, double *, const double *, int);
 
+// residMPI's expression
+__device__ __forceinline__ double g_res7(double xp, double xm, double yp, double ym, double zp, double zm, double u,
+                                         double h2i, double rhs) {
+  return -h2i * (xp + xm + yp + ym + zp + zm - 6.0 * u) + rhs;
+}
+
 // residMPI (SG8:918-952) and its exchange at one node of split level l: node
 // (i,j,k) of rank c, a ghost taken to the node it is a copy of (whose
 // neighbours, ghosts included, are in its own block); zero at the x-end nodes.
@@ -634,7 +671,7 @@ __device__ __forceinline__ double g_resid(const GravGeo &G, const double *phi2, 
   const double h = G.Lbox / (double)((n[0] - 1) * G.S[0]);
   const double h2i = 1.0 / (h * h);
   const long J = n[1] + 1, JK = J * (n[2] + 1), sx = JK, sy = 1 + JK, sz = J + JK;
-  return -h2i * (u[sx] + u[-sx] + u[sy] + u[-sy] + u[sz] + u[-sz] - 6.0 * u[0]) + rhs2[p];
+  return g_res7(u[sx], u[-sx], u[sy], u[-sy], u[sz], u[-sz], u[0], h2i, rhs2[p]);
 }
 
 // The way down from split level lc+1 to lc: residual, its restriction
@@ -697,8 +734,9 @@ __device__ __forceinline__ double pro_node(const F &C, int i, int j, int k) {
 // nodes; mode 0 adds to it (addintMPI, SG8:602-624; the interpolant is
 // neither stored nor exchanged).  An odd coordinate's two coarse nodes are
 // one and the same, and 0.5 (c + c) = c, so every node takes eight loads and
-// no branch.
-__global__ void k_grav_prolong(GravGeo G, double *phif, const double *phic, int lf, int mode, const double *bphi2) {
+// no branch.  flat: the coarse level lies as k_grav_bottom leaves it, whole,
+// without ghosts.
+__global__ void k_grav_prolong(GravGeo G, double *phif, const double *phic, int lf, int mode, const double *bphi2, int flat) {
   const int *nf = G.n[lf], *nc = G.n[lf - 1];
   const int m[3] = {nf[0] + 1, nf[1] + 1, nf[2] + 1};
   const long cnt = (long)m[0] * m[1] * m[2], t = g_tid();
@@ -721,14 +759,24 @@ __global__ void k_grav_prolong(GravGeo G, double *phif, const double *phic, int 
   if (mode == 1 && side >= 0) {
     v = bphi2[G.boff[lf] + (2L * rs + side) * (long)(nf[1] + 1) * (nf[2] + 1) + j + (long)(nf[1] + 1) * k];
   } else {
-    const long J = nc[1] + 1, JK = J * (nc[2] + 1);
-    const double *u = phic + G.off[lf - 1] + rs * G.bsz[lf - 1] + g_idx(nc, (i + 2) / 2, (j + 2) / 2, (k + 2) / 2);
     // the upper coarse node of each axis is (f+2)/2; the lower one f/2 at an
     // even coordinate, the same node at an odd one
-    const long sx = (i & 1) ? 0 : JK, sy = (j & 1) ? 0 : 1 + JK, sz = (k & 1) ? 0 : J + JK;
-    auto w = [&](long o) { return .5 * (u[-o] + u[-o - sx]); };
-    auto vv = [&](long o) { return .5 * (w(o) + w(o + sy)); };
-    v = .5 * (vv(0) + vv(sz));
+    const int iu = (i + 2) / 2, ju = (j + 2) / 2, ku = (k + 2) / 2;
+    auto mean = [](const double *u, long sx, long sy, long sz) {
+      auto w = [&](long o) { return .5 * (u[-o] + u[-o - sx]); };
+      auto vv = [&](long o) { return .5 * (w(o) + w(o + sy)); };
+      return .5 * (vv(0) + vv(sz));
+    };
+    if (flat) {
+      const int Nc = 1 << (lf - 1), X = c[0] * (nc[0] - 1) + iu, Y = c[1] * (nc[1] - 1) + ju, Z = c[2] * (nc[2] - 1) + ku;
+      const int Yw = Y > Nc ? 1 : Y, Zw = Z > Nc ? 1 : Z, sy = Nc + 1, sz = sy * Nc;
+      v = mean(phic + (X - 1) + sy * (Yw - 1) + sz * (Zw - 1), !(i & 1), (j & 1) ? 0 : sy * (Yw == Y ? 1 : 1 - Nc),
+               (k & 1) ? 0 : sz * (Zw == Z ? 1 : 1 - Nc));
+    } else {
+      const long J = nc[1] + 1, JK = J * (nc[2] + 1);
+      v = mean(phic + G.off[lf - 1] + rs * G.bsz[lf - 1] + g_idx(nc, iu, ju, ku), (i & 1) ? 0 : JK, (j & 1) ? 0 : 1 + JK,
+               (k & 1) ? 0 : J + JK);
+    }
   }
   if (mode == 1) phif[out] = v;
   else phif[out] = phif[out] + v;
@@ -803,25 +851,25 @@ struct Coarse {
   double *phi, *rhs, *res; // LDS, 1-based
 };
 
-__device__ __forceinline__ long c_at(long off, int n, int i, int j, int k) {
-  return off + (i - 1) + (long)n * ((j - 1) + (long)n * (k - 1));
+__device__ __forceinline__ int c_at(int off, int n, int i, int j, int k) {
+  return off + (i - 1) + n * ((j - 1) + n * (k - 1));
 }
 
 // rstrct (SG8:459-497): inner nodes weighted, the six faces copied, mode 1
 // zeroes the x faces
-__device__ void c_rstrct(double *uc, long offc, const double *uf, long offf, int nc, int mode) {
+__device__ void c_rstrct(double *uc, int offc, const double *uf, int offf, int nc, int mode) {
   const int nf = 2 * nc - 1;
-  const long cnt = (long)nc * nc * nc;
-  for (long q = threadIdx.x; q < cnt; q += blockDim.x) {
-    const int ic = 1 + (int)(q % nc), jc = 1 + (int)((q / nc) % nc), kc = 1 + (int)(q / ((long)nc * nc));
+  const int cnt = nc * nc * nc;
+  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
+    const int ic = 1 + q % nc, jc = 1 + (q / nc) % nc, kc = 1 + q / (nc * nc);
     const bool face = ic == 1 || ic == nc || jc == 1 || jc == nc || kc == 1 || kc == nc;
-    const long p = c_at(offf, nf, 2 * ic - 1, 2 * jc - 1, 2 * kc - 1);
+    const int p = c_at(offf, nf, 2 * ic - 1, 2 * jc - 1, 2 * kc - 1);
     double v;
     if (face) {
       v = uf[p];
     } else {
       const double w = 1.0 / 12.0;
-      v = 0.5 * uf[p] + w * (uf[p + 1] + uf[p - 1] + uf[p + nf] + uf[p - nf] + uf[p + (long)nf * nf] + uf[p - (long)nf * nf]);
+      v = 0.5 * uf[p] + w * (uf[p + 1] + uf[p - 1] + uf[p + nf] + uf[p - nf] + uf[p + nf * nf] + uf[p - nf * nf]);
     }
     if (mode == 1 && (ic == 1 || ic == nc)) v = 0.0;
     uc[c_at(offc, nc, ic, jc, kc)] = v;
@@ -830,14 +878,14 @@ __device__ void c_rstrct(double *uc, long offc, const double *uf, long offf, int
 }
 
 // interp (SG8:557-599); mode 1 sets the x faces from the end-plane potential
-__device__ void c_interp(const Coarse &S, double *uf, long offf, const double *uc, long offc, int nf, long np, int mode) {
+__device__ void c_interp(const Coarse &S, double *uf, int offf, const double *uc, int offc, int nf, int np, int mode) {
   const int nc = nf / 2 + 1;
-  const long cnt = (long)nf * nf * nf;
-  for (long q = threadIdx.x; q < cnt; q += blockDim.x) {
-    const int i = 1 + (int)(q % nf), j = 1 + (int)((q / nf) % nf), k = 1 + (int)(q / ((long)nf * nf));
+  const int cnt = nf * nf * nf;
+  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
+    const int i = 1 + q % nf, j = 1 + (q / nf) % nf, k = 1 + q / (nf * nf);
     double v;
     if (mode == 1 && (i == 1 || i == nf)) {
-      v = S.B.bphi1[(i == 1 ? 0 : S.G.needb1 + 1) + np + (j - 1) + (long)nf * (k - 1)];
+      v = S.B.bphi1[(i == 1 ? 0 : S.G.needb1 + 1) + np + (j - 1) + nf * (k - 1)];
     } else {
       auto C = [&](int a, int b, int e) { return uc[c_at(offc, nc, (a + 1) / 2, (b + 1) / 2, (e + 1) / 2)]; };
       v = pro_node(C, i, j, k);
@@ -847,43 +895,88 @@ __device__ void c_interp(const Coarse &S, double *uf, long offf, const double *u
   __syncthreads();
 }
 
-// relax (SG8:873-915): x nodes 2..n-1, y and z wrapped with period n
-// Hyperplanes i+j+k = t; each thread keeps one (j,k) column for the whole
-// sweep (n^2 <= 289 columns, fewer than the workgroup's threads), with its
-// wrapped neighbours' offsets formed once.
-static_assert(((1 << GRAV_MAX_NGCR) + 1) * ((1 << GRAV_MAX_NGCR) + 1) <= GRAV_COARSE_THREADS,
-              "one thread per column of the whole-domain levels");
-__device__ void c_relax(const Coarse &S, double *u, long off, const double *rhs, int n) {
+// relax (SG8:873-915): x nodes 2..n-1, y and z wrapped with period n.
+// Hyperplanes i+j+k = t; only levels below NGcr are relaxed here (n <= 9), so
+// the workgroup's first wave sweeps alone, each lane on one or two (j,k)
+// columns with their wrapped neighbours' offsets formed once.  The LDS serves
+// a wave's accesses in order, so a plane needs no barrier: it takes an LDS
+// round trip and its nine dependent operations (0.12 us; 0.55 us with a barrier
+// of sixteen waves).
+static_assert(((1 << (GRAV_MAX_NGCR - 1)) + 1) * ((1 << (GRAV_MAX_NGCR - 1)) + 1) <= 128, "two columns per lane");
+__device__ void c_relax(const Coarse &S, double *u, int off, const double *rhs, int n, int times) {
   const double w = 1.0 / 6.0;
   const double h = S.G.Lbox / (double)(n - 1);
   const double h2 = h * h;
-  const int q = threadIdx.x;
-  const bool on = q < n * n;
-  const int j = 1 + q % n, k = 1 + q / n;
-  const int jm = j == 1 ? n : j - 1, jp = j == n ? 1 : j + 1;
-  const int km = k == 1 ? n : k - 1, kp = k == n ? 1 : k + 1;
-  const long base = c_at(off, n, 0, j, k);
-  const long oyp = (long)n * (jp - j), oym = (long)n * (jm - j), ozp = (long)n * n * (kp - k),
-             ozm = (long)n * n * (km - k);
-  for (int t = 4; t <= (n - 1) + 2 * n; ++t) {
-    const int i = t - j - k;
-    if (on && i >= 2 && i <= n - 1) {
-      const long p = base + i;
-      u[p] = w * (u[p + 1] + u[p - 1] + u[p + oyp] + u[p + oym] + u[p + ozp] + u[p + ozm] - h2 * rhs[p]);
+  if (threadIdx.x < 64) {
+    int base[2], oyp[2], oym[2], ozp[2], ozm[2], lo[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int q = threadIdx.x + 64 * e, j = q < n * n ? 1 + q % n : 1, k = q < n * n ? 1 + q / n : 1;
+      lo[e] = q < n * n ? j + k + 2 : 1 << 20; // no node on any plane
+      base[e] = c_at(off, n, 0, j, k) - j - k;
+      oym[e] = n * ((j == 1 ? n : j - 1) - j);
+      oyp[e] = n * ((j == n ? 1 : j + 1) - j);
+      ozm[e] = n * n * ((k == 1 ? n : k - 1) - k);
+      ozp[e] = n * n * ((k == n ? 1 : k + 1) - k);
     }
-    __syncthreads();
+    // one or two columns per lane; the x, y and z upper neighbours and the
+    // right-hand side are read a plane ahead (a wrapped one was written n-1
+    // planes before); columns without a node on a plane read what lies there,
+    // at most n+4 entries past the level, and keep nothing
+    auto sweep = [&](auto two) {
+      constexpr int E = decltype(two)::value;
+      for (int s = 0; s < times; ++s) {
+        double xu[E], yu[E], zu[E], rr[E], prev[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const double *P = u + base[e];
+          prev[e] = P[lo[e] < 64 ? lo[e] - 1 : 3];
+          xu[e] = P[5];
+          yu[e] = P[4 + oyp[e]];
+          zu[e] = P[4 + ozp[e]];
+          rr[e] = rhs[base[e] + 4];
+        }
+        for (int tb = 4; tb <= (n - 1) + 2 * n; tb += 4) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const int t = tb + g;
+            double v[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+              const double *P = u + base[e];
+              const double ym = P[t + oym[e]], zm = P[t + ozm[e]];
+              v[e] = w * (xu[e] + prev[e] + yu[e] + ym + zu[e] + zm - h2 * rr[e]);
+              xu[e] = P[t + 2];
+              yu[e] = P[t + 1 + oyp[e]];
+              zu[e] = P[t + 1 + ozp[e]];
+              rr[e] = rhs[base[e] + t + 1];
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+              const bool act = (unsigned)(t - lo[e]) < (unsigned)(n - 2);
+              if (act) u[base[e] + t] = v[e];
+              prev[e] = act ? v[e] : prev[e];
+            }
+            wave_order();
+          }
+        }
+      }
+    };
+    if (n * n <= 64) sweep(std::integral_constant<int, 1>{});
+    else sweep(std::integral_constant<int, 2>{});
   }
+  __syncthreads();
 }
 
 // resid (SG8:955-971): the y and z neighbours at flat offsets +-n, +-n^2,
 // past the level's ends for its first and last rows and planes
-__device__ void c_resid(const Coarse &S, double *res, const double *u, const double *rhs, long off, int n) {
+__device__ void c_resid(const Coarse &S, double *res, const double *u, const double *rhs, int off, int n) {
   const double h = S.G.Lbox / (double)(n - 1);
   const double h2i = 1.0 / (h * h);
-  const long cnt = (long)n * n * n, nn = (long)n * n;
-  for (long q = threadIdx.x; q < cnt; q += blockDim.x) {
-    const int i = 1 + (int)(q % n);
-    const long p = off + q;
+  const int cnt = n * n * n, nn = n * n;
+  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
+    const int i = 1 + q % n;
+    const int p = off + q;
     if (i == 1 || i == n) {
       res[p] = 0.0;
     } else {
@@ -893,15 +986,15 @@ __device__ void c_resid(const Coarse &S, double *res, const double *u, const dou
   __syncthreads();
 }
 
-__device__ void c_fill0(double *u, long off, int n) {
-  const long cnt = (long)n * n * n;
-  for (long q = threadIdx.x; q < cnt; q += blockDim.x) u[off + q] = 0.0;
+__device__ void c_fill0(double *u, int off, int n) {
+  const int cnt = n * n * n;
+  for (int q = threadIdx.x; q < cnt; q += blockDim.x) u[off + q] = 0.0;
   __syncthreads();
 }
 
-__device__ void c_copy(double *dst, long off, const double *src, int n) {
-  const long cnt = (long)n * n * n;
-  for (long q = threadIdx.x; q < cnt; q += blockDim.x) dst[off + q] = src[off + q];
+__device__ void c_copy(double *dst, int off, const double *src, int n) {
+  const int cnt = n * n * n;
+  for (int q = threadIdx.x; q < cnt; q += blockDim.x) dst[off + q] = src[off + q];
   __syncthreads();
 }
 
@@ -913,7 +1006,7 @@ __device__ __forceinline__ double w3(int j, int k, int jp, int kp) {
 // (SG8:682-737) with the end-plane potential on the x faces
 __device__ void c_slvsml(const Coarse &S, const double *rhs, int b) {
   const double h = 0.5 * S.G.Lbox;
-  const long off = S.G.p1[1];
+  const int off = S.G.p1[1];
   double *u = S.phi;
   const int q = threadIdx.x;
   if (q < 9) {
@@ -956,8 +1049,8 @@ __device__ void c_slvsml(const Coarse &S, const double *rhs, int b) {
 __device__ void c_addint(const Coarse &S, int l) {
   const int nf = (1 << l) + 1;
   c_interp(S, S.res, S.G.p1[l], S.phi, S.G.p1[l - 1], nf, 0, 0);
-  const long cnt = (long)nf * nf * nf, off = S.G.p1[l];
-  for (long q = threadIdx.x; q < cnt; q += blockDim.x) S.phi[off + q] = S.phi[off + q] + S.res[off + q];
+  const int cnt = nf * nf * nf, off = S.G.p1[l];
+  for (int q = threadIdx.x; q < cnt; q += blockDim.x) S.phi[off + q] = S.phi[off + q] + S.res[off + q];
   __syncthreads();
 }
 
@@ -967,7 +1060,7 @@ __device__ void c_vcycle_lower(const Coarse &S, int top) {
   const GravGeo &G = S.G;
   for (int jj = top - 1; jj >= 2; --jj) {
     const int n = (1 << jj) + 1;
-    for (int p = 0; p < 5; ++p) c_relax(S, S.phi, G.p1[jj], S.rhs, n);
+    c_relax(S, S.phi, G.p1[jj], S.rhs, n, 5);
     c_resid(S, S.res, S.phi, S.rhs, G.p1[jj], n);
     c_rstrct(S.rhs, G.p1[jj - 1], S.res, G.p1[jj], (1 << (jj - 1)) + 1, 1);
     c_fill0(S.phi, G.p1[jj - 1], (1 << (jj - 1)) + 1);
@@ -975,8 +1068,18 @@ __device__ void c_vcycle_lower(const Coarse &S, int top) {
   c_slvsml(S, S.rhs, 0);
   for (int jj = 2; jj <= top - 1; ++jj) {
     c_addint(S, jj);
-    for (int p = 0; p < 5; ++p) c_relax(S, S.phi, G.p1[jj], S.rhs, (1 << jj) + 1);
+    c_relax(S, S.phi, G.p1[jj], S.rhs, (1 << jj) + 1, 5);
   }
+}
+
+// below the coarsest split level L: the collected residual restricted, the
+// lower levels, then the correction of level L
+__device__ void c_below(const Coarse &S, int L) {
+  const int nc = (1 << (L - 1)) + 1;
+  c_rstrct(S.rhs, S.G.p1[L - 1], S.res, S.G.p1[L], nc, 1);
+  c_fill0(S.phi, S.G.p1[L - 1], nc);
+  c_vcycle_lower(S, L);
+  c_addint(S, L);
 }
 
 // 2D restriction of an end plane (PB, SG8:1394-1460): 1/2 centre + 1/8
@@ -1048,31 +1151,377 @@ __global__ __launch_bounds__(GRAV_COARSE_THREADS) void k_grav_coarse(GravGeo G, 
     c_interp(S, sphi, G.p1[jst], sphi, G.p1[jst - 1], nf, G.pb1[jst], 1);
     c_copy(srhs, G.p1[jst], B.rho1, nf);
     for (int cyc = 0; cyc < 2; ++cyc) {
-      for (int p = 0; p < 5; ++p) c_relax(S, sphi, G.p1[jst], srhs, nf);
+      c_relax(S, sphi, G.p1[jst], srhs, nf, 5);
       c_resid(S, sres, sphi, srhs, G.p1[jst], nf);
       c_rstrct(srhs, G.p1[jst - 1], sres, G.p1[jst], (1 << (jst - 1)) + 1, 1);
       c_fill0(sphi, G.p1[jst - 1], (1 << (jst - 1)) + 1);
       c_vcycle_lower(S, jst);
       c_addint(S, jst);
-      for (int p = 0; p < 5; ++p) c_relax(S, sphi, G.p1[jst], srhs, nf);
+      c_relax(S, sphi, G.p1[jst], srhs, nf, 5);
     }
   } else if (prog == 2) {
     // FMG stage NGcr, whole-domain part
     c_interp(S, sphi, G.p1[L], sphi, G.p1[L - 1], N1, G.pb1[L], 1);
     c_copy(srhs, G.p1[L], B.rho1, N1);
   } else {
-    // below the coarsest split level: the collected residual restricted,
-    // the lower levels, then the correction of level NGcr
-    const int nc = (1 << (L - 1)) + 1;
-    c_rstrct(srhs, G.p1[L - 1], sres, G.p1[L], nc, 1);
-    c_fill0(sphi, G.p1[L - 1], nc);
-    c_vcycle_lower(S, L);
-    c_addint(S, L);
+    c_below(S, L);
   }
   for (long p = threadIdx.x; p <= need; p += blockDim.x) {
     B.phi1[p] = sphi[p];
     B.rhs1[p] = srhs[p];
     B.res1[p] = sres[p];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// V-cycles of the small split levels, one workgroup
+// ---------------------------------------------------------------------------
+// Levels NGcr..top (top <= GRAV_BOT_TOP, NGcr >= 2) as whole domains in LDS:
+// nodes 1..N+1 x 1..N x 1..N of each level (N = 2^l), y and z wrapped, in two
+// copies, and the right-hand side.  Rows of x are N+2 apart and z planes
+// N(N+2)+9: the columns of a hyperplane (x falls as y or z rises) then spread
+// evenly over the banks (with N+1 eight of them met in one bank).  The blocks
+// of the split show in the sweeps alone: a node's lower neighbours inside its
+// block are the sweep's own results (the copy written), all others the values
+// from before it (the copy read), which is what the exchanged ghosts of a
+// split level hold.  The whole-domain levels below NGcr are k_grav_coarse's;
+// the whole-domain form of NGcr itself is level NGcr here, its nodes N+1 along
+// y and z apart from the wrapped node 1 only in the correction: divide hands
+// them to the last ranks' high ghosts and leaves the first ranks' low ghosts
+// as they were, so the first sweep after it takes these from ghost planes.
+//
+// Bound by the chain of planes (an LDS round trip of 68 cycles and seven
+// dependent FP64 operations of 13 each: 0.1 us a plane in a wave alone; a
+// barrier of eight waves a plane doubles it).  On separate launches these
+// levels cost a launch per sweep, 5 to 9 us each for 0.3 to 3 us of work: a
+// V-cycle from level 4 takes 80 us instead of about 300 on 2x2x2 blocks, 110
+// instead of 190 on 8x8x8; a step with self-gravity 3.48 -> 2.0 ms at 64^3 on
+// 2x2x2, 15.8 -> 15.0 ms at 256^3 on 8x8x8.
+
+// The thread's index, read anew: what is formed from it is not carried in
+// registers from one part of the kernel to the next (128 are all there are).
+__device__ __forceinline__ int b_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+struct Bot {
+  const GravGeo &G;
+  double *s; // level NGcr's two copies and right-hand side, then the next level's
+  int flip; // bit l: the level's current copy
+  __device__ __forceinline__ static int rs(int l) { return (1 << l) + 2; }
+  __device__ __forceinline__ static int zs(int l) { return (rs(l) << l) + 9; }
+  __device__ __forceinline__ static int size(int l) { return zs(l) << l; }
+  __device__ __forceinline__ double *level(int l) const { // two copies, then the right-hand side
+    int o = 0;
+    for (int q = G.NGcr; q < l; ++q) o += 3 * size(q);
+    return s + o;
+  }
+  __device__ __forceinline__ double *cur(int l) const { return level(l) + ((flip >> l) & 1) * size(l); }
+  __device__ __forceinline__ double *other(int l) const { return level(l) + (~(flip >> l) & 1) * size(l); }
+  __device__ __forceinline__ double *rhs(int l) const { return level(l) + 2 * size(l); }
+  // node (X, Y, Z), 1-based
+  __device__ __forceinline__ static int at(int l, int X, int Y, int Z) {
+    return (X - 1) + rs(l) * (Y - 1) + zs(l) * (Z - 1);
+  }
+  // f(X, Y, Z) at every node, dealt out to the threads
+  template <class F> __device__ __forceinline__ static void each(int l, F f) {
+    const int N = 1 << l, NX = N + 1;
+    for (int q = b_tid(); q < NX << (2 * l); q += blockDim.x) {
+      const int yz = q / NX;
+      f(1 + q - yz * NX, 1 + (yz & (N - 1)), 1 + (yz >> l));
+    }
+  }
+  __device__ __forceinline__ double h(int l) const { return G.Lbox / (double)((G.n[l][0] - 1) * G.S[0]); }
+};
+
+// ghost planes of level NGcr, size = (N+1) N each: low and high y, low and high z
+struct BotGhost {
+  double *base;
+  int size;
+  __device__ __forceinline__ double *p(int d) const { return base + d * size; }
+};
+
+// times Gauss-Seidel sweeps of level l, a thread per column of a block, two
+// where there are more than 1024 (S0 N^2), the block's columns side by side: in one wave when
+// there are at most 64, so that its planes need no barrier.  ghosts: the first
+// sweep takes its y and z ghosts from the planes gh.
+template <int E>
+__device__ __forceinline__ void b_sweeps(Bot &b, int l, int times, const BotGhost &gh, bool ghosts) {
+  const GravGeo &G = b.G;
+  const int *n = G.n[l];
+  const int m0 = n[0] - 1, m1 = n[1] - 1, m2 = n[2] - 1, T = m0 + m1 + m2, N = 1 << l, cols = N * N * G.S[0];
+  const int s1 = __ffs(m1) - 1, s12 = s1 + __ffs(m2) - 1, s0 = __ffs(G.S[0]) - 1, s01 = s0 + __ffs(G.S[1]) - 1;
+  const double w = 1.0 / 6.0, h = b.h(l), h2 = h * h;
+  const int tid = b_tid();
+  const bool bar = m1 * m2 > 64;
+  const bool idle = __builtin_amdgcn_readfirstlane((int)threadIdx.x) >= cols; // no column in this wave
+  // rows of the column and its neighbours, shifted so that entry t is the node
+  // on plane t.  Columns without a node on a plane read what lies there (at
+  // most m1+m2 entries before a row, as many and 6 past it: inside the LDS
+  // array, whose ends are the ghost planes and the whole-domain levels).
+  int row[E], ryp[E], rzp[E], rym[E], rzm[E], lo[E], cnt[E], d[E], Y[E], Z[E];
+  bool iny[E], inz[E], last[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int q_ = tid + GRAV_COARSE_THREADS * e, q = q_ < cols ? q_ : 0;
+    const int r = q >> s12, jk = q & ((1 << s12) - 1), j = 1 + (jk & (m1 - 1)), k = 1 + (jk >> s1);
+    const int c0 = r & (G.S[0] - 1), c1 = (r >> s0) & (G.S[1] - 1), c2 = r >> s01;
+    const int X0 = c0 * m0;
+    Y[e] = c1 * m1 + j;
+    Z[e] = c2 * m2 + k;
+    d[e] = j + k;
+    row[e] = Bot::at(l, X0, Y[e], Z[e]) - d[e];
+    ryp[e] = Bot::at(l, X0, Y[e] == N ? 1 : Y[e] + 1, Z[e]) - d[e];
+    rzp[e] = Bot::at(l, X0, Y[e], Z[e] == N ? 1 : Z[e] + 1) - d[e];
+    rym[e] = Bot::at(l, X0, Y[e] == 1 ? N : Y[e] - 1, Z[e]) - d[e];
+    rzm[e] = Bot::at(l, X0, Y[e], Z[e] == 1 ? N : Z[e] - 1) - d[e];
+    iny[e] = j > 1;
+    inz[e] = k > 1;
+    last[e] = q_ < cols && c0 == G.S[0] - 1;
+    // node 1 of the first x block is the boundary, kept
+    lo[e] = d[e] + (c0 == 0 ? 2 : 1);
+    cnt[e] = q_ < cols ? d[e] + m0 + 1 - lo[e] : 0;
+  }
+#pragma unroll 1
+  for (int s = 0; s < times; ++s) {
+    if (idle) {
+      if (bar)
+        for (int t = 3; t <= T; t += 4) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) lds_barrier();
+        }
+    } else {
+      double *U = gh.base; // everything as an offset from the LDS array's start
+      const int A = (int)(b.cur(l) - U), B = (int)(b.other(l) - U), R = (int)(b.rhs(l) - U);
+      int yp[E], zp[E], ym[E], zm[E];
+      double xu[E], yu[E], zu[E], rr[E], prev[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        yp[e] = A + ryp[e];
+        zp[e] = A + rzp[e];
+        ym[e] = (iny[e] ? B : A) + rym[e];
+        zm[e] = (inz[e] ? B : A) + rzm[e];
+        if (ghosts && s == 0) {
+          const int X0 = row[e] + d[e] - Bot::at(l, 0, Y[e], Z[e]);
+          const int gy = X0 - 1 + (N + 1) * (Z[e] - 1) - d[e], gz = X0 - 1 + (N + 1) * (Y[e] - 1) - d[e];
+          if (Y[e] == 1) ym[e] = gy;
+          if (Y[e] == N) yp[e] = gh.size + gy;
+          if (Z[e] == 1) zm[e] = 2 * gh.size + gz;
+          if (Z[e] == N) zp[e] = 3 * gh.size + gz;
+        }
+        const double *a = U + A + row[e];
+        prev[e] = a[lo[e] - 1];
+        xu[e] = a[4]; // the upper neighbours and the right-hand side a plane ahead, as in k_grav_relax_lds
+        yu[e] = U[yp[e] + 3];
+        zu[e] = U[zp[e] + 3];
+        rr[e] = U[R + row[e] + 3];
+        if (lo[e] - d[e] == 2 && cnt[e] > 0) U[B + row[e] + d[e] + 1] = a[d[e] + 1];
+        if (last[e]) U[B + row[e] + d[e] + m0 + 1] = a[d[e] + m0 + 1];
+      }
+      wave_order();
+      for (int tb = 3; tb <= T; tb += 4) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int t = tb + g;
+          double v[E];
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const double ymv = U[ym[e] + t], zmv = U[zm[e] + t];
+            v[e] = w * (xu[e] + prev[e] + yu[e] + ymv + zu[e] + zmv - h2 * rr[e]);
+            xu[e] = U[A + row[e] + t + 2];
+            yu[e] = U[yp[e] + t + 1];
+            zu[e] = U[zp[e] + t + 1];
+            rr[e] = U[R + row[e] + t + 1];
+          }
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const bool act = (unsigned)(t - lo[e]) < (unsigned)cnt[e];
+            if (act) U[B + row[e] + t] = v[e];
+            prev[e] = act ? v[e] : prev[e];
+          }
+          if (bar) lds_barrier();
+          else wave_order();
+        }
+      }
+    }
+    b.flip ^= 1 << l;
+    __syncthreads();
+  }
+}
+__device__ __forceinline__ void b_relax(Bot &b, int l, int times, const BotGhost &gh, bool ghosts) {
+  if ((b.G.S[0] << (2 * l)) > GRAV_COARSE_THREADS) b_sweeps<2>(b, l, times, gh, ghosts);
+  else b_sweeps<1>(b, l, times, gh, ghosts);
+}
+
+// residMPI at every node of level l into its other copy
+__device__ void b_resid(Bot &b, int l) {
+  const int N = 1 << l, sy = Bot::rs(l), sz = Bot::zs(l);
+  const double h = b.h(l), h2i = 1.0 / (h * h);
+  const double *u = b.cur(l), *rhs = b.rhs(l);
+  double *res = b.other(l);
+  Bot::each(l, [&](int X, int Y, int Z) {
+    const int q = Bot::at(l, X, Y, Z);
+    double v = 0.0;
+    if (X > 1 && X <= N)
+      v = g_res7(u[q + 1], u[q - 1], u[q + (Y == N ? 1 - N : 1) * sy], u[q + (Y == 1 ? N - 1 : -1) * sy],
+                 u[q + (Z == N ? 1 - N : 1) * sz], u[q + (Z == 1 ? N - 1 : -1) * sz], u[q], h2i, rhs[q]);
+    res[q] = v;
+  });
+  __syncthreads();
+}
+
+// the way down from level l (k_grav_down)
+__device__ void b_down(Bot &b, int l) {
+  b_resid(b, l);
+  const int lc = l - 1, Nc = 1 << lc, sy = Bot::rs(l), sz = Bot::zs(l);
+  const double *res = b.other(l);
+  double *rhs = b.rhs(lc), *u = b.cur(lc);
+  Bot::each(lc, [&](int X, int Y, int Z) {
+    const int q = Bot::at(lc, X, Y, Z);
+    u[q] = 0.0;
+    double v = 0.0;
+    if (X > 1 && X <= Nc) {
+      const int p = Bot::at(l, 2 * X - 1, 2 * Y - 1, 2 * Z - 1);
+      v = res[p];
+      if (Y > 1 && Z > 1) {
+        const double w = 1.0 / 12.0;
+        v = 0.5 * v + w * (res[p + 1] + res[p - 1] + res[p + sy] + res[p - sy] + res[p + sz] + res[p - sz]);
+      }
+    }
+    rhs[q] = v;
+  });
+  __syncthreads();
+}
+
+// the interpolant of a coarser level (row and plane strides sy, sz) at node
+// (X, Y, Z); wrap: its nodes 1..Nc along y and z are periodic
+__device__ __forceinline__ double b_interp(const double *uc, int Nc, int sy, int sz, bool wrap, int X, int Y, int Z) {
+  const int xu = (X + 2) / 2 - 1, yu = (Y + 2) / 2 - 1, zu = (Z + 2) / 2 - 1; // 0-based
+  const int xl = xu - !(X & 1), yl = yu - !(Y & 1), zl = zu - !(Z & 1);
+  const int y0 = (wrap && yu == Nc ? 0 : yu) * sy, y1 = yl * sy, z0 = (wrap && zu == Nc ? 0 : zu) * sz, z1 = zl * sz;
+  auto w = [&](int o) { return .5 * (uc[o + xu] + uc[o + xl]); };
+  auto vv = [&](int o) { return .5 * (w(o + y0) + w(o + y1)); };
+  return .5 * (vv(z0) + vv(z1));
+}
+
+// addintMPI from level l-1 (k_grav_prolong, mode 0)
+__device__ void b_add(Bot &b, int l) {
+  const int lc = l - 1;
+  const double *uc = b.cur(lc);
+  double *u = b.cur(l);
+  Bot::each(l, [&](int X, int Y, int Z) {
+    const int q = Bot::at(l, X, Y, Z);
+    u[q] = u[q] + b_interp(uc, 1 << lc, Bot::rs(lc), Bot::zs(lc), true, X, Y, Z);
+  });
+  __syncthreads();
+}
+
+// the whole-domain levels below L = NGcr: the residual of L restricted
+// (rstrct, mode 1; its nodes N+1 along y and z are the wrapped first ones),
+// the lower levels, the correction of L (addint) with the ghost planes of the
+// sweep after it
+__device__ void b_below(Bot &b, const Coarse &S, const BotGhost &gh) {
+  const GravGeo &G = b.G;
+  const int L = G.NGcr, N = 1 << L, NX = N + 1, nc = N / 2 + 1, sy = Bot::rs(L), sz = Bot::zs(L);
+  b_resid(b, L);
+  const double *res = b.other(L);
+  double *u = b.cur(L);
+  for (int q = b_tid(); q < nc * nc * nc; q += blockDim.x) {
+    const int ic = 1 + q % nc, jc = 1 + (q / nc) % nc, kc = 1 + q / (nc * nc);
+    double v = 0.0;
+    if (ic > 1 && ic < nc) {
+      const int p = Bot::at(L, 2 * ic - 1, jc == nc ? 1 : 2 * jc - 1, kc == nc ? 1 : 2 * kc - 1);
+      v = res[p];
+      if (jc > 1 && jc < nc && kc > 1 && kc < nc) {
+        const double w = 1.0 / 12.0;
+        v = 0.5 * v + w * (res[p + 1] + res[p - 1] + res[p + sy] + res[p - sy] + res[p + sz] + res[p - sz]);
+      }
+    }
+    S.rhs[G.p1[L - 1] + q] = v;
+    S.phi[G.p1[L - 1] + q] = 0.0;
+  }
+  // the residual of level L-1 reads on into the first rows of level L
+  for (int q = b_tid(); q < nc * nc; q += blockDim.x) S.phi[G.p1[L] + q] = u[Bot::at(L, 1 + q % NX, 1 + q / NX, 1)];
+  __syncthreads();
+  c_vcycle_lower(S, L);
+  const double *uc = S.phi + G.p1[L - 1];
+  Bot::each(L, [&](int X, int Y, int Z) {
+    const int q = Bot::at(L, X, Y, Z), gy = (X - 1) + NX * (Z - 1), gz = (X - 1) + NX * (Y - 1);
+    const double o = u[q];
+    auto pro = [&](int y, int z) { return b_interp(uc, N / 2, nc, nc * nc, false, X, y, z); };
+    if (Y == N) gh.p(0)[gy] = o;
+    if (Y == 1) gh.p(1)[gy] = o + pro(NX, Z);
+    if (Z == N) gh.p(2)[gz] = o;
+    if (Z == 1) gh.p(3)[gz] = o + pro(Y, NX);
+    u[q] = o + pro(Y, Z);
+  });
+  __syncthreads();
+}
+
+// cycles V-cycles from split level top: right-hand side from its blocks, the
+// potential from its blocks (phi) or zero (no phi), the result to out, nodes
+// 1..N+1 x 1..N x 1..N (k_grav_prolong reads it there).  sweeps before and
+// after on the levels above NGcr, five after the correction of NGcr.
+__global__ __launch_bounds__(GRAV_COARSE_THREADS) void k_grav_bottom(GravGeo G, GravBuf B, const double *phi, double *out,
+                                                                     int top, int sweeps, int cycles) {
+  __shared__ double lds[GRAV_BOT_LDS];
+  const int L = G.NGcr, N1 = (1 << L) + 1, Ng = 1 << L, need = (int)G.p1[L], tail = (Ng / 2 + 1) * (Ng / 2 + 1);
+  const BotGhost gh{lds, N1 * Ng};
+  Bot b{G, lds + 4 * gh.size, 0};
+  double *sphi = b.level(top + 1), *srhs = sphi + need + tail, *sres = srhs + need;
+  const Coarse S{G, B, sphi, srhs, sres};
+  const int *n = G.n[top], N = 1 << top, NX = N + 1;
+  const int h0 = __ffs(n[0] - 1) - 1, h1 = __ffs(n[1] - 1) - 1, h2 = __ffs(n[2] - 1) - 1;
+  const int bs = (int)G.bsz[top];
+  const double *u2 = phi ? phi + G.off[top] : nullptr, *r2 = B.rhs2 + G.off[top];
+  // node (X, Y, Z) of the level, its high ghosts included, in its block
+  auto slot = [&](int X, int Y, int Z) {
+    const int c0 = min((X - 1) >> h0, G.S[0] - 1), c1 = min((Y - 1) >> h1, G.S[1] - 1), c2 = min((Z - 1) >> h2, G.S[2] - 1);
+    return g_rid(G, c0, c1, c2) * bs + (int)g_idx(n, X - (c0 << h0), Y - (c1 << h1), Z - (c2 << h2));
+  };
+  {
+    double *u = b.cur(top), *rhs = b.rhs(top);
+    Bot::each(top, [&](int X, int Y, int Z) {
+      const int a = slot(X, Y, Z), q = Bot::at(top, X, Y, Z);
+      u[q] = u2 ? u2[a] : 0.0;
+      rhs[q] = r2[a];
+    });
+    for (int q = b_tid(); q < need; q += blockDim.x) {
+      sphi[q] = B.phi1[q];
+      srhs[q] = B.rhs1[q];
+      sres[q] = B.res1[q];
+    }
+    if (top == L) // the ghosts as they are
+      for (int q = b_tid(); q < gh.size; q += blockDim.x) {
+        const int X = 1 + q % N1, e = 1 + q / N1;
+        gh.p(0)[q] = u2 ? u2[slot(X, 1, e) - 1 - (n[1] + 1) * (n[2] + 1)] : 0.0;
+        gh.p(1)[q] = u2 ? u2[slot(X, Ng + 1, e)] : 0.0;
+        gh.p(2)[q] = u2 ? u2[slot(X, e, 1) - (n[1] + 1) * (n[2] + 2)] : 0.0;
+        gh.p(3)[q] = u2 ? u2[slot(X, e, Ng + 1)] : 0.0;
+      }
+  }
+  __syncthreads();
+  for (int cyc = 0; cyc < cycles; ++cyc) {
+    for (int l = top; l > L; --l) {
+      b_relax(b, l, sweeps, gh, false);
+      b_down(b, l);
+    }
+    b_relax(b, L, sweeps, gh, top == L && cyc == 0);
+    b_below(b, S, gh);
+    b_relax(b, L, 5, gh, true);
+    for (int l = L + 1; l <= top; ++l) {
+      b_add(b, l);
+      b_relax(b, l, sweeps, gh, false);
+    }
+  }
+  const double *u = b.cur(top);
+  Bot::each(top, [&](int X, int Y, int Z) { out[(X - 1) + NX * ((Y - 1) + ((Z - 1) << top))] = u[Bot::at(top, X, Y, Z)]; });
+  for (int q = b_tid(); q < need; q += blockDim.x) {
+    B.phi1[q] = sphi[q];
+    B.rhs1[q] = srhs[q];
+    B.res1[q] = sres[q];
   }
 }
 

@@ -1008,8 +1008,8 @@ static int grav_setup(mcf_ctx *x) {
   const long n1 = ev(G.need1 + 1), nb1 = ev(2 * (G.needb1 + 1));
   const long nz = 4 * ev(tot2) + 4 * n1 + nb1 + ev(totb); // cleared at every solve
   const long nZ = 2L * npl * nn2 * H, nS = 2L * npl * nn2, nD = 2L * 2 * nn2 * H, nSD = 2L * 2 * nn2;
-  const long ntab = 4L * (q4 + 2);
-  const long total = nz + ev((long)x->ncell) + nZ + nS + nD + nSD + ntab + 4 * ev(npl) + 16;
+  const long ntab = 4L * (q4 + 2), nflat = ((1L << GRAV_BOT_TOP) + 1) << (2 * GRAV_BOT_TOP);
+  const long total = nz + ev((long)x->ncell) + nZ + nS + nD + nSD + ntab + nflat + 4 * ev(npl) + 16;
   HIPCHK(hipMalloc(&x->gpool, total * sizeof(double)));
   double *p = x->gpool;
   auto take = [&](long c) { double *r = p; p += ev(c); return r; };
@@ -1029,6 +1029,7 @@ static int grav_setup(mcf_ctx *x) {
   x->pbS = (double2 *)take(nS);
   x->pbD = (double2 *)take(nD);
   x->pbSD = (double2 *)take(nSD);
+  x->gb.flat = take(nflat);
   double2 *wf = (double2 *)take(2L * (q4 + 2));
   double2 *wi = (double2 *)take(2L * (q4 + 2));
   double *dzp = take(npl);
@@ -1185,6 +1186,17 @@ static int do_grav_solve(mcf_ctx *x) {
     const long nr = (long)(G.n[NGL][0] + 1) * (G.n[NGL][1] + 1) * (G.n[NGL][2] + 1) * G.npe;
     KLAUNCH_N("k_grav_rhs", k_grav_rhs, dim3(gblocks(nr)), dim3(TPB), 16.0 * nr, G, x->U[F_RHO], x->g, B.rhs2);
   }
+  // Split levels NGcr..bot go through k_grav_bottom, whole V-cycles at a time:
+  // up to 16^3 nodes fit one workgroup's LDS with the levels below them.  An
+  // unsplit grid (NGcr = 1) has no whole-domain level below NGcr and takes the
+  // launches, whose whole-domain part reads its arrays' first entries there as
+  // the reference does.
+  const int bot = NGcr >= 2 ? std::min(GRAV_BOT_TOP, NGL - 1) : 0;
+  auto bottom = [&](const double *phi, int top, int sweeps, int cycles) {
+    KLAUNCH_N("k_grav_bottom", k_grav_bottom, dim3(1), dim3(GRAV_COARSE_THREADS), 24.0 * (1L << (3 * top)), G, B, phi, B.flat,
+              top, sweeps, cycles);
+    return MCF_OK;
+  };
   auto rstrct = [&](double *uc, const double *uf, int lc) -> int {
     const long nr = (long)G.n[lc][0] * G.n[lc][1] * G.n[lc][2] * G.npe;
     KLAUNCH_N("k_grav_rstrct", k_grav_rstrct, dim3(gblocks(nr)), dim3(TPB), 64.0 * nr, G, uc, uf, lc);
@@ -1211,8 +1223,8 @@ static int do_grav_solve(mcf_ctx *x) {
   };
   auto prolong = [&](int lf, int mode) -> int {
     const long nr = (long)(G.n[lf][0] + 1) * (G.n[lf][1] + 1) * (G.n[lf][2] + 1) * G.npe;
-    KLAUNCH_N("k_grav_prolong", k_grav_prolong, dim3(gblocks(nr)), dim3(TPB), 24.0 * nr, G, cur(lf), cur(lf - 1),
-              lf, mode, B.bphi2);
+    KLAUNCH_N("k_grav_prolong", k_grav_prolong, dim3(gblocks(nr)), dim3(TPB), 24.0 * nr, G, cur(lf), lf - 1 <= bot ? B.flat : cur(lf - 1),
+              lf, mode, B.bphi2, lf - 1 <= bot ? 1 : 0);
     return MCF_OK;
   };
   CHK(rstrct(B.rho2, B.rhs2, NGL - 1));
@@ -1232,9 +1244,14 @@ static int do_grav_solve(mcf_ctx *x) {
       CHK(prolong(j, 1));
       if (j != NGL) CHK(copy_level(B.rhs2, B.rho2, j));
     }
+    const int sweeps = j >= NGL ? 2 : 5;
+    if (j <= bot) {
+      CHK(bottom(cur(j), j, sweeps, 2));
+      continue;
+    }
     for (int cyc = 0; cyc < 2; ++cyc) {
-      for (int jj = j; jj >= NGcr; --jj) {
-        CHK(grav_relax(x, jj, j >= NGL ? 2 : 5));
+      for (int jj = j; jj >= NGcr && jj > bot; --jj) {
+        CHK(grav_relax(x, jj, sweeps));
         if (jj == NGcr) {
           const long N1 = (1L << NGcr) + 1;
           KLAUNCH_N("k_grav_collect_resid", k_grav_collect_resid, dim3(gblocks(N1 * N1 * N1)), dim3(TPB),
@@ -1246,12 +1263,16 @@ static int do_grav_solve(mcf_ctx *x) {
                     cur(jj - 1), B.rhs2, jj - 1);
         }
       }
-      CHK(coarse(3, j));
-      CHK(divide());
-      CHK(grav_relax(x, NGcr, 5));
-      for (int jj = NGcr + 1; jj <= j; ++jj) {
+      if (bot) {
+        CHK(bottom(nullptr, bot, sweeps, 1));
+      } else {
+        CHK(coarse(3, j));
+        CHK(divide());
+        CHK(grav_relax(x, NGcr, 5));
+      }
+      for (int jj = (bot ? bot : NGcr) + 1; jj <= j; ++jj) {
         CHK(prolong(jj, 0));
-        CHK(grav_relax(x, jj, j >= NGL ? 2 : 5));
+        CHK(grav_relax(x, jj, sweeps));
       }
     }
   }

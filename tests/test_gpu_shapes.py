@@ -62,6 +62,17 @@ def test_step_shapes_vs_oracle(n, nsplit, periodic, precision):
 
 
 @pytest.mark.parametrize("n,nsplit", [
+    (16, (1, 2, 2)),   # all levels but the finest in one workgroup
+    (16, (1, 4, 4)),   # the coarsest split level is the highest that one takes
+    (64, (4, 1, 2)),   # its sweeps: blocks of 2 x 8 x 4 and 4 x 16 x 8 cells, a barrier per plane at 16 x 8
+    (64, (4, 4, 4)),   # 1024 columns of blocks, two whole-domain levels below
+    (128, (8, 2, 1)),  # two columns of blocks per thread, a barrier per plane
+])
+def test_gravity_small_levels_vs_oracle(n, nsplit):
+    check_gravity(n, nsplit)
+
+
+@pytest.mark.parametrize("n,nsplit", [
     (32, (2, 4, 1)),   # blocks of 17 x 9 x 33 nodes: in LDS and streamed, unequal axes
     (32, (1, 1, 2)),   # one block along x and y: a block is its own neighbour
     (64, (1, 2, 2)),   # 65 x 33 x 33 nodes: four columns per thread
@@ -72,6 +83,10 @@ def test_gravity_blocks_vs_oracle(n, nsplit):
     Phi after a step, at 1e-12, then Phi of a second solve of the same
     density, bit for bit (a solve starts from the same potential whatever the
     previous one left)."""
+    check_gravity(n, nsplit)
+
+
+def check_gravity(n, nsplit):
     p = box(n, n, n, False)
     p.ifgrv = 2
     st = ics.random_state(p, seed=n + sum(nsplit))

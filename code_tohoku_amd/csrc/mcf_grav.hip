@@ -296,22 +296,30 @@ struct GPush {
     if (dz) k = dz < 0 ? n[2] : 0;
     level[g_rid(G, a, b, e) * bsz + g_idx(n, i, j, k)] = v;
   }
-  // the images of all nodes next to a face; val(i, j, k) is the node's new
+  // The images of all nodes next to a face; val(i, j, k) is the node's new
   // value.  Combinations with x over the x faces, with y but not x over the
   // y faces, z alone over the z faces.
+  // xface: node 1 (s = 0) or n-1 (s = 1) along x of column (j, k).
+  __device__ __forceinline__ void xface(int s, int j, int k, double v) const {
+    const int i = s ? n[0] - 1 : 1, dx = s ? 1 : -1;
+    if (c[0] + dx < 0 || c[0] + dx >= G.S[0]) return;
+    const int dy = axis(1, j), dz = axis(2, k);
+    put(dx, 0, 0, i, j, k, v);
+    if (dy) put(dx, dy, 0, i, j, k, v);
+    if (dz) put(dx, 0, dz, i, j, k, v);
+    if (dy && dz) put(dx, dy, dz, i, j, k, v);
+  }
   template <class F> __device__ __forceinline__ void all(F val) const {
     const int m0 = n[0] - 1, m1 = n[1] - 1, m2 = n[2] - 1;
-    const int me = c[0] == G.S[0] - 1 ? n[0] : m0; // last node along x carried
     for (int q = threadIdx.x; q < 2 * m1 * m2; q += blockDim.x) {
-      const int s = q >= m1 * m2, r = q - s * m1 * m2, j = 1 + r % m1, k = 1 + r / m1, i = s ? m0 : 1, dx = s ? 1 : -1;
-      if (c[0] + dx < 0 || c[0] + dx >= G.S[0]) continue;
-      const int dy = axis(1, j), dz = axis(2, k);
-      const double v = val(i, j, k);
-      put(dx, 0, 0, i, j, k, v);
-      if (dy) put(dx, dy, 0, i, j, k, v);
-      if (dz) put(dx, 0, dz, i, j, k, v);
-      if (dy && dz) put(dx, dy, dz, i, j, k, v);
+      const int s = q >= m1 * m2, r = q - s * m1 * m2, j = 1 + r % m1, k = 1 + r / m1;
+      xface(s, j, k, val(s ? m0 : 1, j, k));
     }
+    yzfaces(val);
+  }
+  template <class F> __device__ __forceinline__ void yzfaces(F val) const {
+    const int m0 = n[0] - 1, m1 = n[1] - 1, m2 = n[2] - 1;
+    const int me = c[0] == G.S[0] - 1 ? n[0] : m0; // last node along x carried
     for (int q = threadIdx.x; q < 2 * me * m2; q += blockDim.x) {
       const int s = q >= me * m2, r = q - s * me * m2, i = 1 + r % me, k = 1 + r / me, j = s ? m1 : 1, dy = s ? 1 : -1;
       const int dz = axis(2, k);
@@ -451,9 +459,18 @@ __global__ __launch_bounds__(GRAV_LDS_THREADS) void k_grav_relax_lds(GravGeo G, 
 // ring of registers: memory answers in about 2.4 us, four times a plane.
 // Loads and stores go through buffer resources, which drop the offsets of idle
 // lanes: with loads or stores inside a branch the compiler cannot count how
-// many are in flight and waits for all of them.  A wave runs only the planes on which one of its
-// columns, or a column next to them, has a node, and waits at the barriers of
-// the others.
+// many are in flight and waits for all of them.  A wave runs only the planes on
+// which one of its columns, or a column next to them, has a node, and waits at
+// the barriers of the others.
+//
+// The x faces go out from registers (a column's first and last result); read
+// back from memory they take a cache line per node.  256^3 on 8x8x8: 295 -> 280
+// us a sweep, 1.44 TB/s of its compulsory 24 B per node; it moves 1.2 GB, three
+// times that, most of it lines of the ghost faces along x and y.  Not kept: the
+// y and z faces put into LDS as they are formed (270 us there, but 50 -> 62 us
+// for 8 blocks at 64^3, where the chain of planes counts), two workgroups per
+// CU (no change), several face values fetched before the first goes out (no
+// change).
 template <int LMAX, int D>
 __global__ __launch_bounds__(GRAV_RELAX_THREADS) void k_grav_relax_col(GravGeo G, const double *src, double *dst,
                                                                        const double *rhs2, int l) {
@@ -476,18 +493,37 @@ __global__ __launch_bounds__(GRAV_RELAX_THREADS) void k_grav_relax_col(GravGeo G
   const int li = c[0] == 0 ? 1 : 0;
   const int m0 = n[0] - 1, m1 = n[1] - 1, m2 = n[2] - 1, LJ = n[1] + 1, T = m0 + m1 + m2, I1 = n[0] + 1;
   const int JK = LJ * (n[2] + 1);
-  for (int q = threadIdx.x; q < I1 * (n[2] + 1); q += blockDim.x) {
-    lds[4 * LMAX + q] = u[g_idx(n, q % I1, 0, q / I1)];
-    lds[6 * LMAX + q] = u[g_idx(n, q % I1, n[1], q / I1)];
-  }
-  for (int q = threadIdx.x; q < I1 * (n[1] + 1); q += blockDim.x) {
-    lds[5 * LMAX + q] = u[g_idx(n, q % I1, q / I1, 0)];
-    lds[7 * LMAX + q] = u[g_idx(n, q % I1, q / I1, n[2])];
+  {
+    const int cy = I1 * (n[2] + 1), cz = I1 * (n[1] + 1); // nodes of a y and of a z face; eight loads in flight
+    for (int q0 = threadIdx.x; q0 < max(cy, cz); q0 += 2 * blockDim.x) {
+      double f[2][4];
+#pragma unroll
+      for (int h_ = 0; h_ < 2; ++h_) {
+        const int q = q0 + h_ * blockDim.x, y = q < cy ? q : 0, z = q < cz ? q : 0;
+        const int yi = y % I1, yk = y / I1, zi = z % I1, zj = z / I1;
+        f[h_][0] = u[g_idx(n, yi, 0, yk)];
+        f[h_][1] = u[g_idx(n, zi, zj, 0)];
+        f[h_][2] = u[g_idx(n, yi, n[1], yk)];
+        f[h_][3] = u[g_idx(n, zi, zj, n[2])];
+      }
+#pragma unroll
+      for (int h_ = 0; h_ < 2; ++h_) {
+        const int q = q0 + h_ * blockDim.x;
+        if (q < cy) {
+          lds[4 * LMAX + q] = f[h_][0];
+          lds[6 * LMAX + q] = f[h_][2];
+        }
+        if (q < cz) {
+          lds[5 * LMAX + q] = f[h_][1];
+          lds[7 * LMAX + q] = f[h_][3];
+        }
+      }
+    }
   }
   const int q = min((int)threadIdx.x, m1 * m2 - 1), j = 1 + q % m1, k = 1 + q / m1, jk = j + k, cell = j + LJ * k;
   // threads past the last column run it once more (the same values) and store nothing
   const bool on = (int)threadIdx.x < m1 * m2;
-  double prev = u[cell + JK * jk];
+  double prev = u[cell + JK * jk], v1 = 0.0; // v1: the new value of node 1; prev ends as that of the last node
   const double u1 = u[cell + JK * (jk + 1)]; // nodes 0 and 1 before the sweep
   // planes of this wave: from two before its first column's first node (the
   // old value a neighbour needs, passed on one plane ahead) to its last one
@@ -538,6 +574,7 @@ __global__ __launch_bounds__(GRAV_RELAX_THREADS) void k_grav_relax_col(GravGeo G
       lds[wc[e]] = v; // read only by the columns that have this i on the next plane
       lds[wx[e]] = rx[(s + 1) % D];
       prev = act ? v : prev;
+      v1 = i == 1 ? v : v1;
       __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(g_u2, v), db, act && on ? so : 0xffffffffu, 0, 0);
       fetch(s, i + D, so + D * sk);
       ym[e] += ay;
@@ -557,7 +594,11 @@ __global__ __launch_bounds__(GRAV_RELAX_THREADS) void k_grav_relax_col(GravGeo G
     }
   __syncthreads(); // the block's stores, before they are read again
   const GPush P{G, dst + G.off[l], n, {c[0], c[1], c[2]}, G.bsz[l]};
-  P.all([&](int a, int b, int e) { return d[g_idx(n, a, b, e)]; });
+  if (on) {
+    P.xface(0, j, k, v1);
+    P.xface(1, j, k, prev);
+  }
+  P.yzfaces([&](int a, int b, int e) { return d[g_idx(n, a, b, e)]; });
 }
 template __global__ void k_grav_relax_col<1156, GRAV_RELAX_D>(GravGeo, const double *, double *, const double *, int);
 
@@ -903,7 +944,7 @@ __device__ void c_interp(const Coarse &S, double *uf, int offf, const double *uc
 // round trip and its nine dependent operations (0.12 us; 0.55 us with a barrier
 // of sixteen waves).
 static_assert(((1 << (GRAV_MAX_NGCR - 1)) + 1) * ((1 << (GRAV_MAX_NGCR - 1)) + 1) <= 128, "two columns per lane");
-__device__ void c_relax(const Coarse &S, double *u, int off, const double *rhs, int n, int times) {
+__device__ __forceinline__ void c_relax(const Coarse &S, double *u, int off, const double *rhs, int n, int times) {
   const double w = 1.0 / 6.0;
   const double h = S.G.Lbox / (double)(n - 1);
   const double h2 = h * h;

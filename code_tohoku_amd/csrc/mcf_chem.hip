@@ -48,7 +48,9 @@ __device__ __forceinline__ double wave_scan_down(double v, int lane) {
 //   pass 3: the columns from the right, plus the totals of the blocks right of b.
 // Lane l always handles cell 64*chunk + l of a block, so every lane reads
 // back only the temp values it wrote itself; the right-hand columns come
-// from downward scans over the chunks taken last to first.
+// from downward scans over the chunks taken last to first.  Bound by memory
+// with the scans' lane exchanges beside it: 136 us at 128^3, 1.02 ms at 256^3
+// (4.6 TB/s of the arrays touched) at 96 registers; at 127 it took 1.13 ms.
 template <int DIR>
 __device__ __forceinline__ void shield_pass(const ShieldArgs &S, const Geo &g, int j, int k, int lane,
                                             const double (*tot)[5]) {
@@ -138,7 +140,11 @@ __global__ __launch_bounds__(256) void k_shield(ShieldArgs S, Geo g) {
   shield_pass<1>(S, g, j, k, lane, tot);
 }
 
-// Chemistry network (M3:2576-2774) over the interior cells
+// Chemistry network (M3:2576-2774) over the interior cells.  Bound by FP64
+// issue (about 3900 vector instructions a cell, most of them exponentials,
+// logarithms and powers; its 208 bytes a cell would take 75 us at 128^3): 248
+// -> 173 us there by forming one side of each switch of the rates, one
+// exponential per reaction and one reciprocal per shared denominator.
 __global__ __launch_bounds__(256) void k_chem(ChemArgs A, Geo g, double dt) {
   const long n = (long)g.n[0] * g.n[1] * g.n[2];
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -178,7 +178,7 @@ __global__ void k_fill_f32(float *a, int n, float v) {
 // (flag[i] = 1) are queued in fq for k_cool_fallback, which runs IMC on
 // dense waves.  A block gathers its rejected cells in LDS and takes one range
 // of the queue: one global atomic per wave on the one counter bounded the
-// kernel (222 us for 2^20 cells, fallback included; 111 now, bound by the network's 128
+// kernel (222 us for 2^20 cells, fallback included; 103 now, bound by the network's 128
 // exponentials and reciprocals per cell and the Newton steps' FP64
 // exponentials).
 __global__ __launch_bounds__(256, 2) void k_cool_solve(const double *P0, const double *nn, const double *dt,

@@ -311,7 +311,9 @@ static long boxsize(const Box &b) { return (long)b.cnt[0] * b.cnt[1] * b.cnt[2];
 // below 256^3: 64^3 mixed 355 us per sweep against 62 (4 cells), 128^3 681
 // against 215 (32), FP64 200 x 72 x 136 along z 1726 (two waves) against
 // 452, 64 x 8 x 8 174 against 57 (1 cell).  256^3 keeps whole columns (1.43
-// / 2.33 ms; 128 cells 1.43 / 2.36, 64 cells 1.51 / 2.45).
+// / 2.33 ms; 128 cells 1.43 / 2.36, 64 cells 1.51 / 2.45).  These are times of
+// one kernel at all segments; with its limiter branches and shared reciprocals
+// since, 256^3 takes 1.00 / 1.77.
 constexpr int COL_RAMP = 6;
 static int col_seg(const mcf_ctx *x, int n, long ncol) {
   const long nb = (ncol + SWEEP_COLS - 1) / SWEEP_COLS;

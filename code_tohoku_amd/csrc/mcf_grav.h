@@ -94,11 +94,9 @@ __global__ void k_grav_relax_col4(GravGeo G, const double *src, double *dst, con
 __global__ void k_grav_down(GravGeo G, const double *phif, double *phic, double *rhs2, int lc);
 __global__ void k_grav_prolong(GravGeo G, double *phif, const double *phic, int lf, int mode, const double *bphi2, int flat);
 __global__ void k_grav_collect(GravGeo G, double *u1, const double *u2);
-__global__ void k_grav_collect_resid(GravGeo G, double *phi1, double *res1, const double *phi2, const double *rhs2);
 __global__ void k_grav_divide(GravGeo G, double *u2, const double *u1);
 // the whole-domain part of the solve as one workgroup (prog: 0 set-up,
-// 1 FMG stage j < NGcr, 2 FMG stage NGcr before the split levels, 3 the
-// bottom of a V-cycle below the coarsest split level)
+// 1 FMG stage j < NGcr, 2 FMG stage NGcr before the split levels)
 __global__ void k_grav_coarse(GravGeo G, GravBuf B, int prog, int j);
 // V-cycles of the split levels NGcr..top and of those below, one workgroup
 __global__ void k_grav_bottom(GravGeo G, GravBuf B, const double *phi, double *out, int top, int sweeps, int cycles);

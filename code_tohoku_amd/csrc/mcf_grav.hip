@@ -21,8 +21,8 @@
 // The split levels of at most 16^3 cells and all levels below them run whole
 // V-cycles in one workgroup's LDS (k_grav_bottom).
 //
-// The whole-domain levels 1..NGcr (at most 17^3 nodes) of the set-up, and of
-// an unsplit grid's V-cycles, run as one workgroup (k_grav_coarse) with the potential, right-hand side and
+// The whole-domain levels 1..NGcr (at most 17^3 nodes) of the set-up run as
+// one workgroup (k_grav_coarse) with the potential, right-hand side and
 // residual of all levels in LDS (3 x 45 KB), the reference's level-stacked
 // layout kept so that the residual's reads past a level's ends hit the same
 // neighbouring values.
@@ -843,23 +843,6 @@ __global__ void k_grav_collect(GravGeo G, double *u1, const double *u2) {
   u1[G.p1[L] + t] = u2[G.off[L] + r * G.bsz[L] + g_idx(m, lo[0], lo[1], lo[2])];
 }
 
-// collect of the potential and of the residual at split level NGcr (the
-// residual formed where it is read)
-__global__ void k_grav_collect_resid(GravGeo G, double *phi1, double *res1, const double *phi2, const double *rhs2) {
-  const int L = G.NGcr, N1 = (1 << L) + 1;
-  const int *m = G.n[L];
-  const long t = g_tid();
-  if (t >= (long)N1 * N1 * N1) return;
-  const int g3[3] = {1 + (int)(t % N1), 1 + (int)((t / N1) % N1), 1 + (int)(t / ((long)N1 * N1))};
-  int c[3], lo[3];
-  for (int d = 0; d < 3; ++d) {
-    c[d] = min((g3[d] - 1) / (m[d] - 1), G.S[d] - 1);
-    lo[d] = g3[d] - c[d] * (m[d] - 1);
-  }
-  phi1[G.p1[L] + t] = phi2[G.off[L] + g_rid(G, c[0], c[1], c[2]) * G.bsz[L] + g_idx(m, lo[0], lo[1], lo[2])];
-  res1[G.p1[L] + t] = g_resid(G, phi2, rhs2, L, c, lo[0], lo[1], lo[2]);
-}
-
 // divide (SG8:369-382): whole-domain level NGcr into the rank blocks, the
 // node-0 planes of the first rank along each axis left as they are
 __global__ void k_grav_divide(GravGeo G, double *u2, const double *u1) {
@@ -1115,16 +1098,6 @@ __device__ void c_vcycle_lower(const Coarse &S, int top) {
   }
 }
 
-// below the coarsest split level L: the collected residual restricted, the
-// lower levels, then the correction of level L
-__device__ void c_below(const Coarse &S, int L) {
-  const int nc = (1 << (L - 1)) + 1;
-  c_rstrct(S.rhs, S.G.p1[L - 1], S.res, S.G.p1[L], nc, 1);
-  c_fill0(S.phi, S.G.p1[L - 1], nc);
-  c_vcycle_lower(S, L);
-  c_addint(S, L);
-}
-
 // 2D restriction of an end plane (PB, SG8:1394-1460): 1/2 centre + 1/8
 // per in-plane neighbour, a missing neighbour's weight moved to the centre
 __device__ __forceinline__ double plane_restrict(const double *bf, long kf, long stride, int ic, int jc, int mcx, int mcy) {
@@ -1202,12 +1175,10 @@ __global__ __launch_bounds__(GRAV_COARSE_THREADS) void k_grav_coarse(GravGeo G, 
       c_addint(S, jst);
       c_relax(S, sphi, G.p1[jst], srhs, nf, 5);
     }
-  } else if (prog == 2) {
+  } else {
     // FMG stage NGcr, whole-domain part
     c_interp(S, sphi, G.p1[L], sphi, G.p1[L - 1], N1, G.pb1[L], 1);
     c_copy(srhs, G.p1[L], B.rho1, N1);
-  } else {
-    c_below(S, L);
   }
   for (long p = threadIdx.x; p <= need; p += blockDim.x) {
     B.phi1[p] = sphi[p];

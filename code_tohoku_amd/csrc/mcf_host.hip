@@ -1189,11 +1189,11 @@ static int do_grav_solve(mcf_ctx *x) {
     KLAUNCH_N("k_grav_rhs", k_grav_rhs, dim3(gblocks(nr)), dim3(TPB), 16.0 * nr, G, x->U[F_RHO], x->g, B.rhs2);
   }
   // Split levels NGcr..bot go through k_grav_bottom, whole V-cycles at a time:
-  // up to 16^3 nodes fit one workgroup's LDS with the levels below them.  An
-  // unsplit grid (NGcr = 1) has no whole-domain level below NGcr and takes the
-  // launches, whose whole-domain part reads its arrays' first entries there as
-  // the reference does.
-  const int bot = NGcr >= 2 ? std::min(GRAV_BOT_TOP, NGL - 1) : 0;
+  // up to 16^3 nodes fit one workgroup's LDS with the levels below them.  The
+  // V-cycle of an unsplit grid (NGcr = 1) ends at level 2, where mglin's loops
+  // over the levels do (SG8:200-270): level 1 is never relaxed, its potential
+  // stays zero, and level 2 takes no correction.
+  const int bot = NGcr >= 2 ? std::min(GRAV_BOT_TOP, NGL - 1) : 0, low = bot ? bot + 1 : 2;
   auto bottom = [&](const double *phi, int top, int sweeps, int cycles) {
     KLAUNCH_N("k_grav_bottom", k_grav_bottom, dim3(1), dim3(GRAV_COARSE_THREADS), 24.0 * (1L << (3 * top)), G, B, phi, B.flat,
               top, sweeps, cycles);
@@ -1252,28 +1252,17 @@ static int do_grav_solve(mcf_ctx *x) {
       continue;
     }
     for (int cyc = 0; cyc < 2; ++cyc) {
-      for (int jj = j; jj >= NGcr && jj > bot; --jj) {
+      for (int jj = j; jj >= low; --jj) {
         CHK(grav_relax(x, jj, sweeps));
-        if (jj == NGcr) {
-          const long N1 = (1L << NGcr) + 1;
-          KLAUNCH_N("k_grav_collect_resid", k_grav_collect_resid, dim3(gblocks(N1 * N1 * N1)), dim3(TPB),
-                    40.0 * N1 * N1 * N1, G, B.phi1, B.res1, cur(NGcr), B.rhs2);
-        } else {
-          const int *m = G.n[jj - 1];
-          const long nr = (long)(m[0] - 1) * (m[1] - 1) * (m[2] - 1) * G.npe;
-          KLAUNCH_N("k_grav_down", k_grav_down, dim3(gblocks(nr)), dim3(TPB), 16.0 * 8.0 * nr + 8.0 * nr, G, cur(jj),
-                    cur(jj - 1), B.rhs2, jj - 1);
-        }
+        if (jj == low && !bot) break;
+        const int *m = G.n[jj - 1];
+        const long nr = (long)(m[0] - 1) * (m[1] - 1) * (m[2] - 1) * G.npe;
+        KLAUNCH_N("k_grav_down", k_grav_down, dim3(gblocks(nr)), dim3(TPB), 16.0 * 8.0 * nr + 8.0 * nr, G, cur(jj),
+                  cur(jj - 1), B.rhs2, jj - 1);
       }
-      if (bot) {
-        CHK(bottom(nullptr, bot, sweeps, 1));
-      } else {
-        CHK(coarse(3, j));
-        CHK(divide());
-        CHK(grav_relax(x, NGcr, 5));
-      }
-      for (int jj = (bot ? bot : NGcr) + 1; jj <= j; ++jj) {
-        CHK(prolong(jj, 0));
+      if (bot) CHK(bottom(nullptr, bot, sweeps, 1));
+      for (int jj = low; jj <= j; ++jj) {
+        if (jj > low || bot) CHK(prolong(jj, 0));
         CHK(grav_relax(x, jj, sweeps));
       }
     }

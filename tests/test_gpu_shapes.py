@@ -86,6 +86,15 @@ def test_gravity_blocks_vs_oracle(n, nsplit):
     check_gravity(n, nsplit)
 
 
+@pytest.mark.parametrize("n", [16, 32, 64, 128])
+def test_gravity_unsplit_vs_oracle(n):
+    """One block: mglin's V-cycles end at level 2, above the coarsest split
+    level (level 1), and every y and z ghost is the block's own.  The finest
+    levels take the four relaxation kernels in turn (17, 33, 65 and 129 nodes
+    a side)."""
+    check_gravity(n, (1, 1, 1))
+
+
 def check_gravity(n, nsplit):
     p = box(n, n, n, False)
     p.ifgrv = 2

@@ -594,7 +594,7 @@ static int do_sweep(mcf_ctx *x, int d, double dt) {
     const int n = x->g.n[d], ntr = x->g.n[d == 1 ? 2 : 1];
     const long ncol = (long)x->g.n[0] * ntr;
     const int seg = col_seg(x, n, ncol);
-    dim3 gr((unsigned)((n + seg - 1) / seg), (unsigned)((ncol + SWEEP_COLS - 1) / SWEEP_COLS), 1u);
+    dim3 gr((unsigned)((n + seg - 1) / seg) * (unsigned)((ncol + SWEEP_COLS - 1) / SWEEP_COLS));
     // reads rho, v(3), p, Bcc(3), face B_n, species(8); writes rho, v(3), p, species(8)
     const double by = 8.0 * (double)x->g.n[0] * x->g.n[1] * x->g.n[2] * 30;
     if (x->mixed) {

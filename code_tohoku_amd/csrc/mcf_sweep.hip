@@ -1056,6 +1056,16 @@ __global__ __launch_bounds__(256) void k_remap_col(SweepIO A, Geo g, double dt) 
   }
 }
 
+// The workgroups lie on the grid's x axis alone, a column block's nseg segments
+// side by side: the column blocks of a flat box (65729 at 4104 x 8 x 4100) are
+// more than the y axis of a grid takes (65536).
+__device__ __forceinline__ void col_tile(int nseg, int &bseg, int &bcol) {
+  int t, b1, b2;
+  xcd_tile(t, b1, b2);
+  bseg = t % nseg;
+  bcol = t / nseg;
+}
+
 // ---------------------------------------------------------------------------
 // A whole y or z sweep in one column march
 // ---------------------------------------------------------------------------
@@ -1092,8 +1102,8 @@ __global__ __launch_bounds__(256) void k_sweep_col(SweepIO A, Geo g, double dt, 
   constexpr int BT1 = (D + 1) % 3, BT2 = (D + 2) % 3;
   const int nx = g.n[0];
   const int n = g.n[D], ntr = g.n[D == 1 ? 2 : 1];
-  int bseg, bcol, b2;
-  xcd_tile(bseg, bcol, b2);
+  int bseg, bcol;
+  col_tile((n + seg - 1) / seg, bseg, bcol);
   const int id = SWEEP_COLS * bcol + (int)threadIdx.x; // column of the (x, transverse) plane, x fastest
   const int tr = 1 + id / nx, i = 1 + id % nx;
   const int p0 = 1 + seg * bseg;
@@ -1358,8 +1368,8 @@ __global__ __launch_bounds__(512) void k_sweep_col2(SweepIO A, Geo g, double dt,
   constexpr int BT1 = (D + 1) % 3, BT2 = (D + 2) % 3;
   const int nx = g.n[0];
   const int n = g.n[D], ntr = g.n[D == 1 ? 2 : 1];
-  int bseg, bcol, b2;
-  xcd_tile(bseg, bcol, b2);
+  int bseg, bcol;
+  col_tile((n + seg - 1) / seg, bseg, bcol);
   const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6, r4 = wv & 3;
   const bool producer = wv < 4;
   const int id_ = SWEEP_COLS * bcol + 64 * r4 + lane, ncol = nx * ntr;

@@ -61,6 +61,18 @@ def test_step_shapes_vs_oracle(n, nsplit, periodic, precision):
     check_step(p, ics.random_state(p, seed=sum(n)), nsplit, precision)
 
 
+def test_sweep_of_a_flat_box():
+    """4104 x 8 x 4100 cells: 65729 workgroups of columns along y, more than
+    the y axis of a launch grid takes (65536).  The sweep is launched on the
+    zero state and has to come to its end without an error; the shapes above
+    hold its values."""
+    d = mcf.Domain(box(4104, 8, 4100, True), nsplit=(1, 1, 1))
+    print("flat box allocated", flush=True)
+    d.sweep(1, 1.0e-3)
+    d.sync()
+    d.close()
+
+
 @pytest.mark.parametrize("n,nsplit", [
     (16, (1, 2, 2)),   # all levels but the finest in one workgroup
     (16, (1, 4, 4)),   # the coarsest split level is the highest that one takes

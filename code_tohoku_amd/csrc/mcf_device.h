@@ -20,9 +20,13 @@ __device__ __forceinline__ double dmax(double a, double b) { return a > b ? a : 
 __device__ __forceinline__ double dmin(double a, double b) { return a < b ? a : b; }
 
 // (0.5-sign(0.5,-Q))*Q + (0.5+sign(0.5,-Q))*U : positivity fallback (M3:1389).
-// One of the two weights is 1 and the other 0, so for finite Q and U it is
-// Q where Q's sign bit is clear and U elsewhere.
-__device__ __forceinline__ double posfix(double Q, double U) { return signbit(Q) ? U : Q; }
+// One of the two weights is 1 and the other 0: Q where Q's sign bit is clear
+// and U elsewhere, plus 0 times the other one, which keeps a NaN or an
+// infinity of a blown-up reconstruction in the state.
+__device__ __forceinline__ double posfix(double Q, double U) {
+  const bool neg = signbit(Q);
+  return __builtin_fma(0.0, neg ? Q : U, neg ? U : Q);
+}
 
 // n / d for several n over one d, each correctly rounded: the reciprocal y of
 // d once (an IEEE division), then per quotient q = n*y corrected by its exact

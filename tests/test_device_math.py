@@ -1,0 +1,48 @@
+"""Point routines of the kernels (csrc/mcf_device.h, mcf_prec.h), compiled for
+the host from the same headers, against the expressions they stand for: the
+reference's weighted sums at finite and non-finite operands."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+SRC = os.path.join(HERE, "device_math")
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("device_math") / "point.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-I", SRC,
+                    "-I", os.path.join(HERE, os.pardir, "code_tohoku_amd", "csrc"), os.path.join(SRC, "point.cpp"),
+                    "-o", so], check=True)
+    return C.CDLL(so)
+
+
+def call(fn, a, b, dtype=np.float64):
+    a, b = np.broadcast_arrays(np.asarray(a, np.float64), np.asarray(b, np.float64))
+    a, b = np.ascontiguousarray(a).ravel(), np.ascontiguousarray(b).ravel()
+    out = np.empty(a.size, dtype)
+    fn(C.c_long(a.size), a.ctypes.data_as(C.c_void_p), b.ctypes.data_as(C.c_void_p), out.ctypes.data_as(C.c_void_p))
+    return out
+
+
+def pairs(values):
+    a, b = np.meshgrid(values, values)
+    return a.ravel(), b.ravel()
+
+
+EDGE = np.array([0.0, 5e-324, 1e-20, 1.0, 3.0, 1e300, np.inf, np.nan])
+EDGE = np.concatenate([EDGE, -EDGE])
+
+
+def test_positivity_fallback(lib):
+    """(0.5 - sign(0.5,-Q)) Q + (0.5 + sign(0.5,-Q)) U, non-finite states
+    included: a NaN or infinity is not replaced by the cell's value."""
+    Q, U = pairs(EDGE)
+    with np.errstate(invalid="ignore"):
+        w = np.copysign(0.5, -Q)
+        ref = (0.5 - w) * Q + (0.5 + w) * U
+    np.testing.assert_array_equal(call(lib.v_posfix, Q, U), ref)

@@ -61,6 +61,26 @@ def test_step_shapes_vs_oracle(n, nsplit, periodic, precision):
     check_step(p, ics.random_state(p, seed=sum(n)), nsplit, precision)
 
 
+@pytest.mark.parametrize("precision", [mcf.PREC_FP64, mcf.PREC_MIXED])
+@pytest.mark.parametrize("value", [np.nan, -np.nan, np.inf])
+@pytest.mark.parametrize("field", [0, 1, 6])
+def test_non_finite_cell_stays_visible(field, value, precision):
+    """A blown-up cell does not turn into plausible numbers: with a NaN or an
+    infinity in rho, v_x or B_y of one cell, that cell and its neighbours
+    along each axis hold one after a step."""
+    p = box(24, 20, 16, True)
+    st = ics.random_state(p, seed=5)
+    k, j, i = 9, 11, 13
+    st[field, k, j, i] = value
+    g = mcf.Domain(p, nsplit=(2, 2, 2), precision=precision)
+    g.upload(st)
+    g.step(1.0e-4)
+    got = g.download()
+    g.close()
+    for dk, dj, di in ((0, 0, 0), (0, 0, 1), (0, 0, -1), (0, 1, 0), (0, -1, 0), (1, 0, 0), (-1, 0, 0)):
+        assert not np.isfinite(got[:, k + dk, j + dj, i + di]).all(), (dk, dj, di)
+
+
 def test_sweep_of_a_flat_box():
     """4104 x 8 x 4100 cells: 65729 workgroups of columns along y, more than
     the y axis of a launch grid takes (65536).  The sweep is launched on the

@@ -97,10 +97,15 @@ template <> struct QuotR<float> {
 };
 
 // minmod(a, b) as VLIMIT blends it: the smaller magnitude where the signs
-// agree, zero elsewhere.  In FP32 that is the median of a, b and 0.
+// agree, zero elsewhere, and NaN where either is not finite (the reference's
+// sum of both candidates): the minima and maxima pass over a NaN, the
+// multiply-adds with weight 0 do not.  Seven instructions; selects on the
+// operands' signs and magnitudes, which lost some NaNs, took eight.  In FP32
+// the median of a, b and 0; it passes over a NaN, as the comparisons of vslope
+// do, and the NaN cell's own states carry it on.
 __device__ __forceinline__ double minmod2(double a, double b) {
-  const bool same = (__double2hiint(a) ^ __double2hiint(b)) >= 0;
-  return same ? copysign(dmin(fabs(a), fabs(b)), a) : 0.0;
+  const double up = __builtin_fmax(__builtin_fmin(a, b), 0.0), dn = __builtin_fmin(__builtin_fmax(a, b), 0.0);
+  return __builtin_fma(0.0, a, up) + __builtin_fma(0.0, b, dn);
 }
 __device__ __forceinline__ float minmod2(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, 0.0f); }
 

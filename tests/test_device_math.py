@@ -46,3 +46,13 @@ def test_positivity_fallback(lib):
         w = np.copysign(0.5, -Q)
         ref = (0.5 - w) * Q + (0.5 + w) * U
     np.testing.assert_array_equal(call(lib.v_posfix, Q, U), ref)
+
+
+def test_minmod(lib):
+    """(0.5 + sign(0.5, a b)) sign(1, a) min(|a|, |b|) at finite operands, the
+    weight from the operands' signs; NaN at any other."""
+    a, b = pairs(EDGE)
+    m = np.copysign(np.minimum(np.abs(a), np.abs(b)), a)
+    ref = np.where(np.signbit(a) == np.signbit(b), m, 0.0)
+    ref[~(np.isfinite(a) & np.isfinite(b))] = np.nan
+    np.testing.assert_array_equal(call(lib.v_minmod2, a, b), ref)

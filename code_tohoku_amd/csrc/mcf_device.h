@@ -46,14 +46,14 @@ struct Quot {
 };
 
 // The limiter switch of VLIMIT (M3:1721): whether T = 1.27*U5/(kb*rho),
-// rounded, is at least 3.  That is a/b >= 3 - 2^-52 for a = 1.27*U5 and
-// b = kb*rho (the lower half of 3's rounding interval; no quotient of two
-// doubles is its end point), which the exact a - 3b decides without the
-// division.
+// rounded, is at least 3.  That is a/b > 3 - 2^-52 for a = 1.27*U5 and
+// b = kb*rho (the lower end of 3's rounding interval, which no quotient of two
+// doubles meets), which the exact a - 3b decides without the division; the
+// strict comparison also holds for zero and infinite a or b.
 __device__ __forceinline__ bool t_at_least_3(double u5, double rho) {
   const double a = 1.27 * u5, b = KB * rho;
   const double s = __builtin_fma(-3.0, b, a), t = -0x1p-52 * b;
-  return b > 0.0 ? s >= t : s <= t;
+  return signbit(b) ? s < t : s > t;
 }
 
 // RIEMAN (M3:1474-1551): four unrolled two-shock iterations with the

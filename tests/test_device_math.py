@@ -56,3 +56,20 @@ def test_minmod(lib):
     ref = np.where(np.signbit(a) == np.signbit(b), m, 0.0)
     ref[~(np.isfinite(a) & np.isfinite(b))] = np.nan
     np.testing.assert_array_equal(call(lib.v_minmod2, a, b), ref)
+
+
+def test_limiter_switch(lib):
+    """sign(0.5, 1.27 U5 / (kb rho) - 3) is +0.5, decided without the
+    division: every edge pair whose quotient is a number, and pressures a few
+    units in the last place around the switch."""
+    u, r = pairs(EDGE)
+    rng = np.random.default_rng(3)
+    rho = 10.0 ** rng.uniform(-30, 30, 200000) * rng.choice([-1.0, 1.0], 200000)
+    near = 3.0 * (8.63359 * rho) / 1.27
+    for s in range(-6, 7):
+        u = np.append(u, near * (1.0 + s * 2.0 ** -52))
+        r = np.append(r, rho)
+    with np.errstate(all="ignore"):
+        T = (1.27 * u) / (8.63359 * r)
+    ok = ~np.isnan(T)
+    np.testing.assert_array_equal(call(lib.v_switch, u[ok], r[ok], np.int32), ~np.signbit(T[ok] - 3.0))

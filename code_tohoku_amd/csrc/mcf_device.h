@@ -31,10 +31,13 @@ __device__ __forceinline__ double posfix(double Q, double U) {
 // n / d for several n over one d, each correctly rounded: the reciprocal y of
 // d once (an IEEE division), then per quotient q = n*y corrected by its exact
 // remainder, q + (n - q*d)*y (Markstein's correction step), and the hardware's
-// fix-up of zero, infinite and NaN operands.  Equal to the IEEE quotient in
-// 4e8 random and adversarial operand pairs; a quotient costs 4 instructions
-// instead of the 11 of a division.  Valid while y and n - q*d are normal
-// numbers: |d| in [2^-1022, 2^1022], |n| above 2^-968.
+// fix-up of zero, infinite and NaN operands.  A quotient costs 4 instructions
+// instead of the 11 of a division.  Correct while y and n - q*d are normal
+// numbers: |d| in [2^-1022, 2^1022], |n| above 2^-968 (below it about one
+// quotient in 400 is off by one unit in the last place).  A quotient that
+// overflows comes out NaN where the division gives an infinity; telling them
+// apart would cost an instruction a quotient, and both mark a blown-up state.
+// tests/test_device_math.py holds these bounds.
 struct Quot {
   double d, y;
   __device__ __forceinline__ explicit Quot(double d_) : d(d_), y(1.0 / d_) {}

@@ -73,3 +73,42 @@ def test_limiter_switch(lib):
         T = (1.27 * u) / (8.63359 * r)
     ok = ~np.isnan(T)
     np.testing.assert_array_equal(call(lib.v_switch, u[ok], r[ok], np.int32), ~np.signbit(T[ok] - 3.0))
+
+
+def near_powers_of_two(rng, n, emin, emax):
+    """2^e (1 + k ulp), k = -4 .. 4, and a third of them any mantissa."""
+    m = np.where(rng.random(n) < 0.33, 1.0 + rng.random(n), 1.0 + rng.integers(-4, 5, n) * 2.0 ** -52)
+    return np.ldexp(m * rng.choice([-1.0, 1.0], n), rng.integers(emin, emax, n))
+
+
+def test_shared_reciprocal_quotients(lib):
+    """n/d by a shared reciprocal is the IEEE quotient over the stated range:
+    |d| from 2^-1022, |n| from 2^-967 up, quotients from normal to the largest
+    double; and at zero, infinite and NaN operands of a normal one."""
+    rng = np.random.default_rng(11)
+    n = 3000000
+    den = near_powers_of_two(rng, n, -1021, 1020)
+    num = near_powers_of_two(rng, n, -966, 1023)
+    common = slice(0, n // 2)  # widths and densities of the fields
+    den[common] = near_powers_of_two(rng, n // 2, -40, 40)
+    num[common] = near_powers_of_two(rng, n // 2, -200, 200)
+    with np.errstate(over="ignore", under="ignore"):
+        ref = num / den
+    ok = (np.abs(ref) >= 2.0 ** -1021) & np.isfinite(ref)
+    assert ok.sum() > n // 2
+    np.testing.assert_array_equal(call(lib.v_quot, num[ok], den[ok]), ref[ok])
+    over = np.isinf(ref)
+    assert over.any() and not np.isfinite(call(lib.v_quot, num[over], den[over])).any()
+    a, b = pairs(np.array([0.0, -0.0, 1.0, -2.5, np.inf, -np.inf, np.nan]))
+    with np.errstate(all="ignore"):
+        np.testing.assert_array_equal(call(lib.v_quot, a, b), a / b)
+
+
+def test_shared_reciprocal_tiny_numerators(lib):
+    """Below the stated range a quotient is within one unit in the last place
+    (of the smallest normal number, where the quotient is subnormal)."""
+    rng = np.random.default_rng(12)
+    num = near_powers_of_two(rng, 500000, -1070, -967)
+    den = near_powers_of_two(rng, 500000, -40, 40)
+    ref = num / den
+    assert (np.abs(call(lib.v_quot, num, den) - ref) <= np.spacing(np.abs(ref))).all()

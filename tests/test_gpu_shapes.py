@@ -163,3 +163,33 @@ def test_cool_solve_batch_sizes():
             np.testing.assert_array_equal(p, P[:n])
             np.testing.assert_array_equal(f, fl[:n])
     d.close()
+
+
+def test_cool_solve_full_blocks():
+    """A batch past two full shares a compute unit (2048 cells a block, the
+    last block one cell), in both modes: results and flags as in its prefixes.
+    Then a network whose prediction overflows: every cell of every block is
+    rejected, the reject lists are full, and the fallback's results are mode
+    0's, bit for bit."""
+    n = (1 << 20) + 2049
+    d = mcf.Domain(ics.converging_flow_input(16), nsplit=(1, 1, 1))
+    d.mlp_set_weights(surrogate.load_weights())
+    args = surrogate.stiff_batch(n, 78)
+    imc = None
+    for mode in (0, 1):
+        P, fl, _ = d.cool_solve(*args, mode)
+        imc = P if mode == 0 else imc
+        for m in (1 << 20, 2049):
+            p, f, _ = d.cool_solve(*[a[:m] for a in args], mode)
+            np.testing.assert_array_equal(p, P[:m])
+            np.testing.assert_array_equal(f, fl[:m])
+            p, f, _ = d.cool_solve(*[a[n - m:] for a in args], mode)
+            np.testing.assert_array_equal(p, P[n - m:])
+            np.testing.assert_array_equal(f, fl[n - m:])
+    w = np.zeros(mcf.MLP_NPARAM, np.float32)
+    w[-1] = 1.0e30  # the output's bias
+    d.mlp_set_weights(w)
+    P, fl, _ = d.cool_solve(*args, 1)
+    d.close()
+    assert fl.all()
+    np.testing.assert_array_equal(P, imc)

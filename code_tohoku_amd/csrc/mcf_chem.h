@@ -31,7 +31,7 @@ __device__ __forceinline__ bool ch_on(double x) { return !signbit(x); }
 __device__ __forceinline__ double ch_fesc(double tau) {
   double a = 0.0 * tau, c = 0.0; // an infinite or NaN tau stays NaN
   if (ch_on(0.1 - 1.0e-16 - tau)) a = 0.5 - 0.585 * tau + 0.4563 * (tau * tau);
-  // formed everywhere: behind a branch it took k_shield from 78 to 127 registers
+  // formed everywhere: behind a branch k_shield takes 127 registers instead of 96
   const double m = (1.0 - exp(-2.34 * tau)) / (4.68 * tau + 1.0e-8);
   const double b = ch_on(11.9025 - (tau - 3.55) * (tau - 3.55)) ? m : 0.0;
   if (ch_on(tau - 7.0)) c = 1.0 / (4.0 * tau * sqrt(log(dmax(tau * 0.56419, 4.0))) + 1.0e-8);

@@ -304,16 +304,15 @@ static long boxsize(const Box &b) { return (long)b.cnt[0] * b.cnt[1] * b.cnt[2];
 // A workgroup marches SWEEP_COLS columns and fills a CU (one wave, or one
 // producer/consumer pair, per SIMD), so the launch takes
 // ceil(workgroups / CUs) rounds of seg + COL_RAMP positions (the stencil's
-// run-in is 11 positions of partial work).  COL_RAMP = 5 (FP64) and 6
-// (mixed) fit the times measured over segments of 1..256 cells: 343 / 388 /
-// 604 us at 128^3 in FP64 with 32 / 16 / 64 cells (1, 2 and half a round),
-// 215 / 248 / 365 us mixed.  Whole columns on every grid left most CUs idle
-// below 256^3: 64^3 mixed 355 us per sweep against 62 (4 cells), 128^3 681
-// against 215 (32), FP64 200 x 72 x 136 along z 1726 (two waves) against
-// 452, 64 x 8 x 8 174 against 57 (1 cell).  256^3 keeps whole columns (1.43
-// / 2.33 ms; 128 cells 1.43 / 2.36, 64 cells 1.51 / 2.45).  These are times of
-// one kernel at all segments; with its limiter branches and shared reciprocals
-// since, 256^3 takes 1.00 / 1.77.
+// run-in is 11 positions of partial work).  One-round launches fit a ramp of
+// 4 to 7 positions in FP64 and 8 to 9 mixed; any of 4 to 10 picks the same
+// segments, the fastest measured, on 64 x 8 x 8 (1 cell: 46 us FP64, 30
+// mixed; a whole column 88 / 52), 64^3 (4: 70 / 45; 3 cells, two rounds, 117 /
+// 73; whole 427 / 233), 90 x 44 x 26 (2: 57 / 37; whole 305 / 169), 128^3
+// (32: 262 / 148; 16, two rounds, 293 / 180; 64, half the CUs, 428 / 239; whole
+// 812 / 447), 200 x 72 x 136 along z (34: 263 / 145; 17: 292 / 171; whole 864
+// / 466) and 256^3 (whole columns, 1.55 / 0.98 ms; 128: 1.59 / 1.01; 64: 1.66
+// / 1.05).
 constexpr int COL_RAMP = 6;
 static int col_seg(const mcf_ctx *x, int n, long ncol) {
   const long nb = (ncol + SWEEP_COLS - 1) / SWEEP_COLS;
@@ -590,7 +589,7 @@ static int do_sweep(mcf_ctx *x, int d, double dt) {
     // reads only interior cells (periodic images), so no fills precede it.
     // One kernel instead of k_rhsmoc_col + k_remap_col: the MOC results do
     // not go through HBM (14% less time in both precisions when measured).
-    // 1.04 / 1.79 ms per sweep at 256^3 (mixed / FP64)
+    // 1.00 / 1.66 ms per y sweep in a step at 256^3 (mixed / FP64)
     const int n = x->g.n[d], ntr = x->g.n[d == 1 ? 2 : 1];
     const long ncol = (long)x->g.n[0] * ntr;
     const int seg = col_seg(x, n, ncol);

@@ -117,8 +117,8 @@ __device__ __forceinline__ float minmod2(float a, float b) { return __builtin_am
 // one candidate per quantity (vslope, no branch) takes about 43 instructions
 // a quantity in FP32 against 7 (minmod) or 22 (van Albada) here; waves whose
 // cells disagree run both sides.  256^3, with one slope per cell instead of
-// one per face in REMAP and Quot's shared reciprocals: y sweep 1.43 -> 1.04
-// ms (mixed), 2.36 -> 1.77 (FP64), x sweep 1.29 -> 1.08, 2.45 -> 1.77.
+// one per face in REMAP and Quot's shared reciprocals: y sweep 1.43 -> 1.00
+// ms (mixed), 2.36 -> 1.66 (FP64), x sweep with its fill 1.29 -> 1.11, 2.45 -> 1.71.
 template <class R, int N, class FP, class FM, class FD>
 __device__ __forceinline__ void vslopes(FP dp, FM dm, FD qd, R dxm, R dx0, R dxp, bool mm, R *g) {
   if (mm) {

@@ -123,7 +123,8 @@ def test_gravity_unsplit_vs_oracle(n):
     """One block: mglin's V-cycles end at level 2, above the coarsest split
     level (level 1), and every y and z ghost is the block's own.  The finest
     levels take the four relaxation kernels in turn (17, 33, 65 and 129 nodes
-    a side)."""
+    a side).  The reference's fixtures have 8 and 16 ranks: parity with its
+    build on one block is unpinned, the oracle's schedule is the measure."""
     check_gravity(n, (1, 1, 1))
 
 

@@ -765,8 +765,8 @@ __device__ __forceinline__ double wave_min(double v) {
 // block writes one pair of partial minima, and the last block to finish
 // folds them (min is exact, so the result does not depend on the order) and
 // writes them to host memory, then the launch's number, which the host waits
-// for.  Bound by HBM at 256^3: 0.35 ms for 1.74 GB, 4.9 TB/s.  At 64^3 the
-// launch takes 16 us; a block of 256 threads per row, a second launch and a
+// for.  Bound by HBM at 256^3: 0.36 ms for 1.74 GB, 4.8 TB/s.  At 64^3 the
+// launch takes 17 us; a block of 256 threads per row, a second launch and a
 // copy to the host took 16 + 6 + 2 us and two gaps between launches.
 template <bool CHEM> __global__ __launch_bounds__(64 * DT_WAVES) void k_dtmin(DtArgs A, Geo g) {
   __shared__ double s0[DT_WAVES], s1[DT_WAVES];
@@ -815,20 +815,20 @@ template <bool CHEM> __global__ __launch_bounds__(64 * DT_WAVES) void k_dtmin(Dt
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < DT_WAVES; ++w) { tc = fmin(tc, s0[w]); tl = fmin(tl, s1[w]); }
-    // device-scope stores (past the XCD's L2), acknowledged before the count:
-    // a release fence per block would write back the whole L2 each time
-    // (0.45 against 0.34 ms at 256^3)
-    __hip_atomic_store(A.part + 2 * blockIdx.x, tc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(A.part + 2 * blockIdx.x + 1, tl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lastb = __hip_atomic_fetch_add(A.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    A.part[2 * blockIdx.x] = tc;
+    A.part[2 * blockIdx.x + 1] = tl;
+    // The count releases this block's minima and acquires the others'.  The
+    // release writes back the XCD's L2: 327 -> 335 us at 256^3 and 18.0 -> 19.5
+    // at 64^3 against device-scope stores, a wait for them and a relaxed count,
+    // which the memory model does not order.
+    lastb = __hip_atomic_fetch_add(A.done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
   }
   __syncthreads();
   if (!lastb) return;
   tc = tl = A.tfinal;
   for (int b = threadIdx.x; b < (int)gridDim.x; b += 64 * DT_WAVES) {
-    tc = fmin(tc, __hip_atomic_load(A.part + 2 * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    tl = fmin(tl, __hip_atomic_load(A.part + 2 * b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    tc = fmin(tc, A.part[2 * b]);
+    tl = fmin(tl, A.part[2 * b + 1]);
   }
   tc = wave_min(tc);
   tl = wave_min(tl);
